@@ -1,16 +1,34 @@
 // FP64 GEMM on the CDNA4 matrix cores (v_mfma_f64_16x16x4_f64), gfx950.
 //
-// One kernel serves every dense contraction of the RI G0W0 path:
+// One kernel serves every dense FP64 contraction of the RI G0W0 path:
 //   AO->MO half transforms ((P|mu nu) . C), the Casida SYRK (B^T B scaled by
 //   sqrt(de)), w_s = B (X+Y), the self-energy products w_s^T (P|p i), the
-//   imaginary-axis chi0 = X diag(s(iw)) X^T batched over frequencies and
-//   chi(iw) (P|p m) with a fused column-dot epilogue.
+//   imaginary-axis chi0 = X diag(s(iw)) X^T batched over frequencies,
+//   chi(iw) (P|p m) with a fused column-dot epilogue, and the Hartree /
+//   exchange products of the RI-HF.
 //
-// Tiling: a workgroup of WM x WN wave64s owns a BM x BN tile of C and walks K
-// in slabs of BK = 16 through double-buffered LDS (one barrier per slab, the
-// next slab's global loads in flight during the MFMAs of the current one).
-// Each wave owns (BM/WM) x (BN/WN) and issues (BM/WM/16) * (BN/WN/16)
-// independent MFMA chains per k-step of 4, which hides the MFMA latency.
+// What bounds it: the matrix cores (one 16x16x4 MFMA takes 64 cycles of a
+// SIMD), so everything else only has to stay out of their way.
+//   * A workgroup of WM x WN wave64s owns a BM x BN tile of C and walks K in
+//     slabs of BK = 16 through LDS, the next slab's global loads in flight
+//     during the MFMAs of the current one. What keeps the matrix cores busy is
+//     other workgroups on the same CU: their MFMAs run under this one's
+//     barriers, LDS writes and epilogue. 128x128 tiles (accumulators of 128
+//     registers) fit twice, with two LDS buffers and one barrier per slab;
+//     smaller tiles take one buffer and two barriers and fit three or four
+//     times (128x80 of long K: 46 -> 58 TFLOP/s with three instead of two).
+//     A wave issues its MFMAs at raised priority (128-wide tiles: 64 -> 67
+//     TFLOP/s at 8192 x 8192 x 4096; the copy-bound narrow tiles lose 5 %).
+//   * Global loads are pairs of doubles (16 bytes a lane) along the operand's
+//     contiguous dimension. Rows past the edge read the last row again (their
+//     results are not stored), so only a last slab that is cut by K tests its
+//     elements, and it reads zeros there.
+//   * A wave whose part of the tile lies past the edge or above the diagonal of
+//     a symmetric update leaves the matrix cores to the others.
+//   * With fewer tiles than the GPU's slots, or a last round of workgroups that
+//     would be mostly empty, the K range is split (gemm_f64_splits): partial
+//     products go to a workspace and gemm_f64_reduce_kernel sums them in a
+//     fixed order and applies the epilogue.
 //
 // Fragment layout of v_mfma_f64_16x16x4_f64 (checked on gfx950): operand "a"
 // lane l = a[i = l & 15][k = l >> 4], operand "b" lane l = b[k = l >> 4][j = l & 15],
@@ -36,8 +54,17 @@ namespace mgw {
 namespace {
 
 typedef double d4 __attribute__((ext_vector_type(4)));
+// two doubles at an address that is only 8-byte aligned (odd leading
+// dimensions): global memory takes 16-byte accesses at any dword address
+typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));
+typedef double d2 __attribute__((ext_vector_type(2)));
 
-constexpr int PAD = 1;
+constexpr int BK = 16;         // k per slab
+// LDS row length of a tile of b rows (columns): consecutive k start 144 bytes
+// apart modulo the 256 bytes of the banks, so that neither the 4 k of a
+// fragment read nor the 8 pairs of k that a transposing store writes share
+// banks; even, so that pairs stay 16-byte aligned
+constexpr int lds_row(int b) { return b + (b % 32 == 0 ? 18 : 34); }
 constexpr int GROUP_M = 8;     // tile rows per group of the grouped ordering
 
 struct GemmDev {
@@ -53,33 +80,52 @@ struct GemmDev {
   int lower_only;
   int no_mirror;       // lower_only: leave the strict upper triangle untouched
   int upper_zero;      // lower_only: write zeros above the diagonal instead of the mirror
-  int tri_a;           // A (not transposed) is lower triangular: A(m, k) = 0 for k > m
+  int tri_a;           // A (not transposed) is lower triangular, zeros stored above the diagonal
   int batch_outer;     // walk the tiles of one batch entry before the next
   int tiles_m, tiles_n, batch;
   int64_t nblocks;
+  int splits, kchunk;  // K range per split (a multiple of BK)
+  double* part;        // splits > 1: part[split][batch][n][m], else null
   const double* dotB; int64_t lddot;
   double dot_cc, dot_cd;
   double* dotpart; int64_t strideDot;
   const double* dot_w; int64_t strideDotW;
 };
 
-template <int BM, int BN, int WM, int WN, int BK, bool TA, bool TB, bool DOT, int KLASS>
-__global__ void __launch_bounds__(64 * WM * WN)
+// C(m, n) of the product: scales, diagonal and beta, the mirror or the zero
+// above the diagonal
+__device__ inline void store_result(const GemmDev& g, double* __restrict__ C, const double* __restrict__ dg, int m,
+                                    int n, double acc) {
+  double v = g.alpha * acc;
+  if (g.rowscale) v *= g.rowscale[m];
+  if (g.colscale) v *= g.colscale[n];
+  if (dg && m == n) v += dg[m];
+  const int64_t idx = m + (int64_t)n * g.ldc;
+  if (g.beta != 0.0) v += g.beta * C[idx];
+  C[idx] = v;
+  if (g.lower_only && m > n && !g.no_mirror) C[n + (int64_t)m * g.ldc] = g.upper_zero ? 0.0 : v;
+}
+
+template <int BM, int BN, int WM, int WN, bool TA, bool TB, bool DOT, int KLASS>
+__global__ void __launch_bounds__(64 * WM * WN, WM * WN > 4 ? WM * WN / 4 : BM * BN <= 128 * 64 ? 4 : BM * BN <= 128 * 96 ? 3 : 2)
 gemm_f64_kernel(GemmDev g) {
   constexpr int NT = 64 * WM * WN;
   constexpr int TM = BM / WM;
   constexpr int TN = BN / WN;
   constexpr int FM = TM / 16;
   constexpr int FN = TN / 16;
-  constexpr int LA = BM * BK / NT;   // A elements loaded per thread per slab
-  constexpr int LB = BN * BK / NT;
-  static_assert(BM * BK % NT == 0 && BN * BK % NT == 0, "tile/thread mismatch");
-  // contiguous-dimension strides of the per-thread element walk
-  static_assert(TA ? (NT % BK == 0) : (NT % BM == 0), "A walk");
-  static_assert(TB ? (NT % BN == 0) : (NT % BK == 0), "B walk");
+  static_assert(TM % 16 == 0 && TN % 16 == 0, "wave tile");
+  constexpr bool PRIO = BN >= 128;          // raised priority during the MFMAs
+  constexpr int NBUF = BM * BN <= 128 * 96 ? 1 : 2;
+  // pairs of doubles of a slab, and the walk of a thread over them: an
+  // operand whose contiguous dimension is m (n) has BM / 2 pairs per k, one
+  // whose contiguous dimension is k has BK / 2 per row
+  constexpr int PA = BM * BK / 2, PB = BN * BK / 2;
+  constexpr int LA = (PA + NT - 1) / NT, LB = (PB + NT - 1) / NT;
+  constexpr int ACOLS = TA ? BK / 2 : BM / 2, BCOLS = TB ? BN / 2 : BK / 2;
 
-  __shared__ double As[2][BK][BM + PAD];
-  __shared__ double Bs[2][BK][BN + PAD];
+  __shared__ __attribute__((aligned(16))) double As[NBUF][BK][lds_row(BM)];
+  __shared__ __attribute__((aligned(16))) double Bs[NBUF][BK][lds_row(BN)];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -89,11 +135,13 @@ gemm_f64_kernel(GemmDev g) {
 
   // logical block: batch fastest when the batch entries share operands (the
   // frequencies of one chi0 tile read the same panels), batch slowest when
-  // they do not; then the tile in grouped order
+  // they do not; then the K split; then the tile in grouped order
   const int64_t L = xcd_logical(blockIdx.x, g.nblocks);
-  const int64_t ntile = g.nblocks / g.batch;
-  const int batch = (int)(g.batch_outer ? L / ntile : L % g.batch);
-  const int tile = (int)(g.batch_outer ? L % ntile : L / g.batch);
+  const int64_t per = g.nblocks / g.batch;
+  const int batch = (int)(g.batch_outer ? L / per : L % g.batch);
+  const int ts = (int)(g.batch_outer ? L % per : L / g.batch);
+  const int split = ts % g.splits;
+  const int tile = ts / g.splits;
   int bm, bn;
   if (g.lower_only && BM == BN) {
     tri_grouped(tile, g.tiles_m, bm, bn);
@@ -115,52 +163,151 @@ gemm_f64_kernel(GemmDev g) {
   const double* __restrict__ B = g.B + (int64_t)batch * g.strideB;
   const double* __restrict__ ks = g.kscale ? g.kscale + (int64_t)batch * g.strideK : nullptr;
 
-  // Per-thread walk over a slab: element e = tid + i * NT.
-  //  A non-trans: m = tid % BM fixed, k = tid / BM + i * (NT / BM)
-  //  A trans:     k = tid % BK fixed, m = tid / BK + i * (NT / BK)
-  const int a_fix = TA ? tid % BK : tid % BM;
-  const int a_var = TA ? tid / BK : tid / BM;
-  constexpr int a_step = TA ? NT / BK : NT / BM;
-  const int b_fix = TB ? tid % BN : tid % BK;
-  const int b_var = TB ? tid / BN : tid / BK;
-  constexpr int b_step = TB ? NT / BN : NT / BK;
+  // K range: a lower-triangular A has no terms beyond the tile's last row
+  const int kall = g.tri_a ? min(g.K, m0 + BM) : g.K;
+  const int kb = split * g.kchunk;
+  const int ke = min(kall, kb + g.kchunk);
+  const int nslab = ke > kb ? (ke - kb + BK - 1) / BK : 0;
 
-  double ra[LA], rb[LB];
+  // this thread's pair i of the A slab: column c of ACOLS, row r + i * NT / ACOLS
+  const int ac = tid % ACOLS, ar = tid / ACOLS;
+  const int bc = tid % BCOLS, br = tid / BCOLS;
+  constexpr int AR = NT / ACOLS, BR = NT / BCOLS;
+  static_assert(NT % ACOLS == 0 && NT % BCOLS == 0, "walk");
+  // pairs past the edge of an operand read its last row again: the element
+  // distance of a pair along m (n) is then 0
+  const bool full = m0 + BM <= g.M && n0 + BN <= g.N;
+  const int am = min(m0 + 2 * ac, g.M - 1), bnn = min(n0 + 2 * bc, g.N - 1);
+  const int a2 = m0 + 2 * ac + 1 < g.M ? 1 : 0, b2 = n0 + 2 * bc + 1 < g.N ? 1 : 0;
+  // running pointers to this thread's first pair of the next slab
+  const double* __restrict__ pa =
+      TA ? A + kb + 2 * ac + (int64_t)(m0 + ar) * g.lda : A + am + (int64_t)(kb + ar) * g.lda;
+  const double* __restrict__ pb =
+      TB ? B + bnn + (int64_t)(kb + br) * g.ldb : B + kb + 2 * bc + (int64_t)(n0 + br) * g.ldb;
+  const int64_t aslab = TA ? BK : BK * g.lda, bslab = TB ? BK * g.ldb : BK;
+  const int64_t astep = AR * g.lda, bstep = BR * g.ldb;
 
-  auto load_slab = [&](int k0) {
+  // the slab's values on their way from memory to LDS; the scales of k are
+  // applied there, so that no load is waited for before the MFMAs it runs under
+  d2 ra[LA], rb[LB], rk[LB];
+  auto load_slab = [&](int k0) __attribute__((always_inline)) {
+    if (k0 + BK <= ke && full) {
 #pragma unroll
-    for (int i = 0; i < LA; ++i) {
-      const int v = a_var + i * a_step;
-      const int gm = m0 + (TA ? v : a_fix);
-      const int gk = k0 + (TA ? a_fix : v);
-      double x = 0.0;
-      if (gm < g.M && gk < g.K && (!g.tri_a || gk <= gm))
-        x = TA ? A[gk + (int64_t)gm * g.lda] : A[gm + (int64_t)gk * g.lda];
-      ra[i] = x;
-    }
-#pragma unroll
-    for (int i = 0; i < LB; ++i) {
-      const int v = b_var + i * b_step;
-      const int gn = n0 + (TB ? b_fix : v);
-      const int gk = k0 + (TB ? v : b_fix);
-      double x = 0.0;
-      if (gn < g.N && gk < g.K) {
-        x = TB ? B[gn + (int64_t)gk * g.ldb] : B[gk + (int64_t)gn * g.ldb];
-        if (ks) x *= ks[gk];
+      for (int i = 0; i < LA; ++i) {
+        if (PA % NT != 0 && tid + i * NT >= PA) break;
+        ra[i] = *reinterpret_cast<const d2u*>(pa + i * astep);
       }
-      rb[i] = x;
+#pragma unroll
+      for (int i = 0; i < LB; ++i) {
+        if (PB % NT != 0 && tid + i * NT >= PB) break;
+        rb[i] = *reinterpret_cast<const d2u*>(pb + i * bstep);
+      }
+      if (ks) {
+#pragma unroll
+        for (int i = 0; i < LB; ++i) {
+          if (TB) rk[i] = d2{ks[k0 + br + i * BR], 0.0};
+          else rk[i] = d2{ks[k0 + 2 * bc], ks[k0 + 2 * bc + 1]};
+        }
+      }
+    } else if (k0 + BK <= ke) {
+      // a tile at the edge
+#pragma unroll
+      for (int i = 0; i < LA; ++i) {
+        if (PA % NT != 0 && tid + i * NT >= PA) break;
+        if (TA) {
+          ra[i] = *reinterpret_cast<const d2u*>(A + k0 + 2 * ac + (int64_t)min(m0 + ar + i * AR, g.M - 1) * g.lda);
+        } else {
+          const double* __restrict__ q = pa + i * astep;
+          ra[i] = d2{q[0], q[a2]};
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < LB; ++i) {
+        if (PB % NT != 0 && tid + i * NT >= PB) break;
+        if (TB) {
+          const double* __restrict__ q = pb + i * bstep;
+          rb[i] = d2{q[0], q[b2]};
+          if (ks) rk[i] = d2{ks[k0 + br + i * BR], 0.0};
+        } else {
+          rb[i] = *reinterpret_cast<const d2u*>(B + k0 + 2 * bc + (int64_t)min(n0 + br + i * BR, g.N - 1) * g.ldb);
+          if (ks) rk[i] = d2{ks[k0 + 2 * bc], ks[k0 + 2 * bc + 1]};
+        }
+      }
+    } else {
+      // the slab cut by the end of K: zeros past it, in both operands
+#pragma unroll
+      for (int i = 0; i < LA; ++i) {
+        const int r = ar + i * AR;
+        if (PA % NT != 0 && tid + i * NT >= PA) break;
+        ra[i] = d2{0.0, 0.0};
+        if (TA) {
+          const int k = k0 + 2 * ac;
+          const double* __restrict__ q = A + k + (int64_t)min(m0 + r, g.M - 1) * g.lda;
+          if (k < ke) ra[i][0] = q[0];
+          if (k + 1 < ke) ra[i][1] = q[1];
+        } else if (k0 + r < ke) {
+          const double* __restrict__ q = pa + i * astep;
+          ra[i] = d2{q[0], q[a2]};
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < LB; ++i) {
+        const int r = br + i * BR;
+        if (PB % NT != 0 && tid + i * NT >= PB) break;
+        rb[i] = d2{0.0, 0.0};
+        rk[i] = d2{0.0, 0.0};
+        if (TB) {
+          if (k0 + r < ke) {
+            const double* __restrict__ q = pb + i * bstep;
+            rb[i] = d2{q[0], q[b2]};
+            if (ks) rk[i][0] = ks[k0 + r];
+          }
+        } else {
+          const int k = k0 + 2 * bc;
+          const double* __restrict__ q = B + k + (int64_t)min(n0 + r, g.N - 1) * g.ldb;
+          if (k < ke) {
+            rb[i][0] = q[0];
+            if (ks) rk[i][0] = ks[k];
+          }
+          if (k + 1 < ke) {
+            rb[i][1] = q[1];
+            if (ks) rk[i][1] = ks[k + 1];
+          }
+        }
+      }
     }
+    pa += aslab;
+    pb += bslab;
   };
-  auto store_slab = [&](int buf) {
+  auto store_slab = [&](int buf) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < LA; ++i) {
-      const int v = a_var + i * a_step;
-      if (TA) As[buf][a_fix][v] = ra[i]; else As[buf][v][a_fix] = ra[i];
+      const int r = ar + i * AR;
+      if (PA % NT != 0 && tid + i * NT >= PA) break;
+      if (TA) {
+        As[buf][2 * ac][r] = ra[i][0];
+        As[buf][2 * ac + 1][r] = ra[i][1];
+      } else {
+        *reinterpret_cast<d2*>(&As[buf][r][2 * ac]) = ra[i];
+      }
+    }
+    if (ks) {
+#pragma unroll
+      for (int i = 0; i < LB; ++i) {
+        rb[i][0] *= rk[i][0];
+        rb[i][1] *= TB ? rk[i][0] : rk[i][1];
+      }
     }
 #pragma unroll
     for (int i = 0; i < LB; ++i) {
-      const int v = b_var + i * b_step;
-      if (TB) Bs[buf][v][b_fix] = rb[i]; else Bs[buf][b_fix][v] = rb[i];
+      const int r = br + i * BR;
+      if (PB % NT != 0 && tid + i * NT >= PB) break;
+      if (TB) {
+        *reinterpret_cast<d2*>(&Bs[buf][r][2 * bc]) = rb[i];
+      } else {
+        Bs[buf][2 * bc][r] = rb[i][0];
+        Bs[buf][2 * bc + 1][r] = rb[i][1];
+      }
     }
   };
 
@@ -170,18 +317,16 @@ gemm_f64_kernel(GemmDev g) {
 #pragma unroll
     for (int j = 0; j < FN; ++j) acc[i][j] = d4{0.0, 0.0, 0.0, 0.0};
 
-  // a lower-triangular A has no terms beyond the tile's last row
-  const int kend = g.tri_a ? min(g.K, m0 + BM) : g.K;
-  const int nslab = (kend + BK - 1) / BK;
-  load_slab(0);
-  store_slab(0);
-  __syncthreads();
+  // a wave whose tile lies past the edge or above the diagonal of a symmetric
+  // update only helps to load
+  const int mw = m0 + wm * TM, nw = n0 + wn * TN;
+  const bool active = __builtin_amdgcn_readfirstlane(mw < g.M && nw < g.N && (!g.lower_only || mw + TM - 1 >= nw));
 
   const int fr = lane & 15;
   const int fk = lane >> 4;
-  for (int s = 0; s < nslab; ++s) {
-    const int buf = s & 1;
-    if (s + 1 < nslab) load_slab((s + 1) * BK);
+  auto compute = [&](int buf) __attribute__((always_inline)) {
+    if (!active) return;
+    if (PRIO) __builtin_amdgcn_s_setprio(1);
 #pragma unroll
     for (int k4 = 0; k4 < BK / 4; ++k4) {
       double af[FM], bf[FN];
@@ -195,14 +340,32 @@ gemm_f64_kernel(GemmDev g) {
         for (int j = 0; j < FN; ++j)
           acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(bf[j], af[i], acc[i][j], 0, 0, 0);
     }
-    if (s + 1 < nslab) store_slab(buf ^ 1);
-    __syncthreads();
+    if (PRIO) __builtin_amdgcn_s_setprio(0);
+  };
+
+  if (nslab > 0) {
+    load_slab(kb);
+    if constexpr (NBUF == 2) {
+      store_slab(0);
+      __syncthreads();
+      for (int s = 0; s < nslab; ++s) {
+        if (s + 1 < nslab) load_slab(kb + (s + 1) * BK);
+        compute(s & 1);
+        if (s + 1 < nslab) store_slab((s & 1) ^ 1);
+        __syncthreads();
+      }
+    } else {
+      for (int s = 0; s < nslab; ++s) {
+        store_slab(0);
+        __syncthreads();
+        if (s + 1 < nslab) load_slab(kb + (s + 1) * BK);
+        compute(0);
+        __syncthreads();
+      }
+    }
   }
 
   // ------------------------------------------------------------ epilogue
-  double* __restrict__ C = g.C ? g.C + (int64_t)batch * g.strideC : nullptr;
-  const double* __restrict__ dg = g.diag_add ? g.diag_add + (int64_t)batch * g.strideDiag : nullptr;
-
   if constexpr (DOT) {
     // Column dots of this row block: sum_m C(m,n) (cc C(m,n) + cd D(m,n)),
     // or sum_m w(m) C(m,n)^2 without D (w = 1 without row weights).
@@ -245,6 +408,10 @@ gemm_f64_kernel(GemmDev g) {
     return;
   }
 
+  double* __restrict__ C = g.C + (int64_t)batch * g.strideC;
+  const double* __restrict__ dg = g.diag_add ? g.diag_add + (int64_t)batch * g.strideDiag : nullptr;
+  double* __restrict__ P =
+      g.part ? g.part + ((int64_t)split * g.batch + batch) * (int64_t)g.M * g.N : nullptr;
 #pragma unroll
   for (int i = 0; i < FM; ++i) {
     const int m = m0 + wm * TM + i * 16 + fr;
@@ -255,20 +422,28 @@ gemm_f64_kernel(GemmDev g) {
         const int n = n0 + wn * TN + j * 16 + fk + 4 * r;
         if (m >= g.M || n >= g.N) continue;
         if (g.lower_only && m < n) continue;
-        double v = g.alpha * acc[i][j][r];
-        if (g.rowscale) v *= g.rowscale[m];
-        if (g.colscale) v *= g.colscale[n];
-        if (dg && m == n) v += dg[m];
-        const int64_t idx = m + (int64_t)n * g.ldc;
-        if (g.beta != 0.0) v += g.beta * C[idx];
-        C[idx] = v;
-        if (g.lower_only && m > n && !g.no_mirror) C[n + (int64_t)m * g.ldc] = g.upper_zero ? 0.0 : v;
+        if (P) P[m + (int64_t)n * g.M] = acc[i][j][r];
+        else store_result(g, C, dg, m, n, acc[i][j][r]);
       }
     }
   }
 }
 
-template <int BM, int BN, int WM, int WN, int BK, bool DOT, int KLASS>
+// Sum of the K splits in order, then the epilogue. Memory-bound: a thread
+// owns one (m, n) of one batch entry, consecutive threads consecutive m.
+__global__ void __launch_bounds__(256) gemm_f64_reduce_kernel(GemmDev g) {
+  const int m = blockIdx.x * 256 + threadIdx.x, n = blockIdx.y, b = blockIdx.z;
+  if (m >= g.M || (g.lower_only && m < n)) return;
+  const int64_t mn = (int64_t)g.M * g.N;
+  const double* __restrict__ p = g.part + (int64_t)b * mn + m + (int64_t)n * g.M;
+  double s = 0.0;
+  for (int q = 0; q < g.splits; ++q) s += p[(int64_t)q * g.batch * mn];
+  store_result(g, g.C + (int64_t)b * g.strideC, g.diag_add ? g.diag_add + (int64_t)b * g.strideDiag : nullptr, m, n,
+               s);
+}
+
+// NB: B not transposed only (column tiles that are no power of two)
+template <int BM, int BN, int WM, int WN, bool DOT, int KLASS, bool NB = false>
 int launch_cfg(const GemmF64& h, hipStream_t stream) {
   GemmDev g;
   g.M = h.M; g.N = h.N; g.K = h.K;
@@ -290,39 +465,50 @@ int launch_cfg(const GemmF64& h, hipStream_t stream) {
   g.dotB = h.dotB; g.lddot = h.lddot; g.dotpart = h.dotpart; g.strideDot = h.strideDot;
   g.dot_cc = h.dot_cc; g.dot_cd = h.dot_cd;
   g.dot_w = h.dot_w; g.strideDotW = h.strideDotW;
+  g.splits = std::max(1, h.splits);
+  g.kchunk = ((h.K + g.splits - 1) / g.splits + BK - 1) / BK * BK;
+  g.part = g.splits > 1 ? h.split_work : nullptr;
+  MGW_REQUIRE(g.splits == 1 || (h.split_work && !h.dotpart && h.N <= 65535 && h.batch <= 65535), MGW_ERR_ARG,
+              "gemm_f64: a split K needs a workspace and a plain output");
   // square-tile symmetric updates enumerate the lower triangle of tiles only;
   // other lower-only shapes launch the full grid and skip upper tiles
   const int64_t tiles = (h.lower_only && BM == BN) ? (int64_t)g.tiles_m * (g.tiles_m + 1) / 2
                                                    : (int64_t)g.tiles_m * g.tiles_n;
-  g.nblocks = tiles * h.batch;
-  MGW_REQUIRE(tiles < (1ll << 31) && g.nblocks < (1ll << 31), MGW_ERR_ARG, "gemm_f64: too many tiles");
+  g.nblocks = tiles * g.splits * h.batch;
+  MGW_REQUIRE(tiles * g.splits < (1ll << 31) && g.nblocks < (1ll << 31), MGW_ERR_ARG, "gemm_f64: too many tiles");
   MGW_REQUIRE(h.batch >= 1, MGW_ERR_ARG, "gemm_f64: batch out of range");
   dim3 grid((unsigned)g.nblocks, 1, 1);
   dim3 block(64 * WM * WN, 1, 1);
   const int ta = h.transA ? 1 : 0, tb = h.transB ? 1 : 0;
 #define MGW_GEMM_CASE(TA_, TB_)                                                                        \
-  if (ta == TA_ && tb == TB_) {                                                                        \
-    hipLaunchKernelGGL((gemm_f64_kernel<BM, BN, WM, WN, BK, TA_, TB_, DOT, KLASS>), grid, block, 0,    \
-                       stream, g);                                                                     \
-  }
+  if constexpr (!(NB && TB_))                                                                          \
+    if (ta == TA_ && tb == TB_)                                                                        \
+      hipLaunchKernelGGL((gemm_f64_kernel<BM, BN, WM, WN, TA_, TB_, DOT, KLASS>), grid, block, 0,      \
+                         stream, g);
   MGW_GEMM_CASE(0, 0)
   MGW_GEMM_CASE(0, 1)
   MGW_GEMM_CASE(1, 0)
   MGW_GEMM_CASE(1, 1)
 #undef MGW_GEMM_CASE
   MGW_HIP(hipGetLastError());
+  if (g.splits > 1) {
+    hipLaunchKernelGGL(gemm_f64_reduce_kernel, dim3((h.M + 255) / 256, h.N, h.batch), dim3(256), 0, stream, g);
+    MGW_HIP(hipGetLastError());
+  }
   return MGW_OK;
 }
 
 }  // namespace
 
-int gemm_f64_rowblocks(int M) { return (M + 127) / 128; }   // row tile of the dot epilogue
+// Row blocks of the dot epilogue: 64x64 tiles, whose triangular K ranges stop
+// closer to the diagonal and of which four share a CU (naux 1372, 6304 columns,
+// 16 frequencies: 3.86 ms against 4.53 for 128x128 and 4.15 for 128x64).
+int gemm_f64_dot_rowblocks(int M) { return (M + 63) / 64; }
 
 // ------------------------------------------------------------------ autotuner
 // Candidate tile configurations (all FP64 MFMA, BK = 16):
 //   0: 256x128, 16 waves   1: 128x128, 8 waves   2: 128x128, 4 waves   3: 64x64, 4 waves
-// The defaults were measured on MI355X (0 for large products, 1 for the
-// long-K symmetric update). With tuning on, the first product of a new
+// The defaults (2, and 3 for small products) were measured on MI355X. With tuning on, the first product of a new
 // (class, transposes, lower, log2 M/N/K bucket) times every candidate on
 // the actual operands and keeps the fastest; the table can be persisted.
 namespace {
@@ -373,10 +559,10 @@ void load_table(Tuner& t) {
 template <int KLASS>
 int launch_candidate(int cfg, const GemmF64& h, hipStream_t stream) {
   switch (cfg) {
-    case 0: return launch_cfg<256, 128, 4, 4, 16, false, KLASS>(h, stream);
-    case 1: return launch_cfg<128, 128, 4, 2, 16, false, KLASS>(h, stream);
-    case 2: return launch_cfg<128, 128, 2, 2, 16, false, KLASS>(h, stream);
-    default: return launch_cfg<64, 64, 2, 2, 16, false, KLASS>(h, stream);
+    case 0: return launch_cfg<256, 128, 4, 4, false, KLASS>(h, stream);
+    case 1: return launch_cfg<128, 128, 4, 2, false, KLASS>(h, stream);
+    case 2: return launch_cfg<128, 128, 2, 2, false, KLASS>(h, stream);
+    default: return launch_cfg<64, 64, 2, 2, false, KLASS>(h, stream);
   }
 }
 
@@ -389,6 +575,65 @@ int launch_by_class(int cfg, const GemmF64& h, hipStream_t stream) {
     case MGW_KCLASS_CHOLESKY: return launch_candidate<MGW_KCLASS_CHOLESKY>(cfg, h, stream);
     default: return launch_candidate<MGW_KCLASS_GEMM_OTHER>(cfg, h, stream);
   }
+}
+
+// Column tiles of 16 FN < 128 columns for products of few columns (the
+// transforms of the occupied states or of a window, the exchange's half
+// transform): the FN whose tiles cover N in the least time, 0 when 128-column
+// tiles do. In units of 16 columns at 1 TFLOP/s, measured at 65536 x 16 FN x
+// 4096: FN = 1 .. 8 run at 23, 38, 42, 48, 58, 53, 56 and 65 TFLOP/s (up to 3
+// the rows' traffic bounds them); a workgroup's fixed cost is that of 60 k, or
+// of 150 for the two widest, of which only two share a CU.
+int narrow_fn(int N, int K) {
+  constexpr double w[9] = {0.0, 1 / 23.0, 2 / 38.0, 3 / 42.0, 4 / 48.0, 5 / 58.0, 6 / 53.0, 7 / 56.0, 8 / 65.0};
+  auto cost = [&](int fn) { return (N + 16 * fn - 1) / (16 * fn) * w[fn] * (K + (fn >= 7 ? 150.0 : 60.0)); };
+  int best = 8;
+  for (int fn = 7; fn >= 1; --fn)
+    if (cost(fn) < cost(best)) best = fn;
+  return best == 8 ? 0 : best;
+}
+
+template <int KLASS>
+int launch_narrow(int fn, const GemmF64& h, hipStream_t stream) {
+  switch (fn) {
+    case 1: return launch_cfg<128, 16, 4, 1, false, KLASS, true>(h, stream);
+    case 2: return launch_cfg<128, 32, 4, 1, false, KLASS, true>(h, stream);
+    case 3: return launch_cfg<128, 48, 4, 1, false, KLASS, true>(h, stream);
+    case 4: return launch_cfg<128, 64, 2, 2, false, KLASS, true>(h, stream);
+    case 5: return launch_cfg<128, 80, 4, 1, false, KLASS, true>(h, stream);
+    case 6: return launch_cfg<128, 96, 2, 2, false, KLASS, true>(h, stream);
+    default: return launch_cfg<128, 112, 4, 1, false, KLASS, true>(h, stream);
+  }
+}
+
+int64_t tile_count(int M, int N, int batch, bool lower, int b) {
+  const int64_t tm = (M + b - 1) / b, tn = (N + b - 1) / b;
+  return (lower ? tm * (tm + 1) / 2 : tm * tn) * batch;
+}
+
+// Cost in cycles of a plain product on b x b tiles (128 or 64) with the K range
+// in s splits. Two workgroups of 128x128 or four of 64x64 share a CU's four
+// SIMDs; a round of them lasts as long as its K range plus a fixed prologue
+// and epilogue. A k step costs the sharing workgroups' MFMA cycles at the
+// part of the peak that they reach together (128x128: 0.55 alone, 0.85 for
+// two; 64x64: 0.25, 0.45, 0.6, 0.68), so a last round that does not fill the
+// slots is cheaper than a whole one. Partial products are written and read
+// once at HBM's copy rate (1.9 KB per cycle).
+double tile_cost(int M, int N, int K, int batch, bool lower, int b, int s) {
+  const int64_t tiles = tile_count(M, N, batch, lower, b) * s;
+  constexpr double step128[3] = {0.0, 256.0 / 0.55, 512.0 / 0.85};
+  constexpr double step64[5] = {0.0, 64.0 / 0.25, 128.0 / 0.45, 192.0 / 0.6, 256.0 / 0.68};
+  const double* step = b == 128 ? step128 : step64;
+  const int share = b == 128 ? 2 : 4, slots = 256 * share;
+  double c = ((double)K / s + 48.0) * ((double)(tiles / slots) * step[share] + step[(tiles % slots + 255) / 256]);
+  if (s > 1) c += 10000.0 + 16.0 * s * M * (double)N * batch * (lower ? 0.5 : 1.0) / 1900.0;
+  return c;
+}
+
+// Tiles: 128x128 with four waves, or 64x64 (also when a product fits one such
+// tile: the larger one only adds idle waves).
+int default_cfg(int M, int N, int K, int batch, bool lower, int s) {
+  return tile_cost(M, N, K, batch, lower, 64, s) <= tile_cost(M, N, K, batch, lower, 128, s) ? 3 : 2;
 }
 
 int tune(const GemmF64& h, hipStream_t stream, int* best) {
@@ -412,6 +657,26 @@ int tune(const GemmF64& h, hipStream_t stream, int* best) {
 }
 
 }  // namespace
+
+// K splits of a plain product: the cheapest count by tile_cost. A function of
+// the shape only, so every tile configuration sums in the same order.
+int gemm_f64_splits(int M, int N, int K, int batch, bool lower) {
+  int best = 1;
+  double cost = 0.0;
+  // at most 2 GiB of partial products
+  for (int s = 1; s <= 256 && (s == 1 || (K / s >= 64 && (double)s * M * N * batch <= 268435456.0)); ++s) {
+    const double c = std::min(tile_cost(M, N, K, batch, lower, 128, s), tile_cost(M, N, K, batch, lower, 64, s));
+    if (s == 1 || c < cost) {
+      cost = s == 1 ? 0.95 * c : c;
+      best = s;
+    }
+  }
+  return best;
+}
+
+size_t gemm_f64_split_doubles(int M, int N, int batch, int splits) {
+  return splits > 1 ? (size_t)splits * batch * M * N : 0;
+}
 
 int gemm_autotune_mode(int mode) {
   Tuner& t = tuner();
@@ -490,24 +755,16 @@ int gemm_f64(const GemmF64& h, hipStream_t stream) {
   MGW_REQUIRE(!h.tri_a || (!h.transA && h.M == h.K), MGW_ERR_ARG,
               "gemm_f64: a triangular A must be square and not transposed");
   MGW_REQUIRE(h.dotpart != nullptr || h.C != nullptr, MGW_ERR_ARG, "gemm_f64: no output");
-  if (h.dotpart) return launch_cfg<128, 128, 4, 2, 16, true, MGW_KCLASS_GEMM_WB>(h, stream);
-  // Skinny N: a 256 x 32 tile keeps the matrix cores busy when N is small.
-  if (h.N <= 32 && !h.lower_only) return launch_cfg<256, 32, 4, 1, 16, false, MGW_KCLASS_GEMM_AO2MO>(h, stream);
-  // Defaults measured on MI355X: 256x128 with 16 waves for the large products
-  // (57-62 TF/s), 128x128 with 8 waves for the long-K symmetric updates;
-  // 64x64 tiles when the default would leave most of the 256 CUs idle (the
-  // block columns of the batched Cholesky, small molecules), also when they
-  // give as many workgroups (a product that fits one 64x64 tile: the larger
-  // tiles only add idle waves; the tuner picks 64x64 for every such product
-  // of the Cholesky, 4.26 -> 3.91 ms per solve on the FP16x3 stream).
-  int cfg = h.lower_only ? 1 : 0;
-  {
-    auto wgs = [&](int bm, int bn) {
-      const int64_t tm = (h.M + bm - 1) / bm, tn = (h.N + bn - 1) / bn;
-      return (h.lower_only && bm == bn ? tm * (tm + 1) / 2 : tm * tn) * h.batch;
-    };
-    const int64_t have = h.lower_only ? wgs(128, 128) : wgs(256, 128);
-    if (have < 512 && wgs(64, 64) >= have) cfg = 3;
+  if (h.dotpart) return launch_cfg<64, 64, 2, 2, true, MGW_KCLASS_GEMM_WB>(h, stream);
+  int cfg = default_cfg(h.M, h.N, h.K, h.batch, h.lower_only, std::max(1, h.splits));
+  // few columns, and rows enough to fill the GPU: column tiles that N fills
+  if (h.splits <= 1 && !h.transB && !h.lower_only && h.N < 1024 &&
+      ((int64_t)h.M + 127) / 128 * ((h.N + 111) / 112) * h.batch >= 512) {
+    const int fn = narrow_fn(h.N, h.K);
+    if (fn > 0)
+      return h.klass == MGW_KCLASS_GEMM_AO2MO ? launch_narrow<MGW_KCLASS_GEMM_AO2MO>(fn, h, stream)
+                                              : launch_narrow<MGW_KCLASS_GEMM_OTHER>(fn, h, stream);
+    cfg = 2;
   }
   Tuner& t = tuner();
   const TuneKey key{h.klass, h.transA ? 1 : 0, h.transB ? 1 : 0, h.lower_only ? 1 : 0,

@@ -108,7 +108,7 @@ struct GemmF64 {
   bool lower_only = false;
   bool no_mirror = false;     // lower_only: do not mirror into the upper triangle
   bool upper_zero = false;    // lower_only: write zeros, not the mirror, above the diagonal
-  bool tri_a = false;         // A (not transposed, M == K) is lower triangular
+  bool tri_a = false;         // A (not transposed, M == K) is lower triangular, zeros stored above the diagonal
   bool batch_outer = false;   // tiles of one batch entry before the next (no shared operands)
   // Fused column dot: instead of storing C, accumulate
   // dotpart[(rowblock * N + n) + batch * strideDot]
@@ -120,6 +120,10 @@ struct GemmF64 {
   double dot_cc = 0.0, dot_cd = 1.0;
   double* dotpart = nullptr; int64_t strideDot = 0;
   const double* dot_w = nullptr; int64_t strideDotW = 0;
+  // K split into `splits` partial products (gemm_f64_splits) kept in
+  // split_work (gemm_f64_split_doubles) and summed in order (FP64, no dots)
+  int splits = 1;
+  double* split_work = nullptr;
   // kernel class: the hot classes get their own kernel symbol so that
   // profiler per-kernel statistics separate them
   int klass = MGW_KCLASS_GEMM_OTHER;
@@ -151,11 +155,14 @@ size_t chi0_split_bytes_per_frequency(int naux, int npole, int precision, int no
 size_t chi0_split_workspace(int naux, int npole, int nomega, int precision);
 int chi0_split_syrk(const double* x, int naux, int npole, const double* sw, int nomega, int precision,
                     void* work, size_t work_bytes, double* chi, hipStream_t stream);
-int gemm_f64_rowblocks(int M);
+int gemm_f64_dot_rowblocks(int M);   // row blocks of the FP64 dot epilogue's partials
+int gemm_f64_splits(int M, int N, int K, int batch, bool lower);
+size_t gemm_f64_split_doubles(int M, int N, int batch, int splits);
 // v(n, f) = B_n^T chi(iw_f) B_n = sum_m C (C + 2 B), C = D_f B, from bf16-split
 // operands (MGW_BF16X3 / MGW_BF16X6) of D_f = L_f^-1 - 1 (lower triangle of
 // naux x naux, stride naux^2) and B (naux x ncol); writes the row-block
-// partials dotpart[(f * gemm_f64_rowblocks(naux) + rb) * ncol + n].
+// partials dotpart[(f * wb_split_rowblocks(naux) + rb) * ncol + n].
+int wb_split_rowblocks(int M);
 size_t wb_split_workspace(int naux, int64_t ncol, int nomega, int precision);
 int wb_split_dot(const double* d, int naux, int nomega, const double* b, int64_t ncol, int precision, void* work,
                  size_t work_bytes, double* dotpart, hipStream_t stream);
