@@ -667,10 +667,10 @@ int gw_selfenergy(mgw_ctx* c, const mgw_ranges* r, double spin_fact, double eta,
   double *sigma, *egw_p, *part;
   MGW_TRY(dbuf(c, "sigma", (size_t)2 * nomega * nse, &sigma));
   MGW_TRY(dbuf(c, "sigma_egw", nse, &egw_p));
-  MGW_TRY(dbuf(c, "sigma_part", (size_t)sigma_part_doubles(npole, nse), &part));
   // chunk over i so that w(s, p, i) stays within ~1 GiB
   const size_t per_i = (size_t)npole * nse * sizeof(double);
   int ic = (int)std::max<size_t>(1, std::min<size_t>((size_t)ng, (size_t(1) << 30) / per_i));
+  MGW_TRY(dbuf(c, "sigma_part", (size_t)sigma_part_doubles(npole, nse, ic, nomega), &part));
   double* w = nullptr;
   MGW_TRY(dbuf(c, "sigma_w", (size_t)npole * nse * ic, &w));
   const double* ws = find_buf(c, "wpol_ws");

@@ -147,6 +147,144 @@ int launch_symmetrize(double* m, int n, hipStream_t s) {
   return MGW_OK;
 }
 
+// ------------------------------------------------------------------ Hartree
+// gamma(P) = scale sum_{k, i} h(P, i, k) x(k, i): h (naux x nx x nbf, the half
+// transform of the exchange) is read once, so HBM bounds it. A workgroup owns
+// 64 rows P and a chunk of the columns (i, k); its four waves take every
+// fourth column, four at a time, and the chunks' partial sums are added in
+// order by gamma_reduce_kernel.
+constexpr int GAMMA_ROWS = 64;
+
+__global__ void __launch_bounds__(256)
+gamma_kernel(const double* __restrict__ h, const double* __restrict__ x, int naux, int nbf, int nx, int64_t chunk,
+             double* __restrict__ part) {
+  __shared__ double red[4][GAMMA_ROWS];
+  __shared__ double xs[256];          // x of the next 256 columns
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int P = blockIdx.x * GAMMA_ROWS + lane;
+  const int64_t ncol = (int64_t)nx * nbf;
+  const int64_t c0 = blockIdx.y * chunk, c1 = min(ncol, c0 + chunk);
+  double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
+  for (int64_t cb = c0; cb < c1; cb += 256) {
+    const int n = (int)min((int64_t)256, c1 - cb);
+    __syncthreads();
+    if ((int)threadIdx.x < n) {
+      const int64_t c = cb + threadIdx.x;
+      xs[threadIdx.x] = x[c / nx + (int64_t)nbf * (c % nx)];
+    }
+    __syncthreads();
+    if (P >= naux) continue;
+    const double* __restrict__ q = h + P + cb * naux;
+    int j = wv;
+    for (; j + 12 < n; j += 16) {
+      a0 = fma(q[(int64_t)j * naux], xs[j], a0);
+      a1 = fma(q[(int64_t)(j + 4) * naux], xs[j + 4], a1);
+      a2 = fma(q[(int64_t)(j + 8) * naux], xs[j + 8], a2);
+      a3 = fma(q[(int64_t)(j + 12) * naux], xs[j + 12], a3);
+    }
+    for (; j < n; j += 4) a0 = fma(q[(int64_t)j * naux], xs[j], a0);
+  }
+  red[wv][lane] = (a0 + a1) + (a2 + a3);
+  __syncthreads();
+  if (wv == 0 && P < naux)
+    part[(int64_t)blockIdx.y * naux + P] = (red[0][lane] + red[1][lane]) + (red[2][lane] + red[3][lane]);
+}
+
+__global__ void __launch_bounds__(256)
+gamma_reduce_kernel(const double* __restrict__ part, int nchunk, int naux, double scale, double* __restrict__ gamma) {
+  __shared__ double red[4][GAMMA_ROWS];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int P = blockIdx.x * GAMMA_ROWS + lane;
+  double s = 0.0;
+  if (P < naux)
+    for (int c = wv; c < nchunk; c += 4) s += part[(int64_t)c * naux + P];
+  red[wv][lane] = s;
+  __syncthreads();
+  if (wv == 0 && P < naux) gamma[P] = scale * ((red[0][lane] + red[1][lane]) + (red[2][lane] + red[3][lane]));
+}
+
+// column chunks: about eight workgroups per CU, at least 64 columns each
+static int64_t gamma_chunk(int naux, int nbf, int nx) {
+  const int64_t ncol = (int64_t)nx * nbf, rows = nblocks(naux, GAMMA_ROWS);
+  const int64_t want = std::max<int64_t>(1, std::min<int64_t>(2048 / std::max<int64_t>(1, rows), ncol / 64));
+  return (ncol + want - 1) / want;
+}
+
+int64_t hartree_part_doubles(int naux, int nbf, int nx) {
+  const int64_t ncol = (int64_t)nx * nbf, chunk = gamma_chunk(naux, nbf, nx);
+  return (ncol + chunk - 1) / chunk * naux;
+}
+
+int launch_hartree_gamma(const double* h, const double* x, int naux, int nbf, int nx, double scale, double* part,
+                         double* gamma, hipStream_t s) {
+  const int64_t ncol = (int64_t)nx * nbf, chunk = gamma_chunk(naux, nbf, nx);
+  const int nchunk = (int)((ncol + chunk - 1) / chunk);
+  hipLaunchKernelGGL(gamma_kernel, dim3(nblocks(naux, GAMMA_ROWS), nchunk), dim3(256), 0, s, h, x, naux, nbf, nx,
+                     chunk, part);
+  MGW_LAUNCH_CHECK();
+  hipLaunchKernelGGL(gamma_reduce_kernel, dim3(nblocks(naux, GAMMA_ROWS)), dim3(256), 0, s, part, nchunk, naux, scale,
+                     gamma);
+  MGW_LAUNCH_CHECK();
+  return MGW_OK;
+}
+
+// j(k, l) = sum_P B(P, k, l) gamma(P), one wave per column (k, l) of the lower
+// triangle: B is symmetric in (k, l), so half of the tensor is read, and HBM
+// bounds it.
+__global__ void __launch_bounds__(256)
+hartree_j_kernel(const double* __restrict__ b, const double* __restrict__ gamma, int naux, int nbf,
+                 double* __restrict__ j) {
+  const int lane = threadIdx.x & 63;
+  const int l = blockIdx.y, k = l + blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (k >= nbf) return;
+  const double* __restrict__ q = b + (int64_t)naux * (k + (int64_t)nbf * l);
+  double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
+  int P = lane;
+  for (; P + 192 < naux; P += 256) {
+    a0 = fma(q[P], gamma[P], a0);
+    a1 = fma(q[P + 64], gamma[P + 64], a1);
+    a2 = fma(q[P + 128], gamma[P + 128], a2);
+    a3 = fma(q[P + 192], gamma[P + 192], a3);
+  }
+  for (; P < naux; P += 64) a0 = fma(q[P], gamma[P], a0);
+  double s = (a0 + a1) + (a2 + a3);
+  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+  if (lane == 0) {
+    j[k + (int64_t)nbf * l] = s;
+    j[l + (int64_t)nbf * k] = s;
+  }
+}
+
+int launch_hartree_j(const double* b, const double* gamma, int naux, int nbf, double* j, hipStream_t s) {
+  MGW_REQUIRE(nbf <= 65535, MGW_ERR_ARG, "hartree_j: nbf out of range");
+  hipLaunchKernelGGL(hartree_j_kernel, dim3(nblocks(nbf, 4), nbf), dim3(256), 0, s, b, gamma, naux, nbf, j);
+  MGW_LAUNCH_CHECK();
+  return MGW_OK;
+}
+
+// ------------------------------------------------------------------ batch sum
+__global__ void __launch_bounds__(256)
+batch_sum_kernel(const double* __restrict__ m, int64_t n, int nbatch, int accumulate, double* __restrict__ out) {
+  __shared__ double red[4][64];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int64_t e = (int64_t)blockIdx.x * 64 + lane;
+  double s = 0.0;
+  if (e < n)
+    for (int b = wv; b < nbatch; b += 4) s += m[e + n * b];
+  red[wv][lane] = s;
+  __syncthreads();
+  if (wv != 0 || e >= n) return;
+  s = (red[0][lane] + red[1][lane]) + (red[2][lane] + red[3][lane]);
+  out[e] = accumulate ? out[e] + s : s;
+}
+
+int launch_batch_sum(const double* m, int64_t n, int nbatch, int accumulate, double* out, hipStream_t s) {
+  if (n <= 0) return MGW_OK;
+  hipLaunchKernelGGL(batch_sum_kernel, dim3(nblocks(n, 64)), dim3(256), 0, s, m, n, nbatch, accumulate, out);
+  MGW_LAUNCH_CHECK();
+  return MGW_OK;
+}
+
 // ------------------------------------------------------------------ max |x|
 __global__ void __launch_bounds__(256)
 absmax_kernel(const double* __restrict__ x, int64_t n, double* __restrict__ part) {
@@ -358,110 +496,175 @@ int launch_casida_post(const double* eig, int npole, double* pole, double* cs, h
 // x = E0_p + w_k - e_i (src/m_gw_selfenergy_analytic.f90:126-133), and
 // E_GW += (1 - f_i) occ_p w^2 / (e_p - e_i - Omega_s) for filled p (:135-138).
 //
-// Workgroup = 4 wave64s for one state p and one block of SB poles. Lane k of
-// every wave owns frequency w_k (nomega <= 63); the spare lane 63 accumulates
-// the E_GW term. Wave j walks the poles s = s0 + j, s0 + j + 4, ... of the
-// block, reading w^2 and Omega from LDS (one coalesced load per block per i).
-// The partial sums of the block are written per (sblock, p) and reduced over
-// blocks by sigma_reduce_kernel: the result does not depend on scheduling.
+// Bound by FP64 VALU issue: 11 instructions per (p, i, s, k) term (a reciprocal
+// estimate, which issues at a quarter of the rate, one Newton step and the
+// quotient's correction in place of the full division sequence, two sums).
+//
+// A workgroup owns one state p, one block of SIGMA_SB poles and a chunk of the
+// states i. Its 256 threads are groups of ceil(nomega / KPT) threads; each
+// thread holds KPT frequencies, and group g walks the poles s = g, g + G, ...
+// reading (w^2, Omega) of a pole from LDS once for its KPT terms. With 51
+// frequencies 247 of the 256 threads work (19 groups of 13), with the single
+// frequency of an eigenvalue self-consistent step all of them. The grid is
+// filled by splitting the states i when poles and states p are few.
+// Partial sums go to part[(i chunk, pole block)][p][k] and are summed in that
+// order by sigma_reduce_kernel: the result does not depend on scheduling.
+// Measured at npole 2457, 202 states p and i, 51 frequencies: 5.6 -> 2.6 ms
 constexpr int SIGMA_SB = 512;
+constexpr int SIGMA_MAXK = 255;    // frequencies per launch
 
+// w / d, correctly rounded but for the last bit; infinities, zeros and NaN as
+// by the division
+__device__ inline double quotient(double w, double d) {
+  double y = __builtin_amdgcn_rcp(d);        // 24 bits, 48 after the step
+  y = fma(y, fma(-d, y, 1.0), y);
+  const double q = w * y;
+  return __builtin_amdgcn_div_fixup(fma(fma(-d, q, w), y, q), d, w);
+}
+
+template <int KPT>
 __global__ void __launch_bounds__(256)
-sigma_poles_kernel(const double* __restrict__ w, int npole, int nse, int ni,
+sigma_poles_kernel(const double* __restrict__ w, int npole, int nse, int ni, int ichunk, int nsblock,
                    const double* __restrict__ pole, const double* __restrict__ omega, int nomega,
                    int with_egw, const double* __restrict__ e0p, const double* __restrict__ ei,
                    const double* __restrict__ fi, const double* __restrict__ ep,
                    const double* __restrict__ occp, double spin_fact, double eta,
-                   double* __restrict__ part /* [nsblock][nse][64] complex */) {
-  __shared__ double w2s[SIGMA_SB];
-  __shared__ double oms[SIGMA_SB];
-  __shared__ double red[4][64][2];
-  const int p = blockIdx.y;
-  const int sb = blockIdx.x;
+                   double* __restrict__ part /* [i chunk][nsblock][nse][nomega + 1] complex */) {
+  __shared__ double2 ws[SIGMA_SB];           // (w^2, Omega)
+  __shared__ double red[256][2];
+  const int p = blockIdx.y, sb = blockIdx.x, tid = threadIdx.x;
   const int s0 = sb * SIGMA_SB;
-  const int lane = threadIdx.x & 63;
-  const int wv = threadIdx.x >> 6;
   const int ns = min(SIGMA_SB, npole - s0);
-  const double om_k = lane < nomega ? omega[lane] : 0.0;
+  const int i0 = blockIdx.z * ichunk, i1 = min(ni, i0 + ichunk);
+  const int tk = (nomega + KPT - 1) / KPT;   // threads per group
+  const int ngroup = 256 / tk;
+  const int grp = tid / tk, kb = tid % tk;
+  const bool on = grp < ngroup;
   const double e0 = e0p[p];
   const bool p_full = ((spin_fact - occp[p]) / spin_fact) < 1.0e-5;
-  const double occ_p = occp[p];
-  const double eps_p = ep[p];
-  const double eta2 = eta * eta;
-  double re = 0.0, im = 0.0, egw = 0.0;
-  for (int s = threadIdx.x; s < ns; s += 256) oms[s] = pole[s0 + s];
-  for (int ii = 0; ii < ni; ++ii) {
+  const double occ_p = occp[p], eps_p = ep[p], eta2 = eta * eta;
+  double om[KPT], re[KPT], im[KPT], egw = 0.0;
+#pragma unroll
+  for (int u = 0; u < KPT; ++u) {
+    const int k = kb + u * tk;
+    om[u] = e0 + (on && k < nomega ? omega[k] : 0.0);
+    re[u] = im[u] = 0.0;
+  }
+  for (int s = tid; s < ns; s += 256) ws[s].y = pole[s0 + s];
+  for (int ii = i0; ii < i1; ++ii) {
     __syncthreads();
     const double* wcol = w + (int64_t)npole * ((int64_t)p + (int64_t)nse * ii) + s0;
-    for (int s = threadIdx.x; s < ns; s += 256) {
+    for (int s = tid; s < ns; s += 256) {
       const double v = wcol[s];
-      w2s[s] = v * v;
+      ws[s].x = v * v;
     }
     __syncthreads();
     const double f_full = fi[ii] / spin_fact;
     const double f_empty = (spin_fact - fi[ii]) / spin_fact;
-    const double x = e0 + om_k - ei[ii];
-    if (lane < nomega) {
-      if (f_full != 0.0) {
-        double sre = 0.0, sim = 0.0;
-        for (int s = wv; s < ns; s += 4) {
-          const double a = x + oms[s];
-          const double r = w2s[s] / (a * a + eta2);
-          sre = fma(a, r, sre);
-          sim += r;
+    const double e_i = ei[ii];
+    // sign +1: occupied i (x + Omega); -1: empty i (x - Omega)
+    for (int branch = 0; branch < 2; ++branch) {
+      const double f = branch == 0 ? f_full : f_empty;
+      if (f == 0.0) continue;
+      if (on) {
+        double sre[KPT], sim[KPT], x[KPT];
+#pragma unroll
+        for (int u = 0; u < KPT; ++u) {
+          sre[u] = sim[u] = 0.0;
+          x[u] = om[u] - e_i;
+          asm("" : "+v"(x[u]));     // held, not subtracted again for every pole
         }
-        re = fma(f_full, sre, re);
-        im = fma(f_full * eta, sim, im);
-      }
-      if (f_empty != 0.0) {
-        double sre = 0.0, sim = 0.0;
-        for (int s = wv; s < ns; s += 4) {
-          const double b = x - oms[s];
-          const double r = w2s[s] / (b * b + eta2);
-          sre = fma(b, r, sre);
-          sim += r;
+        for (int s = grp; s < ns; s += ngroup) {
+          const double w2 = ws[s].x, o = branch == 0 ? ws[s].y : -ws[s].y;
+#pragma unroll
+          for (int u = 0; u < KPT; ++u) {
+            const double a = x[u] + o;
+            const double r = quotient(w2, fma(a, a, eta2));
+            sre[u] = fma(a, r, sre[u]);
+            sim[u] += r;
+          }
         }
-        re = fma(f_empty, sre, re);
-        im = fma(-f_empty * eta, sim, im);
+        const double fe = branch == 0 ? f * eta : -f * eta;
+#pragma unroll
+        for (int u = 0; u < KPT; ++u) {
+          re[u] = fma(f, sre[u], re[u]);
+          im[u] = fma(fe, sim[u], im[u]);
+        }
       }
-    } else if (lane == 63 && with_egw && p_full && f_empty != 0.0) {
-      const double d0 = eps_p - ei[ii];
+    }
+    if (with_egw && p_full && f_empty != 0.0) {
+      const double d0 = eps_p - e_i;
       double acc = 0.0;
-      for (int s = wv; s < ns; s += 4) acc += w2s[s] / (d0 - oms[s]);
+      for (int s = tid; s < ns; s += 256) acc += ws[s].x / (d0 - ws[s].y);
       egw = fma(f_empty * occ_p, acc, egw);
     }
   }
-  red[wv][lane][0] = (lane == 63) ? egw : re;
-  red[wv][lane][1] = (lane == 63) ? 0.0 : im;
-  __syncthreads();
-  if (threadIdx.x < 64) {
-    const int k = threadIdx.x;
-    double r0 = 0.0, r1 = 0.0;
-    for (int j = 0; j < 4; ++j) { r0 += red[j][k][0]; r1 += red[j][k][1]; }
-    double* out = part + 2 * (64 * ((int64_t)sb * nse + p) + k);
-    out[0] = r0;
-    out[1] = r1;
+  double* __restrict__ out =
+      part + 2 * (int64_t)(nomega + 1) * (((int64_t)blockIdx.z * nsblock + sb) * nse + p);
+  // sum over the groups, in order
+#pragma unroll
+  for (int u = 0; u < KPT; ++u) {
+    __syncthreads();
+    red[tid][0] = re[u];
+    red[tid][1] = im[u];
+    __syncthreads();
+    const int k = tid + u * tk;
+    if (tid < tk && k < nomega) {
+      double r0 = 0.0, r1 = 0.0;
+      for (int j = 0; j < ngroup; ++j) {
+        r0 += red[tid + j * tk][0];
+        r1 += red[tid + j * tk][1];
+      }
+      out[2 * k] = r0;
+      out[2 * k + 1] = r1;
+    }
+  }
+  if (with_egw) {
+    __syncthreads();
+    for (int o = 32; o > 0; o >>= 1) egw += __shfl_xor(egw, o, 64);
+    if ((tid & 63) == 0) red[tid >> 6][0] = egw;
+    __syncthreads();
+    if (tid == 0) out[2 * nomega] = red[0][0] + red[1][0] + red[2][0] + red[3][0];
   }
 }
 
-// sigma[(k, p)] (+)= sum_sb part[sb][p][k]; egw partial per p in lane 63.
-__global__ void sigma_reduce_kernel(const double* __restrict__ part, int nsblock, int nse, int nomega,
-                                    int nomega_total, int k0, int accumulate,
-                                    double* __restrict__ sigma, double* __restrict__ egw_p) {
+// sigma[(k, p)] (+)= sum over the nblk partial blocks; E_GW per p behind the
+// last frequency. One workgroup per p and 64 frequencies: four waves take
+// every fourth block.
+__global__ void __launch_bounds__(256)
+sigma_reduce_kernel(const double* __restrict__ part, int nblk, int nse, int nomega, int nomega_total, int k0,
+                    int accumulate, double* __restrict__ sigma, double* __restrict__ egw_p) {
+  __shared__ double red[4][64][2];
   const int p = blockIdx.x;
-  const int k = threadIdx.x;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int k = blockIdx.y * 64 + lane;
+  const bool egw = k == nomega;
   double r0 = 0.0, r1 = 0.0;
-  for (int sb = 0; sb < nsblock; ++sb) {
-    const double* q = part + 2 * (64 * ((int64_t)sb * nse + p) + k);
-    r0 += q[0];
-    r1 += q[1];
+  if (k < nomega || (egw && k0 == 0)) {
+    for (int b = wv; b < nblk; b += 4) {
+      const double* q = part + 2 * ((int64_t)(nomega + 1) * ((int64_t)b * nse + p) + k);
+      r0 += q[0];
+      if (!egw) r1 += q[1];
+    }
   }
+  red[wv][lane][0] = r0;
+  red[wv][lane][1] = r1;
+  __syncthreads();
+  if (wv != 0) return;
+  r0 = red[0][lane][0] + red[1][lane][0] + red[2][lane][0] + red[3][lane][0];
+  r1 = red[0][lane][1] + red[1][lane][1] + red[2][lane][1] + red[3][lane][1];
   if (k < nomega) {
     double* o = sigma + 2 * ((int64_t)p * nomega_total + k0 + k);
     if (accumulate) { o[0] += r0; o[1] += r1; } else { o[0] = r0; o[1] = r1; }
-  } else if (k == 63 && k0 == 0) {
+  } else if (egw && k0 == 0) {
     if (accumulate) egw_p[p] += r0; else egw_p[p] = r0;
   }
+}
+
+// chunks of the states i: enough workgroups for eight per CU
+static int sigma_ichunks(int nsb, int nse, int ni) {
+  const int64_t have = (int64_t)nsb * nse;
+  return (int)std::max<int64_t>(1, std::min<int64_t>(ni, (2048 + have - 1) / have));
 }
 
 int launch_sigma_poles(const double* w, int npole, int nse, int ni, const double* pole,
@@ -472,21 +675,27 @@ int launch_sigma_poles(const double* w, int npole, int nse, int ni, const double
   MGW_REQUIRE(nomega >= 1, MGW_ERR_ARG, "sigma_poles: nomega must be positive");
   MGW_REQUIRE(nse <= 65535, MGW_ERR_ARG, "sigma_poles: too many states");
   const int nsb = (npole + SIGMA_SB - 1) / SIGMA_SB;
-  // frequencies in groups of 63 lanes; lane 63 of the first group carries E_GW
-  for (int k0 = 0; k0 < nomega; k0 += 63) {
-    const int ng = std::min(63, nomega - k0);
-    hipLaunchKernelGGL(sigma_poles_kernel, dim3(nsb, nse), dim3(256), 0, s, w, npole, nse, ni, pole,
-                       omega + k0, ng, k0 == 0 ? 1 : 0, e0p, ei, fi, ep, occp, spin_fact, eta, part);
+  const int want = sigma_ichunks(nsb, nse, ni), ichunk = (ni + want - 1) / want, nz = (ni + ichunk - 1) / ichunk;
+  for (int k0 = 0; k0 < nomega; k0 += SIGMA_MAXK) {
+    const int nk = std::min(SIGMA_MAXK, nomega - k0);
+    const dim3 grid(nsb, nse, nz);
+    if (nk < 4)
+      hipLaunchKernelGGL(sigma_poles_kernel<1>, grid, dim3(256), 0, s, w, npole, nse, ni, ichunk, nsb, pole,
+                         omega + k0, nk, k0 == 0 ? 1 : 0, e0p, ei, fi, ep, occp, spin_fact, eta, part);
+    else
+      hipLaunchKernelGGL(sigma_poles_kernel<4>, grid, dim3(256), 0, s, w, npole, nse, ni, ichunk, nsb, pole,
+                         omega + k0, nk, k0 == 0 ? 1 : 0, e0p, ei, fi, ep, occp, spin_fact, eta, part);
     MGW_LAUNCH_CHECK();
-    hipLaunchKernelGGL(sigma_reduce_kernel, dim3(nse), dim3(64), 0, s, part, nsb, nse, ng, nomega, k0,
-                       accumulate, sigma, egw_p);
+    hipLaunchKernelGGL(sigma_reduce_kernel, dim3(nse, nk / 64 + 1), dim3(256), 0, s, part, nz * nsb, nse, nk, nomega,
+                       k0, accumulate, sigma, egw_p);
     MGW_LAUNCH_CHECK();
   }
   return MGW_OK;
 }
 
-int sigma_part_doubles(int npole, int nse) {
-  return ((npole + SIGMA_SB - 1) / SIGMA_SB) * nse * 64 * 2;
+int64_t sigma_part_doubles(int npole, int nse, int ni, int nomega) {
+  const int nsb = (npole + SIGMA_SB - 1) / SIGMA_SB;
+  return (int64_t)sigma_ichunks(nsb, nse, ni) * nsb * nse * (std::min(nomega, SIGMA_MAXK) + 1) * 2;
 }
 
 // ------------------------------------------------------------------ chi (imaginary axis)

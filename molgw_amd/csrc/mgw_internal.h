@@ -320,7 +320,18 @@ int launch_vsum(const double* x, int64_t n, int square, double* partial, int nbl
 int launch_casida_diag(const int32_t* ia, int npole, const double* energy, double* de, double* sq,
                        double* de2, hipStream_t s);
 int launch_casida_post(const double* eig, int npole, double* pole, double* cs, hipStream_t s);
-int sigma_part_doubles(int npole, int nse);
+// partial sums of the pole self-energy: doubles for launches of up to ni
+// states i and nomega frequencies
+int64_t sigma_part_doubles(int npole, int nse, int ni, int nomega);
+// gamma(P) = scale sum_{k, i} h(P, i, k) x(k, i) for h (naux x nx x nbf) and x
+// (nbf x nx); part: hartree_part_doubles(naux, nbf, nx) doubles
+int64_t hartree_part_doubles(int naux, int nbf, int nx);
+int launch_hartree_gamma(const double* h, const double* x, int naux, int nbf, int nx, double scale, double* part,
+                         double* gamma, hipStream_t s);
+// j(k, l) = j(l, k) = sum_P B(P, k, l) gamma(P) for B symmetric in (k, l)
+int launch_hartree_j(const double* b, const double* gamma, int naux, int nbf, double* j, hipStream_t s);
+// out(e) (+)= sum_b m(e + n b) over b < nbatch, in order
+int launch_batch_sum(const double* m, int64_t n, int nbatch, int accumulate, double* out, hipStream_t s);
 int launch_sigma_poles(const double* w, int npole, int nse, int ni, const double* pole,
                        const double* omega, int nomega, const double* e0p, const double* ei,
                        const double* fi, const double* ep, const double* occp, double spin_fact,
