@@ -2011,27 +2011,31 @@ int mgw_hartree_exchange_ri(mgw_ctx* c, const double* x, int nbf, int nx, double
   MGW_REQUIRE((int64_t)naux * nx < ((int64_t)1 << 31) && (int64_t)nbf * nbf < ((int64_t)1 << 31), MGW_ERR_ARG,
               "mgw_hartree_exchange_ri: problem too large");
   const double* B = find_buf(c, "ri_dense");
-  double *xd, *xt, *h, *gam, *jv, *kv;
+  double *xd, *h, *gam, *gpart, *jv, *kv, *kwork = nullptr;
   MGW_TRY(upload(c, "hf_x", x, (size_t)nbf * nx, &xd));
-  std::vector<double> xth((size_t)nx * nbf);   // xt[i + nx k] = x(k, i)
-  for (int k = 0; k < nbf; ++k)
-    for (int i = 0; i < nx; ++i) xth[(size_t)i + (size_t)nx * k] = x[(size_t)k + (size_t)nbf * i];
-  MGW_TRY(upload(c, "hf_xt", xth.data(), xth.size(), &xt));
   MGW_TRY(dbuf(c, "hf_h", (size_t)naux * nx * nbf, &h));
   MGW_TRY(dbuf(c, "hf_gamma", naux, &gam));
+  MGW_TRY(dbuf(c, "hf_gpart", (size_t)hartree_part_doubles(naux, nbf, nx), &gpart));
   MGW_TRY(dbuf(c, "hf_j", (size_t)nbf * nbf, &jv));
   MGW_TRY(dbuf(c, "hf_k", (size_t)nbf * nbf, &kv));
+  // the exchange sums over naux x nx rows into nbf x nbf: few tiles, so the
+  // rows are split (nbf 768, naux 2688, nx 160: 30 -> 5.0 ms); gamma and the
+  // Hartree matrix read their operands once (17 -> 0.44 and 2.9 -> 1.4 ms)
+  const int splits = gemm_f64_splits(nbf, nbf, naux * nx, 1, true);
+  if (splits > 1) MGW_TRY(dbuf(c, "hf_ksplit", gemm_f64_split_doubles(nbf, nbf, 1, splits), &kwork));
   {
     ProfScope ps(&c->prof, MGW_KCLASS_GEMM_OTHER,
                  2.0 * naux * (double)nbf * nbf * nx * 2.0 + 4.0 * naux * (double)nbf * nbf,
                  8.0 * ((double)naux * nbf * nbf * 2.0 + 2.0 * naux * nx * nbf), c->stream);
-    // H(P, i, k) = sum_l B(P, k, l) x(l, i): one product per k (B(:, :, k) is contiguous)
+    // H(P, i, k) = sum_l B(P, k, l) x(l, i): one product per k (B(:, :, k) is
+    // contiguous), all tiles of one k before the next
     GemmF64 g;
     g.M = naux; g.N = nx; g.K = nbf;
     g.A = B; g.lda = naux; g.strideA = (int64_t)naux * nbf;
     g.B = xd; g.ldb = nbf; g.strideB = 0;
     g.C = h; g.ldc = naux; g.strideC = (int64_t)naux * nx;
     g.batch = nbf;
+    g.batch_outer = true;
     MGW_TRY(gemm_f64(g, c->stream));
     // exchange = -H^T H over the rows (P, i)
     GemmF64 k;
@@ -2042,28 +2046,16 @@ int mgw_hartree_exchange_ri(mgw_ctx* c, const double* x, int nbf, int nx, double
     k.C = kv; k.ldc = nbf;
     k.alpha = -1.0;
     k.lower_only = true;
+    k.splits = splits;
+    k.split_work = kwork;
     MGW_TRY(gemm_f64(k, c->stream));
-    // gamma(P) = spin_fact sum_{i,k} H(P, i, k) x(k, i)
-    GemmF64 y;
-    y.M = naux; y.N = 1; y.K = nx * nbf;
-    y.A = h; y.lda = naux;
-    y.B = xt; y.ldb = (int64_t)nx * nbf;
-    y.C = gam; y.ldc = naux;
-    y.alpha = spin_fact;
-    MGW_TRY(gemm_f64(y, c->stream));
-    // hartree(k, l) = sum_P B(P, k, l) gamma(P)
-    GemmF64 jj;
-    jj.M = nbf * nbf; jj.N = 1; jj.K = naux;
-    jj.transA = true;
-    jj.A = B; jj.lda = naux;
-    jj.B = gam; jj.ldb = naux;
-    jj.C = jv; jj.ldc = (int64_t)nbf * nbf;
-    MGW_TRY(gemm_f64(jj, c->stream));
+    MGW_TRY(launch_hartree_gamma(h, xd, naux, nbf, nx, spin_fact, gpart, gam, c->stream));
+    MGW_TRY(launch_hartree_j(B, gam, naux, nbf, jv, c->stream));
   }
   if (hartree_ao) MGW_TRY(download(c, hartree_ao, jv, (size_t)nbf * nbf));
   if (exchange_ao) MGW_TRY(download(c, exchange_ao, kv, (size_t)nbf * nbf));
   MGW_HIP(hipStreamSynchronize(c->stream));
-  for (const char* b : {"hf_x", "hf_xt", "hf_gamma", "hf_j", "hf_k"}) MGW_TRY(scratch_done(c, b));
+  for (const char* b : {"hf_x", "hf_gamma", "hf_gpart", "hf_ksplit", "hf_j", "hf_k"}) MGW_TRY(scratch_done(c, b));
   MGW_TRY(scratch_done(c, "hf_h"));
   return MGW_OK;
 }
