@@ -9,8 +9,8 @@
 // and the self-energy works on D = L^-1 - 1 (chi = L^-T L^-1 - 1), so it
 // never needs the inverse itself.
 //
-// Recursive: the matrix is halved (at a multiple of 64) until 64 x 64
-// leaves, which a one-wave kernel factors and inverts in registers; the
+// Recursive: the matrix is halved (at a multiple of 64) down to leaves of at
+// most 128 x 128, which one workgroup per matrix factors and inverts; the
 // off-diagonal work is four batched MFMA GEMMs per level (the trailing
 // update has K = m/2), so the matrix is swept O(log n) times instead of once
 // per 64-wide block column. The strict upper triangle of the input must be
@@ -111,108 +111,201 @@ __device__ inline double rcp_nr(double d) {
   return r;
 }
 
-// The same factor and inverse with four waves per matrix, row owned, as
-// L D L^T with L unit lower (no square root or division on the sequential
-// path): thread t holds row i = t / 4 of the block at the columns
-// l = 4 c + (t % 4), c = 0 .. 15, in registers (the four threads of a row are
-// neighbouring lanes of one wave). Step j of the elimination publishes
-// column j (its owners write A(i, j), i >= j, to an LDS vector), one
-// barrier, d_j = A(j, j), and every thread updates its own columns j < l <= i:
-//   A(i, l) -= (A(i, j) / d_j) A(l, j),   L(i, j) = A(i, j) / d_j.
-// The unit lower L is inverted by rows without divisions: step l publishes
-// row l of T = L^-1, one barrier, and every row i > l subtracts
-// L(i, l) T(l, :), L(i, l) coming from the row's owner lane by a cross-lane
-// read. Then the Cholesky factor's inverse is D^-1/2 T, row i scaled by
-// d_i^-1/2, and ln det = sum ln d_j, all in parallel. The two LDS vectors
-// alternate, so a step's writes never meet the previous step's reads and one
-// barrier per step suffices. A non-positive pivot is recorded and replaced
-// by 1, as in chol_diag_kernel.
-__global__ void __launch_bounds__(256)
-chol_leaf_kernel(double* __restrict__ A, int n, int64_t strideA, int k, int kb, double* __restrict__ logdet,
-                 int32_t* __restrict__ info) {
-  constexpr int NC = NB / 4;        // columns per thread
-  __shared__ double vec[2][NB];     // published column (elimination) / row (inverse)
-  __shared__ double red[4];
-  const int f = blockIdx.x, t = threadIdx.x;
-  const int i = t >> 2, q = t & 3, lane = t & 63;
+// ---------------------------------------------------------------- leaf on the matrix cores
+// Value of lane `n` (a compile-time constant after unrolling) of each row of
+// 16 lanes.
+__device__ inline double row_bcast(double v, int n) {
+  const long long b = __double_as_longlong(v);
+  int lo = (int)b, hi = (int)(b >> 32);
+#define MGW_ROW_BCAST(N)                                                          \
+  case N:                                                                         \
+    lo = __builtin_amdgcn_update_dpp(0, lo, 0x150 + N, 0xf, 0xf, true);           \
+    hi = __builtin_amdgcn_update_dpp(0, hi, 0x150 + N, 0xf, 0xf, true);           \
+    break;
+  switch (n) {
+    MGW_ROW_BCAST(0) MGW_ROW_BCAST(1) MGW_ROW_BCAST(2) MGW_ROW_BCAST(3)
+    MGW_ROW_BCAST(4) MGW_ROW_BCAST(5) MGW_ROW_BCAST(6) MGW_ROW_BCAST(7)
+    MGW_ROW_BCAST(8) MGW_ROW_BCAST(9) MGW_ROW_BCAST(10) MGW_ROW_BCAST(11)
+    MGW_ROW_BCAST(12) MGW_ROW_BCAST(13) MGW_ROW_BCAST(14) MGW_ROW_BCAST(15)
+  }
+#undef MGW_ROW_BCAST
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+
+typedef double ld4 __attribute__((ext_vector_type(4)));
+
+// Factor and invert the m x m diagonal block at (k, k) of every matrix, m <= 16
+// NBK, one workgroup of NBK waves per matrix. Latency bounds it (a batch has
+// as many workgroups as frequencies), so the sequential part is kept to 16 x 16
+// blocks in the registers of one wave, and everything else runs on the matrix
+// cores beside it. The lower 16 x 16 blocks live in LDS; per block column c:
+//   * wave 0 has factored block (c, c) as L D L^T, L unit lower (no square root
+//     or division on the sequential path), and holds T_cc = D^-1/2 L^-1. Lane
+//     (g, i) of the wave keeps row i, the four groups g of 16 lanes redundantly;
+//     step j broadcasts pivot and column within each row of 16 lanes (DPP, no
+//     LDS, no barrier), and group g updates the columns g, g + 4, .. of T;
+//   * panel: L_ic = A_ic T_cc^T, one wave per block (v_mfma_f64_16x16x4_f64);
+//   * trailing update A_ij -= L_ic L_jc^T: wave 0 takes (c + 1, c + 1) and
+//     factors it at once, under the others' updates;
+//   * inverse by rows under the same factorisation: T_cj = -T_cc sum_k L_ck T_kj,
+//     one wave per j. The sum's result registers are the next product's operand
+//     as they are. T_cj replaces L_cj after the barrier.
+// Rows past m are rows of the identity. A non-positive pivot records its
+// 1-based column in info (first failure only) and is replaced by 1 so the
+// batch stays finite. 32 matrices: m = 64 18 us, 84 29 us, 128 38 us a launch (a
+// leaf on LDS columns with two barriers per column took 85 us for m = 64).
+template <int NBK>
+__global__ void __launch_bounds__(64 * NBK)
+chol_block_kernel(double* __restrict__ A, int n, int64_t strideA, int k, int m, double* __restrict__ logdet,
+                  int32_t* __restrict__ info) {
+  constexpr int LD = 17, BS = 16 * LD, NT = 64 * NBK;
+  __shared__ double sm[NBK * (NBK + 1) / 2 * BS];
+  const int f = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int nb = (m + 15) / 16;
   double* __restrict__ g = A + (int64_t)f * strideA + k + (int64_t)k * n;
-  double a[NC];
+  auto blk = [&](int i, int j) { return sm + (i * (i + 1) / 2 + j) * BS; };
+  // 256 threads per block, four waves to a block: row i, column j of block b;
+  // all loads are in flight before the first is stored
+  constexpr int NLD = NBK * (NBK + 1) / 2 * 256 / NT;
+  const int bq = wave >> 2, ti = tid & 15, tj = (tid >> 4) & 15;
+  double v[NLD];
 #pragma unroll
-  for (int c = 0; c < NC; ++c) {
-    const int l = 4 * c + q;
-    a[c] = (i < kb && l < kb) ? (l <= i ? g[i + (int64_t)l * n] : 0.0) : (i == l ? 1.0 : 0.0);
+  for (int u = 0; u < NLD; ++u) {
+    const int b = u * (NT / 256) + bq;
+    int bi = 0;
+    while ((bi + 1) * (bi + 2) / 2 <= b) ++bi;
+    const int row = 16 * bi + ti, col = 16 * (b - bi * (bi + 1) / 2) + tj;
+    const int lo = max(row, col), hi = min(row, col);      // diagonal blocks hold both triangles
+    v[u] = row == col ? 1.0 : 0.0;
+    if (lo < m) v[u] = g[lo + (int64_t)hi * n];
   }
+#pragma unroll
+  for (int u = 0; u < NLD; ++u) sm[(u * (NT / 256) + bq) * BS + ti * LD + tj] = v[u];
+  __syncthreads();
+
+  const int fr = lane & 15, fk = lane >> 4;
   int failed = 0;
+  double ld = 0.0;
+  auto factor = [&](int c) __attribute__((always_inline)) {
+    double* __restrict__ d = blk(c, c);
+    double x[16], t[4], di = 1.0;
 #pragma unroll
-  for (int j = 0; j < NB; ++j) {
-    double* __restrict__ v = vec[j & 1];
-    if (q == (j & 3) && i >= j) v[i] = a[j >> 2];
-    __syncthreads();
-    double d = v[j];
-    if (!(d > 0.0)) {
-      if (!failed && j < kb) failed = k + j + 1;
-      d = 1.0;
-    }
-    if (i > j) {
-      const double lij = v[i] * rcp_nr(d);
+    for (int l = 0; l < 16; ++l) x[l] = d[fr * LD + l];
 #pragma unroll
-      for (int c = j >> 2; c < NC; ++c) {
-        const int l = 4 * c + q;
-        if (l > j && l <= i) a[c] -= lij * v[l];
+    for (int q = 0; q < 4; ++q) t[q] = 4 * q + fk == fr ? 1.0 : 0.0;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      double dj = row_bcast(x[j], j);
+      if (!(dj > 0.0)) {
+        if (!failed) failed = k + 16 * c + j + 1;
+        dj = 1.0;
       }
-      if (q == (j & 3)) a[j >> 2] = lij;
-    } else if (i == j && q == (j & 3)) {
-      a[j >> 2] = d;                 // D on the diagonal
+      if (fr == j) di = dj;
+      const double lij = fr > j ? x[j] * rcp_nr(dj) : 0.0;
+#pragma unroll
+      for (int l = j + 1; l < 16; ++l) x[l] = fma(-lij, row_bcast(x[j], l), x[l]);
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (4 * q <= j) t[q] = fma(-lij, row_bcast(t[q], j), t[q]);
     }
-  }
-  // d_i of this row from its owner lane; ln det(block) / 2 = sum ln d_i / 2
-  double di = 0.0;
-#pragma unroll
-  for (int c = 0; c < NC; ++c)
-    if (4 * c + q == i) di = a[c];
-  di = __shfl(di, (lane & ~3) | (i & 3), 64);
-  double ld = (q == 0 && i < kb) ? 0.5 * log(di) : 0.0;
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) ld += __shfl_down(ld, off, 64);
-  if (lane == 0) red[t >> 6] = ld;
-  // T = L^-1 by rows (unit diagonal: no divisions)
-  double tt[NC];
-#pragma unroll
-  for (int c = 0; c < NC; ++c) tt[c] = (4 * c + q == i) ? 1.0 : 0.0;
-#pragma unroll
-  for (int l = 0; l < NB; ++l) {
-    double* __restrict__ v = vec[l & 1];
-    const double lil = __shfl(a[l >> 2], (lane & ~3) | (l & 3), 64);   // L(i, l)
-    if (i == l) {
-#pragma unroll
-      for (int c = 0; c < NC; ++c)
-        if (4 * c + q <= l) v[4 * c + q] = tt[c];
-    }
-    __syncthreads();
-    if (i > l) {
-#pragma unroll
-      for (int c = 0; c < NC; ++c)
-        if (4 * c + q <= l) tt[c] -= lil * v[4 * c + q];
-    }
-  }
-  if (i < kb) {
+    if (fk == 0) ld += 0.5 * log(di);
     const double rs = 1.0 / sqrt(di);
 #pragma unroll
-    for (int c = 0; c < NC; ++c) {
-      const int l = 4 * c + q;
-      if (l < kb) g[i + (int64_t)l * n] = l <= i ? tt[c] * rs : 0.0;
+    for (int q = 0; q < 4; ++q) d[fr * LD + 4 * q + fk] = t[q] * rs;
+  };
+  // a operand (rows of X) and, for X^T, b operand of k step s; b operand of X
+  auto rows = [&](const double* X, int s) { return X[fr * LD + 4 * s + fk]; };
+  auto cols = [&](const double* X, int s) { return X[(4 * s + fk) * LD + fr]; };
+
+  if (wave == 0) factor(0);
+  __syncthreads();
+  ld4 tpend = {0.0, 0.0, 0.0, 0.0};       // T(c, wave - 1) of the last block row
+  for (int c = 0; c < nb; ++c) {
+    if (c > 0 && wave >= 1 && wave - 1 < c - 1) {
+      double* __restrict__ w = blk(c - 1, wave - 1);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) w[(fk + 4 * r) * LD + fr] = tpend[r];
     }
+    for (int i = c + 1 + wave; i < nb; i += NBK) {
+      double* __restrict__ a = blk(i, c);
+      const double* __restrict__ tc = blk(c, c);
+      ld4 acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(rows(a, s), rows(tc, s), acc, 0, 0, 0);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) a[(fk + 4 * r) * LD + fr] = acc[r];
+    }
+    __syncthreads();
+    auto update = [&](int i, int j) __attribute__((always_inline)) {
+      double* __restrict__ a = blk(i, j);
+      const double *li = blk(i, c), *lj = blk(j, c);
+      ld4 acc;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[r] = a[(fk + 4 * r) * LD + fr];
+#pragma unroll
+      for (int s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(-rows(li, s), rows(lj, s), acc, 0, 0, 0);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) a[(fk + 4 * r) * LD + fr] = acc[r];
+    };
+    if (wave == 0) {
+      if (c + 1 < nb) {
+        update(c + 1, c + 1);
+        factor(c + 1);
+      }
+    } else {
+      // blocks (i, j), c < j <= i, behind (c + 1, c + 1), in turn
+      int e = wave - 1;
+      for (int i = c + 2; i < nb; ++i)
+        for (int j = c + 1; j <= i; ++j, --e)
+          if (e == 0) {
+            update(i, j);
+            e = NBK - 1;
+          }
+      if (wave - 1 < c) {
+        const int j = wave - 1;
+        ld4 acc = {0.0, 0.0, 0.0, 0.0};
+        for (int q = j; q < c; ++q) {
+          const double *l = blk(c, q), *t = blk(q, j);
+#pragma unroll
+          for (int s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(rows(l, s), cols(t, s), acc, 0, 0, 0);
+        }
+        const double* tc = blk(c, c);
+        tpend = ld4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int s = 0; s < 4; ++s) tpend = __builtin_amdgcn_mfma_f64_16x16x4f64(-rows(tc, s), acc[s], tpend, 0, 0, 0);
+      }
+    }
+    __syncthreads();
   }
-  if (t == 0) {
-    logdet[f] = (k == 0 ? 0.0 : logdet[f]) + red[0] + red[1] + red[2] + red[3];
-    if (k == 0) info[f] = 0;
-    if (failed && info[f] == 0) info[f] = failed;
+  if (wave >= 1 && wave - 1 < nb - 1) {
+    double* __restrict__ w = blk(nb - 1, wave - 1);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) w[(fk + 4 * r) * LD + fr] = tpend[r];
+  }
+  __syncthreads();
+  for (int u = 0; u < NLD; ++u) {
+    const int b = u * (NT / 256) + bq;
+    int bi = 0;
+    while ((bi + 1) * (bi + 2) / 2 <= b) ++bi;
+    const int row = 16 * bi + ti, col = 16 * (b - bi * (bi + 1) / 2) + tj;
+    if (row < m && col < m) g[row + (int64_t)col * n] = row >= col ? sm[b * BS + ti * LD + tj] : 0.0;
+  }
+  if (wave == 0) {
+    for (int o = 8; o > 0; o >>= 1) ld += __shfl_xor(ld, o, 64);
+    if (lane == 0) {
+      logdet[f] = (k == 0 ? 0.0 : logdet[f]) + ld;
+      if (k == 0) info[f] = 0;
+      if (failed && info[f] == 0) info[f] = failed;
+    }
   }
 }
 
-// Leaf kernel: MGW_CHOL_LEAF = 0 (one wave, registers) or 1 (four waves,
-// LDS); read at every factorisation.
-bool chol_leaf_lds() {
+// Leaves: chol_block_kernel on blocks of up to 128, or (MGW_CHOL_LEAF = 0, read
+// at every factorisation) chol_diag_kernel on blocks of up to 64. A 128 leaf
+// takes the place of two 64 leaves and the four products that join them.
+constexpr int LEAF = 2 * NB;
+bool chol_leaf_block() {
   const char* e = std::getenv("MGW_CHOL_LEAF");
   return e ? std::atoi(e) != 0 : true;
 }
@@ -609,17 +702,20 @@ int plane_gemm(const CholCtx& c, const Fp16Planes& da, const _Float16* pa, int a
 //   [A21 A22]   A22 -= L21 L21^T, factor and invert A22 (recursion),
 //               (L^-1)21 = -(L^-1)22 L21 (L^-1)11.
 // The products are batched MFMA GEMMs (FP64, or FP16x3 on planes for the
-// large levels when the factorisation has operand bounds); the 64 x 64
-// leaves are factored and inverted by chol_leaf_kernel (or
-// chol_diag_kernel). `w` is this block's work (chol_need(m) doubles per
+// large levels when the factorisation has operand bounds); the leaves
+// are factored and inverted by chol_block_kernel (or chol_diag_kernel). `w` is this block's work (chol_need(m) doubles per
 // matrix, matrix stride c.sw); `l21_off` the L21-plane stack used by the
 // enclosing levels (elements per matrix).
 int chol_rec(const CholCtx& c, int k0, int m, double* w, int64_t l21_off) {
   const int n = c.n;
   const int64_t s2 = (int64_t)n * n;
-  if (m <= NB) {
-    if (chol_leaf_lds())
-      hipLaunchKernelGGL(chol_leaf_kernel, dim3(c.nbatch), dim3(256), 0, c.stream, c.A, n, s2, k0, m, c.logdet,
+  const bool block = chol_leaf_block();
+  if (m <= (block ? LEAF : NB)) {
+    if (block && m > NB)
+      hipLaunchKernelGGL(chol_block_kernel<8>, dim3(c.nbatch), dim3(512), 0, c.stream, c.A, n, s2, k0, m, c.logdet,
+                         c.info);
+    else if (block)
+      hipLaunchKernelGGL(chol_block_kernel<4>, dim3(c.nbatch), dim3(256), 0, c.stream, c.A, n, s2, k0, m, c.logdet,
                          c.info);
     else
       hipLaunchKernelGGL(chol_diag_kernel, dim3(c.nbatch), dim3(64), 0, c.stream, c.A, n, s2, k0, m, c.logdet,

@@ -126,3 +126,20 @@ def test_qs_self_energy_batched_sum(eng, lo, hi, ncore):
     ref = O.gw_selfenergy_qs(epi, ws, pole, s.energy, s.occupation, rng, eta=0.05)
     size = sum((np.abs(ws.T @ epi[:, :, k]).T @ np.abs(ws.T @ epi[:, :, k])) / 0.05 for k in range(epi.shape[2]))
     assert np.all(np.abs(mo[win, win] - ref) <= 4 * (70 + len(pole) * epi.shape[2]) * EPS * size)
+
+
+@pytest.mark.parametrize('naux', [1, 2, 15, 16, 17, 33, 63, 64, 65, 112, 113, 127, 128, 129, 145])
+def test_chi_leaf_sizes(eng, naux):
+    """(1 - chi0)^-1 of sizes on both sides of the factorisation's blocks of 16
+    and leaves of 64 and 128; bound as in test_chi_with_split_transitions."""
+    s = synthetic_system(20, naux, 6, seed=19, scale=0.3)
+    _load(eng, s)
+    om = np.array([0.2, 1.0, 5.0])
+    _, _, chi = eng.polarizability_grid(selfenergy_set_state_range(s.occupation), om, np.ones(3), return_chi=True)
+    b, c = dense_ri(s), s.c_matrix
+    x = np.einsum('pkl,ka,li->pia', b, c[:, 6:], c[:, :6], optimize=True).reshape(naux, -1)
+    de = (s.energy[None, 6:] - s.energy[:6, None]).reshape(-1)
+    for f in range(3):
+        chi0 = (x * (4.0 * de / (om[f] ** 2 + de ** 2))) @ x.T
+        ref = np.linalg.inv(np.eye(naux) + chi0) - np.eye(naux)
+        assert np.max(np.abs(chi[:, :, f] - ref)) <= 4 * (len(de) + naux) * EPS * (1.0 + np.trace(chi0))
