@@ -198,6 +198,10 @@ struct SyrkArgs {
   int kc_slabs, nkc;
   float* part;
   const double* unscale;   // per frequency of the chunk (FP16X3), else null
+  // part of the lower triangle that this launch covers (`tiles` tiles of it;
+  // partial tiles are addressed by the whole triangle's order): row >= 0, the
+  // tiles (row, 0 .. row) only
+  int row, ptiles;
 };
 
 // Lower-triangle tiles BM x BM, WM x WN waves, one 32-k slab per step.
@@ -236,7 +240,12 @@ chi_syrk_kernel(SyrkArgs g) {
   const int kc = KSPLIT ? (int)((L % per_f) / g.tiles) : 0;
   const int tile = (int)(L % g.tiles);
   int bm, bn;
-  tri_grouped(tile, g.tm, bm, bn);
+  if (g.row >= 0) {
+    bm = g.row;
+    bn = tile;
+  } else {
+    tri_grouped(tile, g.tm, bm, bn);
+  }
   const int m0 = bm * BM, n0 = bn * BM;
 
   const E* __restrict__ Ya = static_cast<const E*>(g.y) + (int64_t)f * g.fstride + (int64_t)m0 * KT;
@@ -363,7 +372,8 @@ chi_syrk_kernel(SyrkArgs g) {
 
   if constexpr (KSPLIT) {
     // FP32 partial tile, column-major BM x BM; summed in FP64 by chi_ksplit_reduce_kernel
-    float* __restrict__ P = g.part + ((int64_t)(f * g.tiles + tile) * g.nkc + kc) * (BM * BM);
+    const int pt = g.row >= 0 ? tri_grouped_index(bm, bn, g.tm) : tile;
+    float* __restrict__ P = g.part + ((int64_t)(f * g.ptiles + pt) * g.nkc + kc) * (BM * BM);
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
@@ -659,6 +669,163 @@ chi_syrk_pipe_kernel(SyrkArgs g) {
 #pragma unroll
       for (int r = 0; r < 4; ++r)
         P[(wm * TM + i * 16 + fr) + (wn * TN + j * 16 + 4 * fq + r) * BM] = part[i][j][r];
+}
+
+// The K-split SYRK on 256 x 256 tiles, eight waves of 128 x 64 in two groups of
+// four (one wave of each group per SIMD) that take turns: while one group
+// reads its fragments of a slab from LDS (24 16-byte reads a lane, 96
+// registers), the other runs its 96 MFMAs, so the matrix cores wait for
+// neither LDS nor memory. A slab (64 KB: 256 rows and 256 columns, two
+// planes, 32 k) has two LDS buffers; all fragments are in registers before
+// the MFMAs start, so a buffer is free again after both groups' reads, and the
+// next copy into it (global_load_lds) has two turns to land. A turn ends at a
+// bare barrier:
+//   turn 2 s:      group 0 reads slab s and starts the copies of slab s + 1 into
+//                  the buffer of slab s - 1; group 1 multiplies slab s - 1
+//   turn 2 s + 1:  group 0 multiplies slab s and waits for its copies of slab
+//                  s + 1; group 1 reads slab s
+// Only group 0 copies, and only behind its reads: the compiler makes an LDS
+// read wait for copies of its own wave that it cannot tell apart from it.
+// Against 128-wide tiles a panel is read half as often from L2 (the 128-wide
+// kernel asks it for two thirds of its rate at full MFMA speed) and LDS is read
+// 0.75 times per MFMA. Same products in the same order per accumulator as
+// chi_syrk_kernel: identical results. 2688 rows, 97280 transitions, 32
+// frequencies: 69 -> 56 ms (1.02 -> 1.32 PFLOP/s of fp16 MFMA).
+constexpr int waitcnt(int vm, int lgkm) { return (vm & 15) | (7 << 4) | (lgkm << 8) | ((vm >> 4) << 14); }
+
+template <bool H>
+__global__ void __launch_bounds__(512, 2)
+chi_syrk_pp_kernel(SyrkArgs g, int t256) {
+  typedef typename PlaneT<H>::E E;
+  typedef typename PlaneT<H>::V V;
+  constexpr int BM = 256, NS = 2, TM = 128, TN = 64, FM = TM / 16, FN = TN / 16;
+  __shared__ __attribute__((aligned(16))) E S0[2][NS][BM][KT];   // [operand][plane][row][k]
+  __shared__ __attribute__((aligned(16))) E S1[2][NS][BM][KT];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // columns 0 - 127 (on in every tile) belong to group 0
+  const int wm = wave & 1, wn = wave >> 1;
+  const int group = wave >> 2;
+  const int64_t L = xcd_logical(blockIdx.x, g.nblocks);
+  const int64_t per_f = (int64_t)g.nkc * g.tiles;
+  const int f = (int)(L / per_f);
+  const int kc = (int)((L % per_f) / g.tiles);
+  const int tile = (int)(L % g.tiles);
+  int bm, bn;
+  tri_grouped(tile, t256, bm, bn);
+  // sub-tile of this wave, in 128-wide tiles; strictly above the diagonal it
+  // only copies
+  const int bm1 = 2 * bm + wm, bn1 = 2 * bn + (wn >> 1);
+  const bool on = bm1 >= bn1;
+
+  // the sixteen copies of a slab of a wave of group 0: the 1 KB windows of 16
+  // rows of one plane (pl) of one operand (op); chunks swizzled as lds_chunk
+  const int op = (wave >> 1) & 1, pl = wave & 1;
+  const int rl = lane >> 2, jl = (lane & 3) ^ ((rl >> 1) & 3);
+  const E* __restrict__ src = static_cast<const E*>(g.y) + (int64_t)f * g.fstride + pl * g.plane +
+                              (int64_t)((op ? bn : bm) * BM) * KT;
+  const unsigned lo = (rl * KT + 8 * jl) * sizeof(E);
+  const int64_t slab = (int64_t)g.ppad * KT;
+  const int fr = lane & 15, fq = lane >> 4;
+  const int fo = 8 * lds_chunk(fr, fq);
+
+  f4 part[FM][FN];
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j) part[i][j] = f4{0.f, 0.f, 0.f, 0.f};
+  V a[NS][FM], b[NS][FN];
+
+#define MGW_PP_ISSUE(S_, SB)                                                                              \
+  _Pragma("unroll") for (int c = 0; c < 16; ++c)                                                          \
+    __builtin_amdgcn_global_load_lds(                                                                     \
+        reinterpret_cast<const unsigned*>(                                                                \
+            reinterpret_cast<const char*>(src + (int64_t)(S_) * slab + c * 16 * KT) + lo),                \
+        reinterpret_cast<unsigned*>(&SB[op][pl][16 * c][0]), 16, 0, 0);
+#define MGW_PP_READ(SB)                                                                                   \
+  _Pragma("unroll") for (int q = 0; q < NS; ++q) {                                                        \
+    _Pragma("unroll") for (int i = 0; i < FM; ++i)                                                        \
+      a[q][i] = *reinterpret_cast<const V*>(&SB[0][q][wm * TM + i * 16 + fr][fo]);                        \
+    _Pragma("unroll") for (int j = 0; j < FN; ++j)                                                        \
+      b[q][j] = *reinterpret_cast<const V*>(&SB[1][q][wn * TN + j * 16 + fr][fo]);                        \
+  }
+  // the empty asm statements and scheduling barriers keep LDS accesses and
+  // MFMAs in their turn
+#define MGW_PP_BARRIER(VM)                                                                                \
+  __builtin_amdgcn_s_waitcnt(waitcnt(VM, 0));                                                             \
+  __asm__ __volatile__("" ::: "memory");                                                                  \
+  __builtin_amdgcn_sched_barrier(0);                                                                      \
+  __builtin_amdgcn_s_barrier();                                                                           \
+  __builtin_amdgcn_sched_barrier(0);                                                                      \
+  __asm__ __volatile__("" ::: "memory");
+  auto multiply = [&]() __attribute__((always_inline)) {
+    constexpr int QA[3] = {1, 0, 0};
+    constexpr int QB[3] = {0, 1, 0};
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int pr = 0; pr < 3; ++pr)
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) part[i][j] = mfma16x16x32<H>(b[QB[pr]][j], a[QA[pr]][i], part[i][j]);
+    __builtin_amdgcn_s_setprio(0);
+  };
+
+  const int s0 = kc * g.kc_slabs;
+  const int ns = min(g.nkt, s0 + g.kc_slabs) - s0;     // >= 1
+  if (group == 0) {
+    MGW_PP_ISSUE(s0, S0)
+    if (ns > 1) { MGW_PP_ISSUE(s0 + 1, S1) }
+    MGW_PP_BARRIER(0)
+#define MGW_PP_G0(S_, SC, SN)                                          \
+  MGW_PP_READ(SC)                                                      \
+  __asm__ __volatile__("" ::: "memory");                               \
+  if ((S_) >= 1 && (S_) + 1 < ns) { MGW_PP_ISSUE(s0 + (S_) + 1, SN) }   \
+  MGW_PP_BARRIER(63)                                                   \
+  multiply();                                                          \
+  MGW_PP_BARRIER(0)
+    int s = 0;
+    for (; s + 1 < ns; s += 2) {
+      MGW_PP_G0(s, S0, S1)
+      MGW_PP_G0(s + 1, S1, S0)
+    }
+    if (s < ns) { MGW_PP_G0(s, S0, S1) }
+#undef MGW_PP_G0
+  } else if (!on) {
+    MGW_PP_BARRIER(63)
+    for (int s = 0; s < 2 * ns; ++s) { MGW_PP_BARRIER(63) }
+    return;
+  } else {
+#define MGW_PP_G1(SC) \
+  multiply();         \
+  MGW_PP_BARRIER(63)  \
+  MGW_PP_READ(SC)     \
+  MGW_PP_BARRIER(63)
+    MGW_PP_BARRIER(63)
+    MGW_PP_BARRIER(63)
+    MGW_PP_READ(S0)
+    MGW_PP_BARRIER(63)
+    int s = 1;
+    for (; s + 1 < ns; s += 2) {
+      MGW_PP_G1(S1)
+      MGW_PP_G1(S0)
+    }
+    if (s < ns) { MGW_PP_G1(S1) }
+#undef MGW_PP_G1
+    multiply();
+  }
+#undef MGW_PP_ISSUE
+#undef MGW_PP_READ
+#undef MGW_PP_BARRIER
+
+  float* __restrict__ P = g.part + ((int64_t)(f * g.ptiles + tri_grouped_index(bm1, bn1, g.tm)) * g.nkc + kc) * (128 * 128) +
+                          (wn & 1) * TN * 128;
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) P[(i * 16 + fr) + (j * 16 + 4 * fq + r) * 128] = part[i][j][r];
 }
 
 // SYRK kernel of the K-split planes path: MGW_CHI_SYRK = 0 (register
@@ -1201,6 +1368,28 @@ chi_scale_kernel(const double* __restrict__ xpart, int nb, const double* __restr
 // bytes in front of the planes: scale, unscale (per frequency), |X| partial maxima
 size_t scale_header_bytes(int nomega) { return ((size_t)(2 * nomega + NB_MAX) * sizeof(double) + 255) / 256 * 256; }
 
+// The lower triangle on 256-wide tiles; with an odd number of 128-wide tile
+// rows, the last row on 128-wide ones.
+constexpr int64_t PP_FILL = 512;
+
+template <bool H>
+int launch_syrk_pp(const SyrkArgs& g0, hipStream_t stream) {
+  SyrkArgs g = g0;
+  const int t256 = g.tm / 2;
+  g.tiles = t256 * (t256 + 1) / 2;
+  g.nblocks = (int64_t)g.tiles * g.nkc * g.nf;
+  hipLaunchKernelGGL((chi_syrk_pp_kernel<H>), dim3((unsigned)g.nblocks), dim3(512), 0, stream, g, t256);
+  MGW_HIP(hipGetLastError());
+  if (g.tm % 2 == 0) return MGW_OK;
+  g.row = g.tm - 1;
+  g.tiles = g.tm;
+  g.nblocks = (int64_t)g.tiles * g.nkc * g.nf;
+  hipLaunchKernelGGL((chi_syrk_kernel<2, H, 128, 2, 2, 4, 1, 1, true>), dim3((unsigned)g.nblocks), dim3(256), 0, stream,
+                     g);
+  MGW_HIP(hipGetLastError());
+  return MGW_OK;
+}
+
 template <int NS, bool H>
 int split_and_syrk(const double* x, int naux, int npole, const double* sw, int nomega, void* work,
                    size_t work_bytes, double* chi, hipStream_t stream) {
@@ -1249,6 +1438,7 @@ int split_and_syrk(const double* x, int naux, int npole, const double* sw, int n
     g.C = chi + (int64_t)f0 * naux * naux; g.strideC = (int64_t)naux * naux;
     g.kc_slabs = L.kc_slabs; g.nkc = L.nkc; g.part = part;
     g.unscale = H ? uns + f0 : nullptr;
+    g.row = -1; g.ptiles = L.tiles;
     const int depth = chi_prefetch_depth(NS);
     const dim3 block(256);
     if (ksplit) {
@@ -1262,8 +1452,14 @@ int split_and_syrk(const double* x, int naux, int npole, const double* sw, int n
       const int var = NS == 2 ? chi_syrk_variant() : 0;
       MGW_REQUIRE((L.bm == 256) == (var == 5 || var == 6), MGW_ERR_ARG,
                   "chi0 split: tile size and SYRK variant disagree");
+      // 256-wide tiles where their workgroups, one per CU, fill the GPU twice
+      const int t256 = L.tm / 2;
+      const bool pp = NS == 2 && !std::getenv("MGW_CHI_SYRK") &&
+                      (int64_t)t256 * (t256 + 1) / 2 * L.nkc * nf >= PP_FILL;
       auto launch = [&](int v) -> int {
         if (v) return launch_syrk_lds(H, v, grid, g, stream);
+        if constexpr (NS == 2)
+          if (pp) return launch_syrk_pp<H>(g, stream);
         hipLaunchKernelGGL((chi_syrk_kernel<NS, H, BM, 2, 2, 4, 1, 1, true>), grid, block, 0, stream, g);
         MGW_HIP(hipGetLastError());
         return MGW_OK;

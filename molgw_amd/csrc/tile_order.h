@@ -45,4 +45,12 @@ __device__ inline void tri_grouped(int t, int T, int& bm, int& bn) {
   bm = r0 + c + u;
 }
 
+// The position of tile (bm, bn), bm >= bn, in that order.
+__device__ inline int tri_grouped_index(int bm, int bn, int T) {
+  const int r0 = bm / TRI_GROUP * TRI_GROUP, g = min(TRI_GROUP, T - r0), base = r0 * (r0 + 1) / 2;
+  if (bn < r0) return base + bn * g + (bm - r0);
+  const int c = bn - r0;
+  return base + r0 * g + c * g - c * (c - 1) / 2 + (bm - bn);
+}
+
 }  // namespace mgw

@@ -453,10 +453,10 @@ int split_and_dot(const double* d, int naux, int nomega, const double* b, int64_
 
 }  // namespace
 
-// Workspace of the W.B split: scales, the B^T planes, and the D planes of as
-// many frequencies as fit in 2 GiB (at least one).
 int wb_split_rowblocks(int M) { return (M + 127) / 128; }   // row tile of the dot epilogue
 
+// Workspace of the W.B split: scales, the B^T planes, and the D planes of as
+// many frequencies as fit in 2 GiB (at least one).
 size_t wb_split_workspace(int naux, int64_t ncol, int nomega, int precision) {
   const int ns = precision == MGW_BF16X6 ? 3 : 2;
   const WbLayout L = wb_layout(naux, ncol);

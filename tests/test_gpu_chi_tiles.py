@@ -1,0 +1,37 @@
+"""The FP16x3 / BF16x3 chi0 build on 256-wide tiles (with a last row of 128-wide
+ones when the tile rows are odd) does the products of the 128-wide kernel in
+the same order: identical chi0 (through its inverse) for sizes at the edges of
+the tiles and odd and even slab counts, with enough frequencies that the
+256-wide tiles are taken."""
+import os
+
+import numpy as np
+import pytest
+
+from molgw_amd.gw import Engine, selfenergy_set_state_range
+from molgw_amd.workloads import synthetic_system
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope='module')
+def eng():
+    with Engine(0) as e:
+        yield e
+
+
+@pytest.mark.parametrize('nbf, naux, nocc', [(40, 250, 13), (61, 257, 30), (60, 384, 31), (70, 511, 35), (70, 513, 33)])
+@pytest.mark.parametrize('precision', ['fp16x3', 'bf16x3'])
+def test_wide_tiles_equal_narrow_tiles(eng, monkeypatch, nbf, naux, nocc, precision):
+    s = synthetic_system(nbf, naux, nocc, seed=20, scale=0.3)
+    eng.set_eri_3center(s.eri_3center, s.index_basis, s.nbf)
+    eng.set_mo(s.c_matrix, s.energy, s.occupation)
+    rng = selfenergy_set_state_range(s.occupation)
+    nomega = 530 if naux < 300 else 200      # 512 workgroups of 256-wide tiles
+    om, wt = np.linspace(0.1, 3.0, nomega), np.ones(nomega)
+    got = eng.polarizability_grid(rng, om, wt, precision=precision, return_chi=True)
+    monkeypatch.setenv('MGW_CHI_SYRK', '0')
+    ref = eng.polarizability_grid(rng, om, wt, precision=precision, return_chi=True)
+    assert os.environ['MGW_CHI_SYRK'] == '0'
+    np.testing.assert_array_equal(got[2], ref[2])
+    assert got[:2] == ref[:2]
