@@ -12,6 +12,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <initializer_list>
 #include <tuple>
 #include <cstring>
 #include <numeric>
@@ -95,6 +96,11 @@ struct mgw_ctx {
   Ledger ledger;
   Profiler prof;
   bool trim_eagerly = false;
+  // pinned host memory (STAGE_BYTES) through which small vectors go to and come
+  // from the device; used up to stage_used since the last synchronisation of
+  // the stream, before which no byte of it is written again
+  char* stage = nullptr;
+  size_t stage_used = 0;
   // A1: resident RI tensor, dense B(P, k, l)
   bool has_ri = false;
   int nbf = 0, naux = 0;
@@ -257,17 +263,84 @@ bool is_resident_input(const std::string& name) {
 // trim eagerly, they are freed here.
 int scratch_done(mgw_ctx* c, const std::string& name);
 
+// Small transfers go through the context's pinned memory, and vectors that are
+// needed together in one copy: from or to pageable memory a copy costs the host
+// 9 us however small it is. A Pade solve of one water molecule (41 functions)
+// made 21 of them and 8 waits in 0.51 ms; with 10 and 4 it takes 0.35 ms.
+constexpr size_t STAGE_BYTES = 128 << 10;
+
+int sync(mgw_ctx* c) {
+  MGW_HIP(hipStreamSynchronize(c->stream));
+  c->stage_used = 0;
+  return MGW_OK;
+}
+
+// room in the pinned memory, or null when the transfer is not a small one
+int stage_room(mgw_ctx* c, size_t bytes, char** out) {
+  *out = nullptr;
+  bytes = (bytes + 63) / 64 * 64;
+  if (!c->stage || bytes > STAGE_BYTES / 2) return MGW_OK;
+  if (c->stage_used + bytes > STAGE_BYTES) MGW_TRY(sync(c));
+  *out = c->stage + c->stage_used;
+  c->stage_used += bytes;
+  return MGW_OK;
+}
+
+int copy_in(mgw_ctx* c, void* dev, const void* host, size_t bytes) {
+  if (!bytes) return MGW_OK;
+  char* st = nullptr;
+  MGW_TRY(stage_room(c, bytes, &st));
+  if (st) std::memcpy(st, host, bytes);
+  MGW_HIP(hipMemcpyAsync(dev, st ? st : host, bytes, hipMemcpyHostToDevice, c->stream));
+  return MGW_OK;
+}
+
 template <class T>
 int upload(mgw_ctx* c, const std::string& name, const T* host, size_t count, T** out) {
   MGW_TRY(dbuf(c, name, count, out));
-  if (count) MGW_HIP(hipMemcpyAsync(*out, host, count * sizeof(T), hipMemcpyHostToDevice, c->stream));
+  return copy_in(c, *out, host, count * sizeof(T));
+}
+
+// Several host vectors into one device buffer, in one copy; dev receives the
+// device address of each.
+struct Part {
+  const void* host;
+  size_t bytes;
+  void** dev;
+};
+template <class T>
+Part part_of(const T* host, size_t count, T** dev) {
+  return Part{host, count * sizeof(T), reinterpret_cast<void**>(dev)};
+}
+
+int upload_group(mgw_ctx* c, const std::string& name, std::initializer_list<Part> parts) {
+  size_t total = 0;
+  for (const Part& p : parts) total += (p.bytes + 15) / 16 * 16;
+  char* d = nullptr;
+  MGW_TRY(dbuf(c, name, total, &d));
+  char* st = nullptr;
+  MGW_TRY(stage_room(c, total, &st));
+  size_t off = 0;
+  for (const Part& p : parts) {
+    *p.dev = d + off;
+    if (st) std::memcpy(st + off, p.host, p.bytes);
+    else if (p.bytes) MGW_HIP(hipMemcpyAsync(d + off, p.host, p.bytes, hipMemcpyHostToDevice, c->stream));
+    off += (p.bytes + 15) / 16 * 16;
+  }
+  if (st && total) MGW_HIP(hipMemcpyAsync(d, st, total, hipMemcpyHostToDevice, c->stream));
   return MGW_OK;
 }
 
 template <class T>
 int download(mgw_ctx* c, T* host, const T* dev, size_t count) {
-  if (count) MGW_HIP(hipMemcpyAsync(host, dev, count * sizeof(T), hipMemcpyDeviceToHost, c->stream));
-  MGW_HIP(hipStreamSynchronize(c->stream));
+  const size_t bytes = count * sizeof(T);
+  char* st = nullptr;
+  if (count) {
+    MGW_TRY(stage_room(c, bytes, &st));
+    MGW_HIP(hipMemcpyAsync(st ? static_cast<void*>(st) : host, dev, bytes, hipMemcpyDeviceToHost, c->stream));
+  }
+  MGW_TRY(sync(c));
+  if (st) std::memcpy(host, st, bytes);
   return MGW_OK;
 }
 
@@ -307,23 +380,25 @@ void transition_table(const mgw_ctx* c, const mgw_ranges* r, double spin_fact, s
   ia.clear();
   const double ce = 1.0e-5;
   const int ns = c->nstate;
-  auto skip = [&](int ib1, int ib2, double o1, double o2) {
-    if (ib1 <= r->ncore_W || ib2 <= r->ncore_W) return true;
-    if (ib1 >= r->nvirtual_W || ib2 >= r->nvirtual_W) return true;
-    if (o1 < ce && o2 < ce) return true;
-    if (o1 > spin_fact - ce && o2 > spin_fact - ce) return true;
-    return false;
-  };
+  const int lo = std::max(1, r->ncore_W + 1), hi = std::min(ns, r->nvirtual_W - 1);
   for (int s = 0; s < c->nspin; ++s) {
     const double* occ = c->occupation.data() + (size_t)s * ns;
-    for (int i = 1; i <= ns; ++i)
-      for (int j = 1; j <= ns; ++j) {
-        const double oj = occ[j - 1], oi = occ[i - 1];
-        if (skip(j, i, oj, oi)) continue;
+    bool numbers = true;
+    for (int j = lo; j <= hi; ++j) numbers = numbers && !std::isnan(occ[j - 1]);
+    for (int i = lo; i <= hi; ++i) {
+      const double oi = occ[i - 1];
+      // an empty i pairs only with occupations of at most its own, empty too:
+      // no pair, and no need to go over the row (60 us at 300 states)
+      if (numbers && oi < ce) continue;
+      for (int j = lo; j <= hi; ++j) {
+        const double oj = occ[j - 1];
+        if (oj < ce && oi < ce) continue;
+        if (oj > spin_fact - ce && oi > spin_fact - ce) continue;
         if (oj - oi > 0.0) continue;
         ia.push_back(s * ns + i - 1);
         ia.push_back(s * ns + j - 1);
       }
+    }
   }
 }
 
@@ -658,12 +733,9 @@ int gw_selfenergy(mgw_ctx* c, const mgw_ranges* r, double spin_fact, double eta,
   for (int k = 0; k < ng; ++k) { ei[k] = eg[glo - 1 + k]; fi[k] = oc[glo - 1 + k]; }
   for (int k = 0; k < nse; ++k) { ep[k] = eg[r->nsemin - 1 + k]; occp[k] = oc[r->nsemin - 1 + k]; }
   double *om_d, *e0p_d, *ei_d, *fi_d, *ep_d, *occp_d;
-  MGW_TRY(upload(c, "se_omega", omega, nomega, &om_d));
-  MGW_TRY(upload(c, "se_e0p", e0p.data(), nse, &e0p_d));
-  MGW_TRY(upload(c, "se_ei", ei.data(), ng, &ei_d));
-  MGW_TRY(upload(c, "se_fi", fi.data(), ng, &fi_d));
-  MGW_TRY(upload(c, "se_ep", ep.data(), nse, &ep_d));
-  MGW_TRY(upload(c, "se_occp", occp.data(), nse, &occp_d));
+  MGW_TRY(upload_group(c, "se_in", {part_of(omega, (size_t)nomega, &om_d), part_of(e0p.data(), (size_t)nse, &e0p_d),
+                                    part_of(ei.data(), (size_t)ng, &ei_d), part_of(fi.data(), (size_t)ng, &fi_d),
+                                    part_of(ep.data(), (size_t)nse, &ep_d), part_of(occp.data(), (size_t)nse, &occp_d)}));
   double *sigma, *egw_p, *part;
   MGW_TRY(dbuf(c, "sigma", (size_t)2 * nomega * nse, &sigma));
   MGW_TRY(dbuf(c, "sigma_egw", nse, &egw_p));
@@ -759,13 +831,18 @@ int polarizability_grid(mgw_ctx* c, const mgw_ranges* r, double spin_fact, int n
   const int npole = (int)ia.size() / 2;
   const int naux = c->naux;
   int32_t* ia_d = nullptr;
-  MGW_TRY(upload(c, "ia", ia.data(), ia.size(), &ia_d));
-  double *om_d, *sw, *n2, *ones, *tr0, *chi;
-  MGW_TRY(upload(c, "chi_omega", omega_im, nomega, &om_d));
+  double *om_d, *sw, *n2, *ones, *chi;
+  MGW_TRY(upload_group(c, "chi_in", {part_of(ia.data(), ia.size(), &ia_d), part_of(omega_im, (size_t)nomega, &om_d)}));
   MGW_TRY(dbuf(c, "chi_sw", (size_t)npole * nomega, &sw));
   MGW_TRY(dbuf(c, "cas_n2", npole, &n2));
   MGW_TRY(dbuf(c, "ones", naux, &ones));
-  MGW_TRY(dbuf(c, "chi_tr0", nomega, &tr0));
+  // what the host needs of the factorisation, in one piece: the trace of chi0,
+  // ln det, the partial sums of ||L^-1||^2 and the flags of every frequency
+  const size_t nres = (size_t)nomega * (2 + FROB_BLOCKS) + (nomega + 1) / 2;
+  double* res = nullptr;
+  MGW_TRY(dbuf(c, "chi_result", nres, &res));
+  double *const tr0 = res, *const logdet = res + nomega, *const frob = res + 2 * (size_t)nomega;
+  int32_t* const info_d = reinterpret_cast<int32_t*>(frob + (size_t)FROB_BLOCKS * nomega);
   // 1 - chi0, then its inverse Cholesky factor, resident for the self-energy
   MGW_TRY(dbuf(c, "wpol_linv", (size_t)naux * naux * nomega, &chi));
   MGW_TRY(launch_fill(ones, naux, 1.0, c->stream));
@@ -818,12 +895,8 @@ int polarizability_grid(mgw_ctx* c, const mgw_ranges* r, double spin_fact, int n
   g.split_work = nullptr;
   if (precision != MGW_FP64) MGW_TRY(scratch_done(c, "chi_split"));
   // 1 - chi0 = L L^T for every frequency, then L^-1 in place (chol.hip)
-  int32_t* info_d = nullptr;
-  double *logdet, *work, *frob;
-  MGW_TRY(dbuf(c, "solver_info", std::max(64, nomega), &info_d));
-  MGW_TRY(dbuf(c, "chol_logdet", nomega, &logdet));
+  double* work = nullptr;
   MGW_TRY(dbuf(c, "chol_work", chol_work_doubles(naux) * nomega, &work));
-  MGW_TRY(dbuf(c, "chol_frob", (size_t)FROB_BLOCKS * nomega, &frob));
   // FP16x3 solves factor with FP16x3 products at the large levels: 1 - chi0
   // >= I holds there (every weight s >= 0), which the operand bounds need
   double* bounds = nullptr;
@@ -839,9 +912,14 @@ int polarizability_grid(mgw_ctx* c, const mgw_ranges* r, double spin_fact, int n
     MGW_TRY(run_chol(c, chi, naux, nomega, logdet, info_d, work, bounds, planes));
   }
   if (planes) MGW_TRY(scratch_done(c, "chol_planes"));
-  std::vector<int32_t> info(nomega);
-  MGW_TRY(download(c, info.data(), info_d, nomega));
-  bool checked_x = false;
+  // D = L^-1 - 1 stays resident: chi = L^-T L^-1 - 1 = D^T D + D + D^T, and
+  // the self-energy product works on the screening part D alone
+  MGW_TRY(launch_lower_frob2(chi, naux, nomega, frob, c->stream));
+  MGW_TRY(launch_diag_add(chi, naux, nomega, -1.0, c->stream));
+  std::vector<double> hres(nres);
+  MGW_TRY(download(c, hres.data(), res, nres));
+  const int32_t* info = reinterpret_cast<const int32_t*>(hres.data() + (size_t)(2 + FROB_BLOCKS) * nomega);
+  bool checked_x = false, rebuilt = false;
   for (int k = 0; k < nomega; ++k) {
     if (info[k] == 0) continue;
     MGW_REQUIRE(precision != MGW_FP64, MGW_ERR_SOLVER,
@@ -870,16 +948,13 @@ int polarizability_grid(mgw_ctx* c, const mgw_ranges* r, double spin_fact, int n
     MGW_REQUIRE(one == 0, MGW_ERR_SOLVER,
                 "Cholesky of the FP64 rebuild of 1-chi0 failed at frequency " + std::to_string(k) + " (column " +
                     std::to_string(one) + "; reduced-precision column " + std::to_string(info[k]) + ")");
+    MGW_TRY(launch_lower_frob2(g1.C, naux, 1, frob + (size_t)FROB_BLOCKS * k, c->stream));
+    MGW_TRY(launch_diag_add(g1.C, naux, 1, -1.0, c->stream));
     ++c->escalations;
+    rebuilt = true;
   }
-  MGW_TRY(launch_lower_frob2(chi, naux, nomega, frob, c->stream));
-  // D = L^-1 - 1 stays resident: chi = L^-T L^-1 - 1 = D^T D + D + D^T, and
-  // the self-energy product works on the screening part D alone
-  MGW_TRY(launch_diag_add(chi, naux, nomega, -1.0, c->stream));
-  std::vector<double> h0(nomega), hl(nomega), fr((size_t)FROB_BLOCKS * nomega);
-  MGW_TRY(download(c, h0.data(), tr0, nomega));
-  MGW_TRY(download(c, hl.data(), logdet, nomega));
-  MGW_TRY(download(c, fr.data(), frob, (size_t)FROB_BLOCKS * nomega));
+  if (rebuilt) MGW_TRY(download(c, hres.data(), res, nres));
+  const double *h0 = hres.data(), *hl = h0 + nomega, *fr = hl + nomega;
   // sum ln(lambda) + 1 - lambda = ln det(1-chi0) + Tr chi0 ;
   // sum -(1-lambda)/lambda + 1 - lambda = n - Tr (1-chi0)^-1 + Tr chi0
   // (src/m_gw_selfenergy_grid.f90:171-173); Tr (1-chi0)^-1 = ||L^-1||_F^2
@@ -946,10 +1021,9 @@ int gw_selfenergy_imag(mgw_ctx* c, const mgw_ranges* r, int ncalc, const double*
   MGW_TRY(launch_dot_reduce(part, nrb, ncol, nomega, nullptr, v, c->stream));
   std::vector<double> ep(np);
   for (int k = 0; k < np; ++k) ep[k] = c->energy_in_g()[c->so() + glo - 1 + k];
-  MGW_TRY(upload(c, "sgi_omega", c->chi_omega.data(), nomega, &om_d));
-  MGW_TRY(upload(c, "sgi_weight", c->chi_weight.data(), nomega, &wt_d));
-  MGW_TRY(upload(c, "sgi_ep", ep.data(), np, &ep_d));
-  MGW_TRY(upload(c, "sgi_wc", omega_calc, (size_t)2 * ncalc, &wc_d));
+  MGW_TRY(upload_group(c, "sgi_in", {part_of(c->chi_omega.data(), (size_t)nomega, &om_d),
+                                     part_of(c->chi_weight.data(), (size_t)nomega, &wt_d),
+                                     part_of(ep.data(), (size_t)np, &ep_d), part_of(omega_calc, (size_t)2 * ncalc, &wc_d)}));
   MGW_TRY(dbuf(c, "sigma_calc", (size_t)2 * ncalc * nse, &sc));
   MGW_TRY(launch_sigma_imag_sum(v, np, nse, nomega, om_d, wt_d, ep_d, wc_d, ncalc, sc, c->stream));
   c->has_sigma_calc = true;
@@ -974,8 +1048,7 @@ int pade_fit(mgw_ctx* c, int nse, int ncalc, const double* omega_calc, const dou
     sc = find_buf(c, "sigma_calc");
   }
   double *wc_d, *om_d, *work, *sigma;
-  MGW_TRY(upload(c, "pade_wc", omega_calc, (size_t)2 * ncalc, &wc_d));
-  MGW_TRY(upload(c, "pade_omega", omega, nomega, &om_d));
+  MGW_TRY(upload_group(c, "pade_in", {part_of(omega_calc, (size_t)2 * ncalc, &wc_d), part_of(omega, (size_t)nomega, &om_d)}));
   MGW_TRY(dbuf(c, "pade_work", (size_t)pade_work_doubles(ncalc, nse), &work));
   MGW_TRY(dbuf(c, "sigma", (size_t)2 * nomega * nse, &sigma));
   MGW_TRY(launch_pade(wc_d, sc, ncalc, nse, om_d, nomega, eta, work, sigma, c->stream));
@@ -1007,10 +1080,8 @@ int find_qp(mgw_ctx* c, const mgw_ranges* r, int nomega, const double* omega, co
     excs[k] = exc ? exc[r->nsemin - 1 + k] : 0.0;
   }
   double *om_d, *se0_d, *exc_d, *e0_d, *out;
-  MGW_TRY(upload(c, "qp_omega", omega, nomega, &om_d));
-  MGW_TRY(upload(c, "qp_se0", se_energy0, nse, &se0_d));
-  MGW_TRY(upload(c, "qp_exc", excs.data(), nse, &exc_d));
-  MGW_TRY(upload(c, "qp_e0", e0s.data(), nse, &e0_d));
+  MGW_TRY(upload_group(c, "qp_in", {part_of(omega, (size_t)nomega, &om_d), part_of(se_energy0, (size_t)nse, &se0_d),
+                                    part_of(excs.data(), (size_t)nse, &exc_d), part_of(e0s.data(), (size_t)nse, &e0_d)}));
   MGW_TRY(dbuf(c, "qp_out", (size_t)3 * nse, &out));
   MGW_TRY(launch_qp(sg, nomega, nse, om_d, se0_d, exc_d, e0_d, out, out + nse, out + 2 * nse, c->stream));
   std::vector<double> h(3 * nse);
@@ -1200,16 +1271,13 @@ int contour_sigma(mgw_ctx* c, const mgw_ranges* r, double eta, int nomega, const
   }
   double *omi_d, *wti_d, *omr_d, *ep_d, *e0_d, *om_d, *sigma;
   int32_t *ps_d, *err_d;
-  MGW_TRY(upload(c, "cd_om_im", c->cd_om_im.data(), nimag, &omi_d));
-  MGW_TRY(upload(c, "cd_wt_im", c->cd_wt_im.data(), nimag, &wti_d));
-  MGW_TRY(upload(c, "cd_om_re", c->cd_om_re.data(), nreal, &omr_d));
-  MGW_TRY(upload(c, "cd_ep", ep.data(), np, &ep_d));
-  MGW_TRY(upload(c, "cd_pstate", ps.data(), np, &ps_d));
-  MGW_TRY(upload(c, "se_e0p", se_energy0, nse, &e0_d));
-  MGW_TRY(upload(c, "se_omega", omega, nomega, &om_d));
-  MGW_TRY(dbuf(c, "sigma", (size_t)2 * nomega * nse, &sigma));
   const int32_t zero = 0;
-  MGW_TRY(upload(c, "cd_err", &zero, 1, &err_d));
+  MGW_TRY(upload_group(c, "cd_in", {part_of(c->cd_om_im.data(), (size_t)nimag, &omi_d),
+                                    part_of(c->cd_wt_im.data(), (size_t)nimag, &wti_d),
+                                    part_of(c->cd_om_re.data(), (size_t)nreal, &omr_d), part_of(ep.data(), (size_t)np, &ep_d),
+                                    part_of(ps.data(), (size_t)np, &ps_d), part_of(se_energy0, (size_t)nse, &e0_d),
+                                    part_of(omega, (size_t)nomega, &om_d), part_of(&zero, (size_t)1, &err_d)}));
+  MGW_TRY(dbuf(c, "sigma", (size_t)2 * nomega * nse, &sigma));
   MGW_TRY(launch_sigma_contour(v, np, nse, nimag, nreal, omi_d, wti_d, omr_d, ep_d, ps_d, r->nhomo_G, nlumo_of(r),
                                e0_d, om_d, nomega, eta, sigma, err_d, c->stream));
   int32_t err = 0;
@@ -1263,8 +1331,19 @@ int mgw_ctx_create(int device, mgw_ctx** out) {
     set_error(std::string("hipStreamCreate: ") + hipGetErrorString(e));
     return MGW_ERR_HIP;
   }
+  void* stage = nullptr;
+  e = hipHostMalloc(&stage, STAGE_BYTES, hipHostMallocDefault);
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    (void)hipStreamDestroy(c->stream);
+    delete c;
+    set_error(std::string("hipHostMalloc: ") + hipGetErrorString(e));
+    return MGW_ERR_NOMEM;
+  }
+  c->stage = static_cast<char*>(stage);
   if (rocblas_create_handle(&c->blas) != rocblas_status_success ||
       rocblas_set_stream(c->blas, c->stream) != rocblas_status_success) {
+    (void)hipHostFree(c->stage);
     (void)hipStreamDestroy(c->stream);
     delete c;
     set_error("rocblas handle creation failed");
@@ -1277,12 +1356,13 @@ int mgw_ctx_create(int device, mgw_ctx** out) {
 int mgw_ctx_destroy(mgw_ctx* c) {
   if (!c) return MGW_OK;
   MGW_HIP(hipSetDevice(c->device));
-  MGW_HIP(hipStreamSynchronize(c->stream));
+  MGW_TRY(sync(c));
   clear_graphs(c);
   for (auto& kv : c->ledger.bufs)
     if (kv.second.ptr) MGW_HIP(hipFreeAsync(kv.second.ptr, c->stream));
-  MGW_HIP(hipStreamSynchronize(c->stream));
+  MGW_TRY(sync(c));
   rocblas_destroy_handle(c->blas);
+  (void)hipHostFree(c->stage);
   MGW_HIP(hipStreamDestroy(c->stream));
   delete c;
   return MGW_OK;
@@ -1300,7 +1380,7 @@ int mgw_set_energy_g(mgw_ctx* c, const double* energy_g) {
 
 int mgw_ctx_graphs(mgw_ctx* c, int enable) {
   MGW_CTX(c);
-  MGW_HIP(hipStreamSynchronize(c->stream));
+  MGW_TRY(sync(c));
   if (!enable) clear_graphs(c);
   c->use_graphs = enable != 0;
   return MGW_OK;
@@ -1308,7 +1388,7 @@ int mgw_ctx_graphs(mgw_ctx* c, int enable) {
 
 int mgw_ctx_synchronize(mgw_ctx* c) {
   MGW_CTX(c);
-  MGW_HIP(hipStreamSynchronize(c->stream));
+  MGW_TRY(sync(c));
   return MGW_OK;
 }
 
@@ -1321,7 +1401,7 @@ int mgw_autotune(int mode, int* previous) {
 
 int mgw_ctx_trim(mgw_ctx* c, int eager) {
   MGW_CTX(c);
-  MGW_HIP(hipStreamSynchronize(c->stream));
+  MGW_TRY(sync(c));
   std::vector<std::string> names;
   for (auto& kv : c->ledger.bufs)
     if (!is_resident_input(kv.first)) names.push_back(kv.first);
@@ -1333,7 +1413,7 @@ int mgw_ctx_trim(mgw_ctx* c, int eager) {
   // that later allocations do not go back to the driver): hand what no
   // context holds back to the device, so that the pool's reserved size stays
   // within what the contexts' ledgers account for
-  MGW_HIP(hipStreamSynchronize(c->stream));
+  MGW_TRY(sync(c));
   hipMemPool_t pool;
   MGW_HIP(hipDeviceGetDefaultMemPool(&pool, c->device));
   MGW_HIP(hipMemPoolTrimTo(pool, 0));
@@ -1342,7 +1422,7 @@ int mgw_ctx_trim(mgw_ctx* c, int eager) {
 
 int mgw_profile_enable(mgw_ctx* c, int enable) {
   MGW_CTX(c);
-  MGW_HIP(hipStreamSynchronize(c->stream));
+  MGW_TRY(sync(c));
   c->prof.reset();
   c->prof.on = enable != 0;
   return MGW_OK;
@@ -1352,7 +1432,7 @@ int mgw_profile_read(mgw_ctx* c, int kernel_class, int64_t* launches, double* to
                      double* algorithmic_flops, double* algorithmic_bytes) {
   MGW_CTX(c);
   MGW_REQUIRE(kernel_class >= 0 && kernel_class < MGW_KCLASS_COUNT, MGW_ERR_ARG, "invalid kernel class");
-  MGW_HIP(hipStreamSynchronize(c->stream));
+  MGW_TRY(sync(c));
   int64_t n = 0;
   double ms = 0.0, fl = 0.0, by = 0.0;
   for (const auto& r : c->prof.recs) {
@@ -1558,9 +1638,11 @@ int mgw_set_eri_3center(mgw_ctx* c, const double* eri, int64_t npair, int nauxil
   MGW_TRY(dbuf(c, "ri_absmax", 1, &amax));
   MGW_TRY(launch_fill(amax, 1, 0.0, c->stream));
   MGW_TRY(launch_unpack_ri(packed, npair, nauxil, kl_d, nbf, dense, c->stream, !complete, amax));
-  MGW_HIP(hipStreamSynchronize(c->stream));
+  MGW_TRY(sync(c));
   MGW_TRY(release(c, "ri_packed"));
-  MGW_TRY(release(c, "ri_kl"));
+  // a free and a new allocation cost the next solve 20 us: a short pair list stays
+  if (kl.size() * sizeof(int32_t) > (1 << 20)) MGW_TRY(release(c, "ri_kl"));
+  else MGW_TRY(scratch_done(c, "ri_kl"));
   c->nbf = nbf;
   c->naux = nauxil;
   c->has_ri = true;
@@ -1611,7 +1693,7 @@ int mgw_inverse_sqrt_eri_2center(mgw_ctx* c, const double* eri_2center, int naux
   if (sqrtinv_out) {
     MGW_HIP(hipMemcpyAsync(sqrtinv_out, s, (size_t)n * kept * sizeof(double), hipMemcpyDefault, c->stream));
   }
-  MGW_HIP(hipStreamSynchronize(c->stream));
+  MGW_TRY(sync(c));
   MGW_TRY(release(c, "metric_u"));
   MGW_TRY(release(c, "metric_eig"));
   MGW_TRY(release(c, "metric_ework"));
@@ -1703,7 +1785,7 @@ int mgw_build_eri_3center(mgw_ctx* c, const double* eri_3center_tmp, int64_t ipa
                              (size_t)mpair * sizeof(double), (size_t)mpair * sizeof(double), nk, hipMemcpyDefault,
                              c->stream));
   }
-  MGW_HIP(hipStreamSynchronize(c->stream));
+  MGW_TRY(sync(c));
   MGW_TRY(release(c, "ri_tmp"));
   MGW_TRY(release(c, "ri_packed"));
   MGW_TRY(release(c, "ri_kl"));
@@ -1865,7 +1947,7 @@ int mgw_eri_2center_ao(mgw_ctx* c, const mgw_shells* auxil, int where, double* e
       MGW_TRY(launch_eri_class(e, c->stream));
     }
   if (where == MGW_MEM_HOST) MGW_TRY(download(c, eri_2center, out, (size_t)naux * naux));
-  MGW_HIP(hipStreamSynchronize(c->stream));
+  MGW_TRY(sync(c));
   for (const char* b : {"int_kfun", "int_pairs", "int_out2"}) MGW_TRY(release(c, b));
   MGW_TRY(release_shells(c, "int_aux"));
   MGW_TRY(release_shells(c, "int_unit"));
@@ -1952,7 +2034,7 @@ int mgw_eri_3center_ao(mgw_ctx* c, const mgw_shells* basis, const mgw_shells* au
         }
   }
   if (eri_3center_tmp && where == MGW_MEM_HOST) MGW_TRY(download(c, eri_3center_tmp, out, (size_t)npair * naux));
-  MGW_HIP(hipStreamSynchronize(c->stream));
+  MGW_TRY(sync(c));
   for (const char* b : {"int_pairmap", "int_pairs", "int_kfun", "int_out3"}) MGW_TRY(release(c, b));
   MGW_TRY(release_shells(c, "int_bas"));
   MGW_TRY(release_shells(c, "int_aux"));
@@ -2054,7 +2136,7 @@ int mgw_hartree_exchange_ri(mgw_ctx* c, const double* x, int nbf, int nx, double
   }
   if (hartree_ao) MGW_TRY(download(c, hartree_ao, jv, (size_t)nbf * nbf));
   if (exchange_ao) MGW_TRY(download(c, exchange_ao, kv, (size_t)nbf * nbf));
-  MGW_HIP(hipStreamSynchronize(c->stream));
+  MGW_TRY(sync(c));
   for (const char* b : {"hf_x", "hf_gamma", "hf_gpart", "hf_ksplit", "hf_j", "hf_k"}) MGW_TRY(scratch_done(c, b));
   MGW_TRY(scratch_done(c, "hf_h"));
   return MGW_OK;
@@ -2084,16 +2166,18 @@ int mgw_set_mo_spin(mgw_ctx* c, const double* c_matrix, int nbf, int nstate, int
     MGW_HIP(hipMemcpyAsync(cd, c_matrix, sizeof(double) * nc, hipMemcpyDeviceToDevice, c->stream));
     MGW_HIP(hipMemcpyAsync(c->energy.data(), energy, sizeof(double) * ne, hipMemcpyDeviceToHost, c->stream));
     MGW_HIP(hipMemcpyAsync(c->occupation.data(), occupation, sizeof(double) * ne, hipMemcpyDeviceToHost, c->stream));
-    MGW_HIP(hipStreamSynchronize(c->stream));
+    MGW_TRY(sync(c));
   } else {
-    MGW_HIP(hipMemcpyAsync(cd, c_matrix, sizeof(double) * nc, hipMemcpyHostToDevice, c->stream));
+    MGW_TRY(copy_in(c, cd, c_matrix, sizeof(double) * nc));
     std::memcpy(c->energy.data(), energy, sizeof(double) * ne);
     std::memcpy(c->occupation.data(), occupation, sizeof(double) * ne);
   }
   double *ed, *od;
   MGW_TRY(upload(c, "energy", c->energy.data(), ne, &ed));
   MGW_TRY(upload(c, "occupation", c->occupation.data(), ne, &od));
-  MGW_HIP(hipStreamSynchronize(c->stream));
+  // small host arrays are in the pinned memory by now; any other may be written
+  // again by its owner once this returns, so its copy has to be over
+  if (where == MGW_MEM_DEVICE || sizeof(double) * nc > STAGE_BYTES / 2) MGW_TRY(sync(c));
   c->nstate = nstate;
   c->nspin = nspin;
   c->spin = 0;
@@ -2139,7 +2223,7 @@ int mgw_calculate_eri_3center_mo(mgw_ctx* c, int mstate_min, int mstate_max, int
                 MGW_ERR_STATE, "a different eri_3center_mo block is resident; destroy it first");
     MGW_TRY(download(c, out, find_buf(c, "eri_3center_mo"), (size_t)c->naux * nm * nn));
   }
-  MGW_HIP(hipStreamSynchronize(c->stream));
+  MGW_TRY(sync(c));
   return MGW_OK;
 }
 
@@ -2217,7 +2301,7 @@ int mgw_polarizability(mgw_ctx* c, const mgw_ranges* r, double spin_fact, int pr
   MGW_TRY(polarizability_casida(c, r, spin_fact, en_rpa, en_gw, precision));
   if (pole_out) MGW_TRY(download(c, pole_out, find_buf(c, "wpol_pole"), c->npole));
   if (w_s_out) MGW_TRY(download(c, w_s_out, find_buf(c, "wpol_ws"), (size_t)c->naux * c->npole));
-  MGW_HIP(hipStreamSynchronize(c->stream));
+  MGW_TRY(sync(c));
   return MGW_OK;
 }
 
@@ -2234,7 +2318,7 @@ int mgw_set_spectral_function(mgw_ctx* c, int npole, int nauxil, const double* p
   const hipMemcpyKind k = where == MGW_MEM_HOST ? hipMemcpyHostToDevice : hipMemcpyDeviceToDevice;
   MGW_HIP(hipMemcpyAsync(pd, pole, sizeof(double) * npole, k, c->stream));
   MGW_HIP(hipMemcpyAsync(wd, w_s, sizeof(double) * nauxil * (size_t)npole, k, c->stream));
-  MGW_HIP(hipStreamSynchronize(c->stream));
+  MGW_TRY(sync(c));
   c->npole = npole;
   c->has_wpol = true;
   c->has_sigma = false;
@@ -2266,7 +2350,7 @@ int mgw_gw_ingredients(mgw_ctx* c, const mgw_ranges* r, double* w_out, double* v
     MGW_TRY(download(c, w_out, w, (size_t)npole * ng * ng));
   }
   if (v_out) MGW_TRY(download(c, v_out, v, (size_t)naux * ng * ng));
-  MGW_HIP(hipStreamSynchronize(c->stream));
+  MGW_TRY(sync(c));
   MGW_TRY(release(c, "ingr_w"));
   MGW_TRY(release(c, "ingr_v"));
   return MGW_OK;
@@ -2305,7 +2389,7 @@ int mgw_polarizability_grid(mgw_ctx* c, const mgw_ranges* r, double spin_fact, i
     MGW_TRY(download(c, chi_out, full, (size_t)n * n * nomega));
     MGW_TRY(release(c, "chi_full"));
   }
-  MGW_HIP(hipStreamSynchronize(c->stream));
+  MGW_TRY(sync(c));
   return MGW_OK;
 }
 
@@ -2328,9 +2412,8 @@ int mgw_gw_selfenergy_qs(mgw_ctx* c, const mgw_ranges* r, double spin_fact, doub
   for (int k = 0; k < ng; ++k) { ei[k] = eg[glo - 1 + k]; fi[k] = oc[glo - 1 + k]; }
   for (int k = 0; k < nse; ++k) eq[k] = eg[r->nsemin - 1 + k];
   double *ei_d, *fi_d, *eq_d, *sig;
-  MGW_TRY(upload(c, "qs_ei", ei.data(), ng, &ei_d));
-  MGW_TRY(upload(c, "qs_fi", fi.data(), ng, &fi_d));
-  MGW_TRY(upload(c, "qs_eq", eq.data(), nse, &eq_d));
+  MGW_TRY(upload_group(c, "qs_in", {part_of(ei.data(), (size_t)ng, &ei_d), part_of(fi.data(), (size_t)ng, &fi_d),
+                                    part_of(eq.data(), (size_t)nse, &eq_d)}));
   MGW_TRY(dbuf(c, "qs_sigma", (size_t)nse * nse, &sig));
   // chunk over i so that w(s, p, i) and its scaled copy stay within ~1 GiB each
   const size_t per_i = (size_t)npole * nse * sizeof(double);
@@ -2402,7 +2485,7 @@ int mgw_gw_selfenergy_qs(mgw_ctx* c, const mgw_ranges* r, double spin_fact, doub
     MGW_TRY(gemm_f64(g4, c->stream));
     MGW_TRY(download(c, selfenergy_ao, t2, (size_t)nbf * nbf));
   }
-  MGW_HIP(hipStreamSynchronize(c->stream));
+  MGW_TRY(sync(c));
   MGW_TRY(scratch_done(c, "sigma_w"));
   MGW_TRY(scratch_done(c, "qs_b"));
   MGW_TRY(scratch_done(c, "qs_sigma_i"));
@@ -2419,7 +2502,7 @@ int mgw_gw_selfenergy(mgw_ctx* c, const mgw_ranges* r, double spin_fact, double 
   MGW_TRY(gw_selfenergy(c, r, spin_fact, eta, nomega, omega, se_energy0, energy_gw, MGW_FP64));
   const int nse = r->nsemax - r->nsemin + 1;
   if (sigma_out) MGW_TRY(download(c, sigma_out, find_buf(c, "sigma"), (size_t)2 * nomega * nse));
-  MGW_HIP(hipStreamSynchronize(c->stream));
+  MGW_TRY(sync(c));
   return MGW_OK;
 }
 
@@ -2431,7 +2514,7 @@ int mgw_gw_selfenergy_imag(mgw_ctx* c, const mgw_ranges* r, int nomega_calc, con
   MGW_TRY(gw_selfenergy_imag(c, r, nomega_calc, omega_calc, MGW_FP64));
   const int nse = r->nsemax - r->nsemin + 1;
   if (sigma_calc_out) MGW_TRY(download(c, sigma_calc_out, find_buf(c, "sigma_calc"), (size_t)2 * nomega_calc * nse));
-  MGW_HIP(hipStreamSynchronize(c->stream));
+  MGW_TRY(sync(c));
   return MGW_OK;
 }
 
@@ -2456,7 +2539,7 @@ int mgw_gw_selfenergy_contour(mgw_ctx* c, const mgw_ranges* r, double spin_fact,
     MGW_TRY(rc);
   }
   if (de_max_out) *de_max_out = de_max;
-  MGW_HIP(hipStreamSynchronize(c->stream));
+  MGW_TRY(sync(c));
   return MGW_OK;
 }
 
@@ -2467,7 +2550,7 @@ int mgw_pade_fit(mgw_ctx* c, int nse, int nomega_calc, const double* omega_calc,
               "mgw_pade_fit: invalid arguments");
   MGW_TRY(pade_fit(c, nse, nomega_calc, omega_calc, sigma_calc, nomega, omega, eta));
   if (sigma_out) MGW_TRY(download(c, sigma_out, find_buf(c, "sigma"), (size_t)2 * nomega * nse));
-  MGW_HIP(hipStreamSynchronize(c->stream));
+  MGW_TRY(sync(c));
   return MGW_OK;
 }
 
@@ -2582,7 +2665,7 @@ int mgw_g0w0(mgw_ctx* c, const mgw_g0w0_params* prm, const mgw_ranges* r, const 
     energies[0] = en_rpa;
     energies[1] = en_gw;
   }
-  MGW_HIP(hipStreamSynchronize(c->stream));
+  MGW_TRY(sync(c));
   return MGW_OK;
 }
 
