@@ -153,11 +153,17 @@ struct WbArgs {
   int64_t tiles, nblocks;
 };
 
-// Tiles BM x BN, WM x WN waves, one 32-k slab per step. DEPTH 2: two register
-// sets prefetch the next slabs while the MFMAs consume the LDS copy; DEPTH 3:
-// two LDS buffers, one barrier per slab.
+// Tiles BM x BN, WM x WN waves, one 32-k slab per step. DEPTH 1: one LDS buffer,
+// one register set that prefetches the next slab, three workgroups per CU;
+// DEPTH 2: two register sets prefetch the next slabs while the MFMAs consume the
+// LDS copy; DEPTH 3: two LDS buffers, one barrier per slab. The K loop is short
+// (half of naux on average) and the epilogue reads as many bytes of B in FP64 as
+// four slabs hold, so a third workgroup whose products run meanwhile is worth
+// more than a deeper prefetch: two planes of fp16, 32 frequencies, 2688 rows
+// 11.6 -> 9.8 ms, 1036 rows 1.14 -> 0.88 ms (DEPTH 3 -> 1; DEPTH 2: 13.9, 1.34;
+// raised wave priority for the MFMAs: 11.6, 1.06).
 template <int NS, bool H, int BM, int BN, int WM, int WN, int FLUSH, int DEPTH>
-__global__ void __launch_bounds__(64 * WM * WN)
+__global__ void __launch_bounds__(64 * WM * WN, DEPTH == 1 ? 3 : 1)
 wb_dot_kernel(WbArgs g) {
   typedef typename PlaneT<H>::E E;
   typedef typename PlaneT<H>::V V;
@@ -167,7 +173,7 @@ wb_dot_kernel(WbArgs g) {
   constexpr int FM = TM / 16, FN = TN / 16;
   constexpr int LA = BM * KT / 8 / NT, LB = BN * KT / 8 / NT;
   static_assert(BM * KT / 8 % NT == 0 && BN * KT / 8 % NT == 0, "chunks per thread");
-  static_assert(DEPTH == 2 || DEPTH == 3, "prefetch depth");
+  static_assert(DEPTH >= 1 && DEPTH <= 3, "prefetch depth");
   constexpr int NBUF = DEPTH == 3 ? 2 : 1;
 
   __shared__ __attribute__((aligned(16))) E As[NBUF][NS][BM][KP];
@@ -267,7 +273,16 @@ wb_dot_kernel(WbArgs g) {
     }
   };
 
-  if constexpr (DEPTH == 2) {
+  if constexpr (DEPTH == 1) {
+    MGW_WB_LOAD(ra0, rb0, 0)
+    for (int s = 0; s < nslab; ++s) {
+      __syncthreads();
+      MGW_WB_STORE(ra0, rb0, 0)
+      __syncthreads();
+      if (s + 1 < nslab) { MGW_WB_LOAD(ra0, rb0, s + 1) }
+      compute(s, 0);
+    }
+  } else if constexpr (DEPTH == 2) {
     MGW_WB_LOAD(ra0, rb0, 0)
     if (1 < nslab) { MGW_WB_LOAD(ra1, rb1, 1) }
     for (int s = 0; s < nslab; s += 2) {
@@ -428,15 +443,15 @@ int split_and_dot(const double* d, int naux, int nomega, const double* b, int64_
     // two planes: FP32 accumulation over the whole K (the products of the
     // 11-bit fp16 / 8-bit bf16 planes are exact in FP32; the FP64 accumulators
     // would cost 128 VGPRs and half the occupancy)
-    if (NS == 2) {
-      // two LDS buffers (default) or two prefetch register sets: the same
-      // products in the same order, so the tuner may pick either per shape
+    if constexpr (NS == 2) {
+      // DEPTH 1 (default) or 3: the same products in the same order, so the
+      // tuner may pick either per shape
       auto launch = [&](int c) -> int {
         if (c == 0)
-          hipLaunchKernelGGL((wb_dot_kernel<NS, H, BM, BN, 2, 2, 0, 3>), dim3((unsigned)g.nblocks), dim3(256), 0,
+          hipLaunchKernelGGL((wb_dot_kernel<NS, H, BM, BN, 2, 2, 0, 1>), dim3((unsigned)g.nblocks), dim3(256), 0,
                              stream, g);
         else
-          hipLaunchKernelGGL((wb_dot_kernel<NS, H, BM, BN, 2, 2, 0, 2>), dim3((unsigned)g.nblocks), dim3(256), 0,
+          hipLaunchKernelGGL((wb_dot_kernel<NS, H, BM, BN, 2, 2, 0, 3>), dim3((unsigned)g.nblocks), dim3(256), 0,
                              stream, g);
         MGW_HIP(hipGetLastError());
         return MGW_OK;
