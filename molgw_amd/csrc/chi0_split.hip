@@ -198,10 +198,6 @@ struct SyrkArgs {
   int kc_slabs, nkc;
   float* part;
   const double* unscale;   // per frequency of the chunk (FP16X3), else null
-  // part of the lower triangle that this launch covers (`tiles` tiles of it;
-  // partial tiles are addressed by the whole triangle's order): row >= 0, the
-  // tiles (row, 0 .. row) only
-  int row, ptiles;
 };
 
 // Lower-triangle tiles BM x BM, WM x WN waves, one 32-k slab per step.
@@ -240,12 +236,7 @@ chi_syrk_kernel(SyrkArgs g) {
   const int kc = KSPLIT ? (int)((L % per_f) / g.tiles) : 0;
   const int tile = (int)(L % g.tiles);
   int bm, bn;
-  if (g.row >= 0) {
-    bm = g.row;
-    bn = tile;
-  } else {
-    tri_grouped(tile, g.tm, bm, bn);
-  }
+  tri_grouped(tile, g.tm, bm, bn);
   const int m0 = bm * BM, n0 = bn * BM;
 
   const E* __restrict__ Ya = static_cast<const E*>(g.y) + (int64_t)f * g.fstride + (int64_t)m0 * KT;
@@ -372,8 +363,7 @@ chi_syrk_kernel(SyrkArgs g) {
 
   if constexpr (KSPLIT) {
     // FP32 partial tile, column-major BM x BM; summed in FP64 by chi_ksplit_reduce_kernel
-    const int pt = g.row >= 0 ? tri_grouped_index(bm, bn, g.tm) : tile;
-    float* __restrict__ P = g.part + ((int64_t)(f * g.ptiles + pt) * g.nkc + kc) * (BM * BM);
+    float* __restrict__ P = g.part + ((int64_t)(f * g.tiles + tile) * g.nkc + kc) * (BM * BM);
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
@@ -688,17 +678,23 @@ chi_syrk_pipe_kernel(SyrkArgs g) {
 // read wait for copies of its own wave that it cannot tell apart from it.
 // Against 128-wide tiles a panel is read half as often from L2 (the 128-wide
 // kernel asks it for two thirds of its rate at full MFMA speed) and LDS is read
-// 0.75 times per MFMA. Same products in the same order per accumulator as
-// chi_syrk_kernel: identical results. 2688 rows, 97280 transitions, 32
-// frequencies: 69 -> 56 ms (1.02 -> 1.32 PFLOP/s of fp16 MFMA).
+// 0.75 times per MFMA. With an odd number of 128-wide tile rows the last row goes
+// in half tiles of 128 x 256, eight waves of 64 x 64 taking the same turns, beside
+// the full tiles of the same K range, whose panels they read: in a launch of
+// their own every frequency's planes are read again (4.9 TB/s, and nothing but).
+// Same products in the same order per accumulator as chi_syrk_kernel: identical
+// results. 2688 rows, 97280 transitions, 32 frequencies: 69 -> 51 ms (1.02 ->
+// 1.45 PFLOP/s of fp16 MFMA; 53 with the last row on 128-wide tiles afterwards,
+// 52 on half tiles afterwards); 1036 rows, 12201 transitions: 1.50 -> 1.30 ms
+// (1.43, 1.36).
 constexpr int waitcnt(int vm, int lgkm) { return (vm & 15) | (7 << 4) | (lgkm << 8) | ((vm >> 4) << 14); }
 
 template <bool H>
 __global__ void __launch_bounds__(512, 2)
-chi_syrk_pp_kernel(SyrkArgs g, int t256) {
+chi_syrk_pp_kernel(SyrkArgs g) {
   typedef typename PlaneT<H>::E E;
   typedef typename PlaneT<H>::V V;
-  constexpr int BM = 256, NS = 2, TM = 128, TN = 64, FM = TM / 16, FN = TN / 16;
+  constexpr int BM = 256, NS = 2, TN = 64, FN = TN / 16;
   __shared__ __attribute__((aligned(16))) E S0[2][NS][BM][KT];   // [operand][plane][row][k]
   __shared__ __attribute__((aligned(16))) E S1[2][NS][BM][KT];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -707,41 +703,44 @@ chi_syrk_pp_kernel(SyrkArgs g, int t256) {
   const int wm = wave & 1, wn = wave >> 1;
   const int group = wave >> 2;
   const int64_t L = xcd_logical(blockIdx.x, g.nblocks);
-  const int64_t per_f = (int64_t)g.nkc * g.tiles;
+  const int t256 = g.tm / 2, nfull = t256 * (t256 + 1) / 2;
+  const int tiles = nfull + (g.tm % 2 ? t256 + 1 : 0);
+  const int64_t per_f = (int64_t)g.nkc * tiles;
   const int f = (int)(L / per_f);
-  const int kc = (int)((L % per_f) / g.tiles);
-  const int tile = (int)(L % g.tiles);
-  int bm, bn;
-  tri_grouped(tile, t256, bm, bn);
-  // sub-tile of this wave, in 128-wide tiles; strictly above the diagonal it
-  // only copies
-  const int bm1 = 2 * bm + wm, bn1 = 2 * bn + (wn >> 1);
+  const int kc = (int)((L % per_f) / tiles);
+  const int tile = (int)(L % tiles);
+  const bool half = tile >= nfull;
+  int bm = 0, bn = tile - nfull;
+  if (!half) tri_grouped(tile, t256, bm, bn);
+  // first row of the panels and, in 128-wide tiles, sub-tile of this wave;
+  // strictly above the diagonal it only copies
+  const int row0 = half ? (g.tm - 1) * 128 : bm * BM;
+  const int bm1 = half ? g.tm - 1 : 2 * bm + wm, bn1 = 2 * bn + (wn >> 1);
   const bool on = bm1 >= bn1;
 
   // the sixteen copies of a slab of a wave of group 0: the 1 KB windows of 16
-  // rows of one plane (pl) of one operand (op); chunks swizzled as lds_chunk
+  // rows of one plane (pl) of one operand (op); chunks swizzled as lds_chunk.
+  // A half tile's row panel and the last column panel of an odd number of
+  // 128-wide tiles have eight.
   const int op = (wave >> 1) & 1, pl = wave & 1;
   const int rl = lane >> 2, jl = (lane & 3) ^ ((rl >> 1) & 3);
   const E* __restrict__ src = static_cast<const E*>(g.y) + (int64_t)f * g.fstride + pl * g.plane +
-                              (int64_t)((op ? bn : bm) * BM) * KT;
+                              (int64_t)(op ? bn * BM : row0) * KT;
+  const bool wide = op ? 2 * bn + 1 < g.tm : !half;
   const unsigned lo = (rl * KT + 8 * jl) * sizeof(E);
   const int64_t slab = (int64_t)g.ppad * KT;
   const int fr = lane & 15, fq = lane >> 4;
   const int fo = 8 * lds_chunk(fr, fq);
 
-  f4 part[FM][FN];
-#pragma unroll
-  for (int i = 0; i < FM; ++i)
-#pragma unroll
-    for (int j = 0; j < FN; ++j) part[i][j] = f4{0.f, 0.f, 0.f, 0.f};
-  V a[NS][FM], b[NS][FN];
-
-#define MGW_PP_ISSUE(S_, SB)                                                                              \
-  _Pragma("unroll") for (int c = 0; c < 16; ++c)                                                          \
+#define MGW_PP_COPY(S_, SB, C0)                                                                           \
+  _Pragma("unroll") for (int c = C0; c < C0 + 8; ++c)                                                     \
     __builtin_amdgcn_global_load_lds(                                                                     \
         reinterpret_cast<const unsigned*>(                                                                \
             reinterpret_cast<const char*>(src + (int64_t)(S_) * slab + c * 16 * KT) + lo),                \
         reinterpret_cast<unsigned*>(&SB[op][pl][16 * c][0]), 16, 0, 0);
+#define MGW_PP_ISSUE(S_, SB)                                                                              \
+  MGW_PP_COPY(S_, SB, 0)                                                                                  \
+  if (wide) { MGW_PP_COPY(S_, SB, 8) }
 #define MGW_PP_READ(SB)                                                                                   \
   _Pragma("unroll") for (int q = 0; q < NS; ++q) {                                                        \
     _Pragma("unroll") for (int i = 0; i < FM; ++i)                                                        \
@@ -758,74 +757,87 @@ chi_syrk_pp_kernel(SyrkArgs g, int t256) {
   __builtin_amdgcn_s_barrier();                                                                           \
   __builtin_amdgcn_sched_barrier(0);                                                                      \
   __asm__ __volatile__("" ::: "memory");
-  auto multiply = [&]() __attribute__((always_inline)) {
-    constexpr int QA[3] = {1, 0, 0};
-    constexpr int QB[3] = {0, 1, 0};
-    __builtin_amdgcn_s_setprio(1);
+  auto run = [&](auto is_half) __attribute__((always_inline)) {
+    constexpr bool HALF = decltype(is_half)::value;
+    constexpr int TM = HALF ? 64 : 128, FM = TM / 16;
+    f4 part[FM][FN];
 #pragma unroll
-    for (int pr = 0; pr < 3; ++pr)
+    for (int i = 0; i < FM; ++i)
 #pragma unroll
-      for (int i = 0; i < FM; ++i)
+      for (int j = 0; j < FN; ++j) part[i][j] = f4{0.f, 0.f, 0.f, 0.f};
+    V a[NS][FM], b[NS][FN];
+    auto multiply = [&]() __attribute__((always_inline)) {
+      constexpr int QA[3] = {1, 0, 0};
+      constexpr int QB[3] = {0, 1, 0};
+      __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-        for (int j = 0; j < FN; ++j) part[i][j] = mfma16x16x32<H>(b[QB[pr]][j], a[QA[pr]][i], part[i][j]);
-    __builtin_amdgcn_s_setprio(0);
-  };
+      for (int pr = 0; pr < 3; ++pr)
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+          for (int j = 0; j < FN; ++j) part[i][j] = mfma16x16x32<H>(b[QB[pr]][j], a[QA[pr]][i], part[i][j]);
+      __builtin_amdgcn_s_setprio(0);
+    };
 
-  const int s0 = kc * g.kc_slabs;
-  const int ns = min(g.nkt, s0 + g.kc_slabs) - s0;     // >= 1
-  if (group == 0) {
-    MGW_PP_ISSUE(s0, S0)
-    if (ns > 1) { MGW_PP_ISSUE(s0 + 1, S1) }
-    MGW_PP_BARRIER(0)
+    const int s0 = kc * g.kc_slabs;
+    const int ns = min(g.nkt, s0 + g.kc_slabs) - s0;     // >= 1
+    if (group == 0) {
+      MGW_PP_ISSUE(s0, S0)
+      if (ns > 1) { MGW_PP_ISSUE(s0 + 1, S1) }
+      MGW_PP_BARRIER(0)
 #define MGW_PP_G0(S_, SC, SN)                                          \
-  MGW_PP_READ(SC)                                                      \
-  __asm__ __volatile__("" ::: "memory");                               \
-  if ((S_) >= 1 && (S_) + 1 < ns) { MGW_PP_ISSUE(s0 + (S_) + 1, SN) }   \
-  MGW_PP_BARRIER(63)                                                   \
-  multiply();                                                          \
-  MGW_PP_BARRIER(0)
-    int s = 0;
-    for (; s + 1 < ns; s += 2) {
-      MGW_PP_G0(s, S0, S1)
-      MGW_PP_G0(s + 1, S1, S0)
-    }
-    if (s < ns) { MGW_PP_G0(s, S0, S1) }
+    MGW_PP_READ(SC)                                                      \
+    __asm__ __volatile__("" ::: "memory");                               \
+    if ((S_) >= 1 && (S_) + 1 < ns) { MGW_PP_ISSUE(s0 + (S_) + 1, SN) }   \
+    MGW_PP_BARRIER(63)                                                   \
+    multiply();                                                          \
+    MGW_PP_BARRIER(0)
+      int s = 0;
+      for (; s + 1 < ns; s += 2) {
+        MGW_PP_G0(s, S0, S1)
+        MGW_PP_G0(s + 1, S1, S0)
+      }
+      if (s < ns) { MGW_PP_G0(s, S0, S1) }
 #undef MGW_PP_G0
-  } else if (!on) {
-    MGW_PP_BARRIER(63)
-    for (int s = 0; s < 2 * ns; ++s) { MGW_PP_BARRIER(63) }
-    return;
-  } else {
+    } else if (!on) {
+      MGW_PP_BARRIER(63)
+      for (int s = 0; s < 2 * ns; ++s) { MGW_PP_BARRIER(63) }
+      return;
+    } else {
 #define MGW_PP_G1(SC) \
-  multiply();         \
-  MGW_PP_BARRIER(63)  \
-  MGW_PP_READ(SC)     \
-  MGW_PP_BARRIER(63)
+    multiply();         \
+    MGW_PP_BARRIER(63)  \
+    MGW_PP_READ(SC)     \
     MGW_PP_BARRIER(63)
-    MGW_PP_BARRIER(63)
-    MGW_PP_READ(S0)
-    MGW_PP_BARRIER(63)
-    int s = 1;
-    for (; s + 1 < ns; s += 2) {
-      MGW_PP_G1(S1)
-      MGW_PP_G1(S0)
-    }
-    if (s < ns) { MGW_PP_G1(S1) }
+      MGW_PP_BARRIER(63)
+      MGW_PP_BARRIER(63)
+      MGW_PP_READ(S0)
+      MGW_PP_BARRIER(63)
+      int s = 1;
+      for (; s + 1 < ns; s += 2) {
+        MGW_PP_G1(S1)
+        MGW_PP_G1(S0)
+      }
+      if (s < ns) { MGW_PP_G1(S1) }
 #undef MGW_PP_G1
-    multiply();
-  }
+      multiply();
+    }
+
+    float* __restrict__ P = g.part + ((int64_t)(f * g.tiles + tri_grouped_index(bm1, bn1, g.tm)) * g.nkc + kc) * (128 * 128) +
+                            (wn & 1) * TN * 128 + (HALF ? wm * TM : 0);
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) P[(i * 16 + fr) + (j * 16 + 4 * fq + r) * 128] = part[i][j][r];
+  };
+  if (half) run(std::true_type{});
+  else run(std::false_type{});
 #undef MGW_PP_ISSUE
+#undef MGW_PP_COPY
 #undef MGW_PP_READ
 #undef MGW_PP_BARRIER
-
-  float* __restrict__ P = g.part + ((int64_t)(f * g.ptiles + tri_grouped_index(bm1, bn1, g.tm)) * g.nkc + kc) * (128 * 128) +
-                          (wn & 1) * TN * 128;
-#pragma unroll
-  for (int i = 0; i < FM; ++i)
-#pragma unroll
-    for (int j = 0; j < FN; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) P[(i * 16 + fr) + (j * 16 + 4 * fq + r) * 128] = part[i][j][r];
 }
 
 // SYRK kernel of the K-split planes path: MGW_CHI_SYRK = 0 (register
@@ -1368,24 +1380,14 @@ chi_scale_kernel(const double* __restrict__ xpart, int nb, const double* __restr
 // bytes in front of the planes: scale, unscale (per frequency), |X| partial maxima
 size_t scale_header_bytes(int nomega) { return ((size_t)(2 * nomega + NB_MAX) * sizeof(double) + 255) / 256 * 256; }
 
-// The lower triangle on 256-wide tiles; with an odd number of 128-wide tile
-// rows, the last row on 128-wide ones.
 constexpr int64_t PP_FILL = 512;
 
 template <bool H>
 int launch_syrk_pp(const SyrkArgs& g0, hipStream_t stream) {
   SyrkArgs g = g0;
   const int t256 = g.tm / 2;
-  g.tiles = t256 * (t256 + 1) / 2;
-  g.nblocks = (int64_t)g.tiles * g.nkc * g.nf;
-  hipLaunchKernelGGL((chi_syrk_pp_kernel<H>), dim3((unsigned)g.nblocks), dim3(512), 0, stream, g, t256);
-  MGW_HIP(hipGetLastError());
-  if (g.tm % 2 == 0) return MGW_OK;
-  g.row = g.tm - 1;
-  g.tiles = g.tm;
-  g.nblocks = (int64_t)g.tiles * g.nkc * g.nf;
-  hipLaunchKernelGGL((chi_syrk_kernel<2, H, 128, 2, 2, 4, 1, 1, true>), dim3((unsigned)g.nblocks), dim3(256), 0, stream,
-                     g);
+  g.nblocks = ((int64_t)t256 * (t256 + 1) / 2 + (g.tm % 2 ? t256 + 1 : 0)) * g.nkc * g.nf;
+  hipLaunchKernelGGL((chi_syrk_pp_kernel<H>), dim3((unsigned)g.nblocks), dim3(512), 0, stream, g);
   MGW_HIP(hipGetLastError());
   return MGW_OK;
 }
@@ -1438,7 +1440,6 @@ int split_and_syrk(const double* x, int naux, int npole, const double* sw, int n
     g.C = chi + (int64_t)f0 * naux * naux; g.strideC = (int64_t)naux * naux;
     g.kc_slabs = L.kc_slabs; g.nkc = L.nkc; g.part = part;
     g.unscale = H ? uns + f0 : nullptr;
-    g.row = -1; g.ptiles = L.tiles;
     const int depth = chi_prefetch_depth(NS);
     const dim3 block(256);
     if (ksplit) {

@@ -1,5 +1,5 @@
-"""The FP16x3 / BF16x3 chi0 build on 256-wide tiles (with a last row of 128-wide
-ones when the tile rows are odd) does the products of the 128-wide kernel in
+"""The FP16x3 / BF16x3 chi0 build on 256-wide tiles (with a last row of half tiles,
+128 x 256, when the 128-wide tile rows are odd) does the products of the 128-wide kernel in
 the same order: identical chi0 (through its inverse) for sizes at the edges of
 the tiles and odd and even slab counts, with enough frequencies that the
 256-wide tiles are taken."""
