@@ -263,6 +263,15 @@ bool is_resident_input(const std::string& name) {
 // trim eagerly, they are freed here.
 int scratch_done(mgw_ctx* c, const std::string& name);
 
+// End of the use of a list that is short for all but the largest molecules: a
+// free costs the host 10 to 20 us and the next call an allocation, so one of up
+// to 1 MiB stays until a trim.
+int release_large(mgw_ctx* c, const std::string& name) {
+  auto it = c->ledger.bufs.find(name);
+  const bool large = it != c->ledger.bufs.end() && it->second.bytes > (1 << 20);
+  return large ? release(c, name) : scratch_done(c, name);
+}
+
 // Small transfers go through the context's pinned memory, and vectors that are
 // needed together in one copy: from or to pageable memory a copy costs the host
 // 9 us however small it is. A Pade solve of one water molecule (41 functions)
@@ -1640,9 +1649,7 @@ int mgw_set_eri_3center(mgw_ctx* c, const double* eri, int64_t npair, int nauxil
   MGW_TRY(launch_unpack_ri(packed, npair, nauxil, kl_d, nbf, dense, c->stream, !complete, amax));
   MGW_TRY(sync(c));
   MGW_TRY(release(c, "ri_packed"));
-  // a free and a new allocation cost the next solve 20 us: a short pair list stays
-  if (kl.size() * sizeof(int32_t) > (1 << 20)) MGW_TRY(release(c, "ri_kl"));
-  else MGW_TRY(scratch_done(c, "ri_kl"));
+  MGW_TRY(release_large(c, "ri_kl"));
   c->nbf = nbf;
   c->naux = nauxil;
   c->has_ri = true;
@@ -1781,14 +1788,17 @@ int mgw_build_eri_3center(mgw_ctx* c, const double* eri_3center_tmp, int64_t ipa
   MGW_TRY(launch_unpack_ri(packed, mpair, nk, kl_d, nbf, dense, c->stream, false, find_buf(c, "ri_absmax")));
   if (eri_3center_out) {
     // rows ipair_first.. of the caller's eri_3center(npair, nauxil_kept)
-    MGW_HIP(hipMemcpy2DAsync(eri_3center_out + (ipair_first - 1), (size_t)npair * sizeof(double), packed,
+    if (mpair == npair)      // contiguous: a plain copy runs at twice the rate of a strided one
+      MGW_HIP(hipMemcpyAsync(eri_3center_out, packed, (size_t)npair * nk * sizeof(double), hipMemcpyDefault, c->stream));
+    else
+      MGW_HIP(hipMemcpy2DAsync(eri_3center_out + (ipair_first - 1), (size_t)npair * sizeof(double), packed,
                              (size_t)mpair * sizeof(double), (size_t)mpair * sizeof(double), nk, hipMemcpyDefault,
                              c->stream));
   }
   MGW_TRY(sync(c));
   MGW_TRY(release(c, "ri_tmp"));
   MGW_TRY(release(c, "ri_packed"));
-  MGW_TRY(release(c, "ri_kl"));
+  MGW_TRY(release_large(c, "ri_kl"));
   c->build_next = ipair_first + mpair;
   if (c->build_next == npair + 1) {
     c->nbf = nbf;
@@ -1835,22 +1845,13 @@ int upload_shells(mgw_ctx* c, const std::string& prefix, const mgw_shells* sh, E
   nfunc = sh->function_offset[n];
   int32_t *l_d, *poff_d, *toff_d, *foff_d;
   double *cen_d, *exp_d, *coef_d, *tm_d;
-  MGW_TRY(upload(c, prefix + "_l", sh->am, n, &l_d));
-  MGW_TRY(upload(c, prefix + "_x0", sh->x0, 3 * (size_t)n, &cen_d));
-  MGW_TRY(upload(c, prefix + "_poff", sh->prim_offset, n + 1, &poff_d));
-  MGW_TRY(upload(c, prefix + "_alpha", sh->alpha, nprim, &exp_d));
-  MGW_TRY(upload(c, prefix + "_coeff", sh->coeff, nprim, &coef_d));
-  MGW_TRY(upload(c, prefix + "_toff", sh->transform_offset, n, &toff_d));
-  MGW_TRY(upload(c, prefix + "_tmat", sh->transform, (size_t)ntmat, &tm_d));
-  MGW_TRY(upload(c, prefix + "_foff", sh->function_offset, n + 1, &foff_d));
+  MGW_TRY(upload_group(c, prefix, {part_of(sh->am, (size_t)n, &l_d), part_of(sh->x0, 3 * (size_t)n, &cen_d),
+                                   part_of(sh->prim_offset, (size_t)n + 1, &poff_d), part_of(sh->alpha, (size_t)nprim, &exp_d),
+                                   part_of(sh->coeff, (size_t)nprim, &coef_d), part_of(sh->transform_offset, (size_t)n, &toff_d),
+                                   part_of(sh->transform, (size_t)ntmat, &tm_d),
+                                   part_of(sh->function_offset, (size_t)n + 1, &foff_d)}));
   out.l = l_d; out.center = cen_d; out.poff = poff_d; out.exps = exp_d; out.coefs = coef_d;
   out.toff = toff_d; out.tmat = tm_d; out.foff = foff_d;
-  return MGW_OK;
-}
-
-int release_shells(mgw_ctx* c, const std::string& prefix) {
-  for (const char* f : {"_l", "_x0", "_poff", "_alpha", "_coeff", "_toff", "_tmat", "_foff"})
-    MGW_TRY(release(c, prefix + f));
   return MGW_OK;
 }
 
@@ -1948,9 +1949,8 @@ int mgw_eri_2center_ao(mgw_ctx* c, const mgw_shells* auxil, int where, double* e
     }
   if (where == MGW_MEM_HOST) MGW_TRY(download(c, eri_2center, out, (size_t)naux * naux));
   MGW_TRY(sync(c));
-  for (const char* b : {"int_kfun", "int_pairs", "int_out2"}) MGW_TRY(release(c, b));
-  MGW_TRY(release_shells(c, "int_aux"));
-  MGW_TRY(release_shells(c, "int_unit"));
+  MGW_TRY(release(c, "int_out2"));
+  for (const char* b : {"int_kfun", "int_pairs", "int_aux", "int_unit"}) MGW_TRY(release_large(c, b));
   return MGW_OK;
 }
 
@@ -1978,9 +1978,15 @@ int mgw_eri_3center_ao(mgw_ctx* c, const mgw_shells* basis, const mgw_shells* au
   // shell pairs (s1, s2) with l1 >= l2, grouped by (l1, l2)
   const int n = basis->nshell;
   std::vector<std::vector<int32_t>> cls(64);
-  for (int a = 0; a < n; ++a)
-    for (int b = 0; b <= a; ++b) {
-      int s1 = a, s2 = b;
+  // deeply contracted shells first: their pairs take longest (64 primitive
+  // pairs where a valence shell has one) and would run alone at a launch's end
+  std::vector<int> order(n);
+  std::iota(order.begin(), order.end(), 0);
+  auto depth = [&](int k) { return basis->prim_offset[k + 1] - basis->prim_offset[k]; };
+  std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return depth(a) > depth(b); });
+  for (int ka = 0; ka < n; ++ka)
+    for (int kb = 0; kb <= ka; ++kb) {
+      int s1 = std::max(order[ka], order[kb]), s2 = std::min(order[ka], order[kb]);
       if (basis->am[s1] < basis->am[s2]) std::swap(s1, s2);
       const int l1 = basis->am[s1], l2 = basis->am[s2];
       MGW_REQUIRE(l1 <= 3, MGW_ERR_ARG, "mgw_eri_3center_ao: orbital angular momentum above 3 is not supported on the GPU");
@@ -2035,9 +2041,8 @@ int mgw_eri_3center_ao(mgw_ctx* c, const mgw_shells* basis, const mgw_shells* au
   }
   if (eri_3center_tmp && where == MGW_MEM_HOST) MGW_TRY(download(c, eri_3center_tmp, out, (size_t)npair * naux));
   MGW_TRY(sync(c));
-  for (const char* b : {"int_pairmap", "int_pairs", "int_kfun", "int_out3"}) MGW_TRY(release(c, b));
-  MGW_TRY(release_shells(c, "int_bas"));
-  MGW_TRY(release_shells(c, "int_aux"));
+  MGW_TRY(release(c, "int_out3"));
+  for (const char* b : {"int_pairmap", "int_pairs", "int_kfun", "int_bas", "int_aux"}) MGW_TRY(release_large(c, b));
   if (!eri_3center_tmp) {
     c->has_ri_tmp3 = true;
     c->ri_tmp3_npair = npair;

@@ -13,16 +13,26 @@
 //
 // Work decomposition. Shell pairs are grouped by (l_a, l_b), ket functions
 // (shell, function) by l_c; one launch per class (l_a, l_b, l_c) with the
-// three angular momenta as template parameters, so every loop below unrolls
-// and indices into R, E and the accumulators are compile-time constants. A
-// workgroup owns one bra shell pair and 128 ket functions of one l_c; the
-// bra's primitive pairs are expanded (E coefficients, P, p) cooperatively
-// into LDS in batches and read as broadcasts. Each thread keeps, per ket
-// primitive, R in one in-place array (levels n = L .. 0, sums t+u+v
-// processed from high to low so that level n + 1 is read before it is
-// overwritten), the ket's Hermite coefficients of its final function, and
-// the Cartesian bra block of its function in registers; the bra is
+// three angular momenta as template parameters, so every index into R, E and
+// the accumulators is a compile-time constant. A workgroup owns one bra shell
+// pair and 128 ket functions of one l_c; the bra's primitive pairs are expanded
+// (E coefficients, P, p) cooperatively into LDS in batches and read as
+// broadcasts. Each thread keeps, per ket primitive, R in one in-place array
+// (levels n = L .. 0, sums t+u+v processed from high to low so that level n + 1
+// is read before it is overwritten), the ket's Hermite coefficients of its final
+// function, and the Cartesian bra block of its function in registers; the bra is
 // transformed to the final functions once at the end.
+//
+// What bounds it: FP64 instructions in the deeply contracted (s s|, (p s|
+// classes (64 primitive pairs a bra), registers and code size in the others,
+// where a bra has one primitive pair and every instruction is fetched for one
+// use. So divisions by constants are products, a primitive takes one division
+// and one square root, an uncontracted ket's coefficients (half of them zero by
+// parity, and skipped) are found once, E is read again from LDS rather than
+// held, and the transform at the end is a loop. All classes of an 8-carbon
+// alkane in cc-pVDZ / cc-pVDZ-RI (202 functions): 2.02 -> 0.93 ms, of which
+// (s s|f) 0.42 -> 0.07 (its coefficients were in scratch memory) and the four
+// (d d| 0.32 -> 0.10.
 //
 // Boys function: F_L(T) by a 7-term Taylor series around the nearest point
 // of a table F_n(k h), h = 0.05, T <= 36 (error below 2e-15 relative), then
@@ -32,9 +42,25 @@
 #include "mgw_internal.h"
 
 #include <cmath>
+#include <type_traits>
+#include <utility>
 
 namespace mgw {
 namespace eri {
+
+// f(0), .., f(N - 1) with the index as a constant expression: the loops below
+// nest four deep with bounds of one another, which the compiler's unroller gives
+// up on at the higher angular momenta; indices it does not know put an array
+// into scratch memory
+template <class F, int... I>
+__device__ __attribute__((always_inline)) inline void unroll_seq(F&& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ __attribute__((always_inline)) inline void unroll(F&& f) {
+  unroll_seq(f, std::make_integer_sequence<int, N>{});
+}
+#define MGW_UNROLL(i, n) unroll<(n)>([&](auto i) __attribute__((always_inline))
 
 constexpr int BOYS_N = 17;          // orders 0 .. 16 in the table (L <= 10 plus 6 Taylor terms)
 constexpr int BOYS_TAYLOR = 6;
@@ -49,6 +75,24 @@ __host__ __device__ constexpr int hidx(int t, int u, int v) {
   const int s = t + u + v, r = u + v;
   return s * (s + 1) * (s + 2) / 6 + r * (r + 1) / 2 + v;
 }
+// and back: the sum s and r = u + v of an index, then t, u, v
+__host__ __device__ constexpr int herm_s(int m) {
+  int s = 0;
+  while (nherm(s) <= m) ++s;
+  return s;
+}
+__host__ __device__ constexpr int herm_r(int m) {
+  const int s = herm_s(m), k = s > 0 ? m - nherm(s - 1) : 0;
+  int r = 0;
+  while ((r + 1) * (r + 2) / 2 <= k) ++r;
+  return r;
+}
+__host__ __device__ constexpr int herm_t(int m) { return herm_s(m) - herm_r(m); }
+__host__ __device__ constexpr int herm_v(int m) {
+  const int s = herm_s(m), r = herm_r(m);
+  return m - (s > 0 ? nherm(s - 1) : 0) - r * (r + 1) / 2;
+}
+__host__ __device__ constexpr int herm_u(int m) { return herm_r(m) - herm_v(m); }
 // Cartesian component c of a shell of angular momentum l: (l - i, i - k, k)
 // for i = 0 .. l, k = 0 .. i (x power decreasing first), as the basis module
 // orders them
@@ -95,16 +139,16 @@ __device__ inline void boys_eval(double T, const double* __restrict__ tab, doubl
     // F_L(T) = sum_j F_{L+j}(t_k) (t_k - T)^j / j!
     double s = row[BOYS_TAYLOR];
 #pragma unroll
-    for (int j = BOYS_TAYLOR - 1; j >= 0; --j) s = row[j] + s * d / (double)(j + 1);
+    for (int j = BOYS_TAYLOR - 1; j >= 0; --j) s = row[j] + s * (d * (1.0 / (double)(j + 1)));
     f[L] = s;
     const double e = exp(-T);
 #pragma unroll
-    for (int n = L - 1; n >= 0; --n) f[n] = (2.0 * T * f[n + 1] + e) / (double)(2 * n + 1);
+    for (int n = L - 1; n >= 0; --n) f[n] = (2.0 * T * f[n + 1] + e) * (1.0 / (double)(2 * n + 1));
   } else {
-    const double e = exp(-T);
-    f[0] = 0.5 * sqrt(3.14159265358979323846 / T);
+    const double e = exp(-T), h = 0.5 / T;
+    f[0] = 0.5 * sqrt(6.28318530717958647693 * h);
 #pragma unroll
-    for (int n = 0; n < L; ++n) f[n + 1] = ((double)(2 * n + 1) * f[n] - e) / (2.0 * T);
+    for (int n = 0; n < L; ++n) f[n + 1] = ((double)(2 * n + 1) * f[n] - e) * h;
   }
 }
 
@@ -140,6 +184,40 @@ __device__ inline void hermite_pair(double a, double b, double xab, double* __re
     }
 }
 
+// Hermite coefficients of one final function of a ket primitive (1 / 2q = h):
+// K(tau nu phi) = (-1)^(tau+nu+phi) sum_c tc[c] Ec[cx][tau] Ec[cy][nu] Ec[cz][phi];
+// zero unless tau + nu + phi has the parity of LC
+template <int LC>
+__device__ inline void ket_hermite(const double* tc, double h, double* K) {
+  double ec[LC + 1][LC + 1];
+#pragma unroll
+  for (int i = 0; i <= LC; ++i)
+#pragma unroll
+    for (int t = 0; t <= LC; ++t) ec[i][t] = 0.0;
+  ec[0][0] = 1.0;
+#pragma unroll
+  for (int i = 1; i <= LC; ++i)
+#pragma unroll
+    for (int t = 0; t <= i; ++t) {
+      double v = 0.0;
+      if (t > 0) v += h * ec[i - 1][t - 1];
+      if (t + 1 <= i - 1) v += (t + 1) * ec[i - 1][t + 1];
+      ec[i][t] = v;
+    }
+#pragma unroll
+  for (int n = 0; n < nherm(LC); ++n) K[n] = 0.0;
+  MGW_UNROLL(c, ncart(LC)) {
+    constexpr int ex = cart_x(LC, c), ey = cart_y(LC, c), ez = cart_z(LC, c);
+    MGW_UNROLL(m, nherm(LC)) {
+      constexpr int t = herm_t(m), u = herm_u(m), v = herm_v(m);
+      if constexpr (t <= ex && u <= ey && v <= ez && !(((ex - t) | (ey - u) | (ez - v)) & 1)) {   // else zero
+        constexpr double sg = (LC & 1) ? -1.0 : 1.0;
+        K[m] += sg * tc[c] * ec[ex][t] * ec[ey][u] * ec[ez][v];
+      }
+    });
+  });
+}
+
 constexpr int WG = 128;   // ket functions per workgroup
 constexpr int NPB = 8;    // bra primitive pairs expanded per LDS batch
 
@@ -150,7 +228,7 @@ __global__ void __launch_bounds__(WG) eri_kernel(EriArgs g) {
   constexpr int LD = LAB + 1;
   constexpr int NE = (LA + 1) * (LB + 1) * LD;
   __shared__ double sE[NPB][3][NE];
-  __shared__ double sQ[NPB][5];   // p, P (3), contraction weight
+  __shared__ double sQ[NPB][5];   // p, P (3), contraction weight / p
 
   const int2 pr = g.pairs[blockIdx.x];
   const int sa = pr.x, sb = pr.y;
@@ -186,6 +264,16 @@ __global__ void __launch_bounds__(WG) eri_kernel(EriArgs g) {
     for (int c = 0; c < NC; ++c) tc[c] = t[c];
   }
 
+  // of a ket of one primitive (an uncontracted auxiliary shell), once for all
+  // bra primitives
+  const bool one = k1 - k0 == 1;
+  double K[nherm(LC)], qe = 1.0, qw = 0.0;
+  if (one) {
+    qe = g.C.exps[k0];
+    qw = 2.0 * 17.493418327624862 / qe * g.C.coefs[k0];   // 2 pi^(5/2)
+    ket_hermite<LC>(tc, 0.5 / qe, K);
+  }
+
   double acc[NA][NB];
 #pragma unroll
   for (int a = 0; a < NA; ++a)
@@ -207,7 +295,7 @@ __global__ void __launch_bounds__(WG) eri_kernel(EriArgs g) {
         sQ[q][1] = (a * ax + b * bx) / p;
         sQ[q][2] = (a * ay + b * by) / p;
         sQ[q][3] = (a * az + b * bz) / p;
-        sQ[q][4] = g.A.coefs[ia0 + ip / nib] * g.B.coefs[ib0 + ip % nib];
+        sQ[q][4] = g.A.coefs[ia0 + ip / nib] * g.B.coefs[ib0 + ip % nib] / p;
       }
     }
     __syncthreads();
@@ -215,8 +303,12 @@ __global__ void __launch_bounds__(WG) eri_kernel(EriArgs g) {
     for (int q = 0; q < nb; ++q) {
       const double p = sQ[q][0], px = sQ[q][1], py = sQ[q][2], pz = sQ[q][3], wab = sQ[q][4];
       for (int k = k0; k < k1; ++k) {
-        const double qe = g.C.exps[k];
-        const double alpha = p * qe / (p + qe);
+        if (!one) {
+          qe = g.C.exps[k];
+          qw = 2.0 * 17.493418327624862 / qe * g.C.coefs[k];
+          ket_hermite<LC>(tc, 0.5 / qe, K);
+        }
+        const double rpq = 1.0 / (p + qe), alpha = p * qe * rpq;
         const double xpc = px - cx, ypc = py - cy, zpc = pz - cz;
         double R[nherm(L)];
         {
@@ -228,171 +320,116 @@ __global__ void __launch_bounds__(WG) eri_kernel(EriArgs g) {
 #pragma unroll
           for (int n = 1; n <= L; ++n) pw[n] = pw[n - 1] * (-2.0 * alpha);
           R[0] = pw[L] * f[L];
-#pragma unroll
-          for (int n = L - 1; n >= 0; --n) {
-#pragma unroll
-            for (int s = L - n; s >= 1; --s)
-#pragma unroll
-              for (int r = s; r >= 0; --r)
-#pragma unroll
-                for (int v = r; v >= 0; --v) {
-                  const int t = s - r, u = r - v;
-                  double val;
-                  if (t > 0) {
-                    val = xpc * R[hidx(t - 1, u, v)];
-                    if (t > 1) val += (t - 1) * R[hidx(t - 2, u, v)];
-                  } else if (u > 0) {
-                    val = ypc * R[hidx(t, u - 1, v)];
-                    if (u > 1) val += (u - 1) * R[hidx(t, u - 2, v)];
-                  } else {
-                    val = zpc * R[hidx(t, u, v - 1)];
-                    if (v > 1) val += (v - 1) * R[hidx(t, u, v - 2)];
-                  }
-                  R[hidx(t, u, v)] = val;
-                }
+          MGW_UNROLL(step, L) {
+            constexpr int n = L - 1 - step, top = nherm(L - n) - 1;
+            MGW_UNROLL(i, top) {
+              constexpr int m = top - i, t = herm_t(m), u = herm_u(m), v = herm_v(m);
+              double val;
+              if constexpr (t > 0) {
+                val = xpc * R[hidx(t - 1, u, v)];
+                if constexpr (t > 1) val += (t - 1) * R[hidx(t - 2, u, v)];
+              } else if constexpr (u > 0) {
+                val = ypc * R[hidx(t, u - 1, v)];
+                if constexpr (u > 1) val += (u - 1) * R[hidx(t, u - 2, v)];
+              } else {
+                val = zpc * R[hidx(t, u, v - 1)];
+                if constexpr (v > 1) val += (v - 1) * R[hidx(t, u, v - 2)];
+              }
+              R[m] = val;
+            });
             R[0] = pw[n] * f[n];
-          }
-        }
-        // ket Hermite coefficients of the final function:
-        // K(tau nu phi) = (-1)^(tau+nu+phi) sum_c tc[c] Ec[cx][tau] Ec[cy][nu] Ec[cz][phi]
-        double K[nherm(LC)];
-        {
-          double ec[LC + 1][LC + 1];
-#pragma unroll
-          for (int i = 0; i <= LC; ++i)
-#pragma unroll
-            for (int t = 0; t <= LC; ++t) ec[i][t] = 0.0;
-          ec[0][0] = 1.0;
-          const double h = 0.5 / qe;
-#pragma unroll
-          for (int i = 1; i <= LC; ++i)
-#pragma unroll
-            for (int t = 0; t <= i; ++t) {
-              double v = 0.0;
-              if (t > 0) v += h * ec[i - 1][t - 1];
-              if (t + 1 <= i - 1) v += (t + 1) * ec[i - 1][t + 1];
-              ec[i][t] = v;
-            }
-#pragma unroll
-          for (int n = 0; n < nherm(LC); ++n) K[n] = 0.0;
-#pragma unroll
-          for (int c = 0; c < NC; ++c) {
-            const int ex = cart_x(LC, c), ey = cart_y(LC, c), ez = cart_z(LC, c);
-#pragma unroll
-            for (int t = 0; t <= ex; ++t)
-#pragma unroll
-              for (int u = 0; u <= ey; ++u)
-#pragma unroll
-                for (int v = 0; v <= ez; ++v) {
-                  if (((ex - t) | (ey - u) | (ez - v)) & 1) continue;   // parity: zero coefficients
-                  const double sg = ((t + u + v) & 1) ? -1.0 : 1.0;
-                  K[hidx(t, u, v)] += sg * tc[c] * ec[ex][t] * ec[ey][u] * ec[ez][v];
-                }
-          }
+          });
         }
         // ket-contracted Hermite integrals G(tuv), t + u + v <= LAB
         double G[nherm(LAB)];
-#pragma unroll
-        for (int s = 0; s <= LAB; ++s)
-#pragma unroll
-          for (int r = 0; r <= s; ++r)
-#pragma unroll
-            for (int v = 0; v <= r; ++v) {
-              const int t = s - r, u = r - v;
-              double sum = 0.0;
-#pragma unroll
-              for (int s2 = 0; s2 <= LC; ++s2)
-#pragma unroll
-                for (int r2 = 0; r2 <= s2; ++r2)
-#pragma unroll
-                  for (int v2 = 0; v2 <= r2; ++v2) {
-                    const int t2 = s2 - r2, u2 = r2 - v2;
-                    sum += K[hidx(t2, u2, v2)] * R[hidx(t + t2, u + u2, v + v2)];
-                  }
-              G[hidx(t, u, v)] = sum;
-            }
-        const double pref = 2.0 * 17.493418327624862 / (p * qe * sqrt(p + qe)) * wab * g.C.coefs[k];   // 2 pi^(5/2)
+        MGW_UNROLL(m, nherm(LAB)) {
+          constexpr int t = herm_t(m), u = herm_u(m), v = herm_v(m);
+          double sum = 0.0;
+          MGW_UNROLL(m2, nherm(LC)) {
+            if constexpr ((herm_s(m2) & 1) == (LC & 1))   // else K = 0
+              sum += K[m2] * R[hidx(t + herm_t(m2), u + herm_u(m2), v + herm_v(m2))];
+          });
+          G[m] = sum;
+        });
+        const double pref = sqrt(rpq) * wab * qw;
         // bra: acc[a][b] += pref sum_tuv Ex Ey Ez G
-#pragma unroll
-        for (int a = 0; a < NA; ++a)
-#pragma unroll
-          for (int b = 0; b < NB; ++b) {
-            const int ix = cart_x(LA, a), iy = cart_y(LA, a), iz = cart_z(LA, a);
-            const int jx = cart_x(LB, b), jy = cart_y(LB, b), jz = cart_z(LB, b);
-            const double* __restrict__ ex = &sE[q][0][(ix * (LB + 1) + jx) * LD];
-            const double* __restrict__ ey = &sE[q][1][(iy * (LB + 1) + jy) * LD];
-            const double* __restrict__ ez = &sE[q][2][(iz * (LB + 1) + jz) * LD];
-            double sum = 0.0;
-#pragma unroll
-            for (int t = 0; t <= ix + jx; ++t)
-#pragma unroll
-              for (int u = 0; u <= iy + jy; ++u) {
-                const double etu = ex[t] * ey[u];
-#pragma unroll
-                for (int v = 0; v <= iz + jz; ++v) sum += etu * ez[v] * G[hidx(t, u, v)];
-              }
-            acc[a][b] += pref * sum;
-          }
+        MGW_UNROLL(ab, NA * NB) {
+          constexpr int a = ab / NB, b = ab % NB;
+          // from (p p| on, E is read again for each function of a: kept for all
+          // of them it takes the registers of acc and G
+          if constexpr (LAB >= 2 && b == 0) __asm__ __volatile__("" ::: "memory");
+          constexpr int ix = cart_x(LA, a), iy = cart_y(LA, a), iz = cart_z(LA, a);
+          constexpr int jx = cart_x(LB, b), jy = cart_y(LB, b), jz = cart_z(LB, b);
+          const double* __restrict__ ex = &sE[q][0][(ix * (LB + 1) + jx) * LD];
+          const double* __restrict__ ey = &sE[q][1][(iy * (LB + 1) + jy) * LD];
+          const double* __restrict__ ez = &sE[q][2][(iz * (LB + 1) + jz) * LD];
+          double sum = 0.0;
+          MGW_UNROLL(t, ix + jx + 1) {
+            MGW_UNROLL(u, iy + jy + 1) {
+              const double etu = ex[t] * ey[u];
+              MGW_UNROLL(v, iz + jz + 1) { sum += etu * ez[v] * G[hidx(t, u, v)]; });
+            });
+          });
+          acc[a][b] += pref * sum;
+        });
       }
     }
   }
   if (!active) return;
 
-  // final functions of the bra: V[fa][fb] = sum_ab Ta[fa][a] Tb[fb][b] acc[a][b]
+  // final functions of the bra: V(fa, fb) = sum_ab Ta[fa][a] Tb[fb][b] acc[a][b].
+  // The loops over the functions stay loops: code that runs once costs its
+  // fetch from memory (unrolled, this part was most of the (d d|c) classes' time)
   const int nfa = g.A.foff[sa + 1] - g.A.foff[sa], nfb = g.B.foff[sb + 1] - g.B.foff[sb];
   const double* __restrict__ ta = g.A.tmat + g.A.toff[sa];
   const double* __restrict__ tb = g.B.tmat + g.B.toff[sb];
-  double half[NA][NB];   // [fa][b]
-#pragma unroll
-  for (int fa = 0; fa < NA; ++fa)
+  double half[NB];
+  auto half_row = [&](int fa) __attribute__((always_inline)) {
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
       double s = 0.0;
-      if (fa < nfa) {
 #pragma unroll
-        for (int a = 0; a < NA; ++a) s += ta[fa * NA + a] * acc[a][b];
-      }
-      half[fa][b] = s;
+      for (int a = 0; a < NA; ++a) s += ta[fa * NA + a] * acc[a][b];
+      half[b] = s;
     }
-  double V[NA][NB];
+  };
+  auto value = [&](int fb) __attribute__((always_inline)) {
+    double s = 0.0;
 #pragma unroll
-  for (int fa = 0; fa < NA; ++fa)
-#pragma unroll
-    for (int fb = 0; fb < NB; ++fb) {
-      double s = 0.0;
-      if (fb < nfb) {
-#pragma unroll
-        for (int b = 0; b < NB; ++b) s += tb[fb * NB + b] * half[fa][b];
-      }
-      V[fa][fb] = s;
-    }
+    for (int b = 0; b < NB; ++b) s += tb[fb * NB + b] * half[b];
+    return s;
+  };
 
   if (g.metric) {
     // (P|Q): the bra's second shell is the unit function; write both triangles
     const int64_t Q = g.C.foff[sc] + fc;
-#pragma unroll
-    for (int fa = 0; fa < NA; ++fa) {
-      if (fa >= nfa) break;
+#pragma unroll 1
+    for (int fa = 0; fa < nfa; ++fa) {
       if (sc == sa && fa < fc) continue;   // one writer per element of a diagonal block
+      half_row(fa);
+      const double v = value(0);
       const int64_t P = g.A.foff[sa] + fa;
-      g.out[P + Q * g.naux] = V[fa][0];
-      g.out[Q + P * g.naux] = V[fa][0];
+      g.out[P + Q * g.naux] = v;
+      g.out[Q + P * g.naux] = v;
     }
     return;
   }
   const int64_t P = g.C.foff[sc] + fc;
   const bool same = sa == sb && g.A.l == g.B.l;
-#pragma unroll
-  for (int fa = 0; fa < NA; ++fa)
-#pragma unroll
-    for (int fb = 0; fb < NB; ++fb) {
-      if (fa >= nfa || fb >= nfb) continue;
+#pragma unroll 1
+  for (int fa = 0; fa < nfa; ++fa)
+#pragma unroll 1
+    for (int fb = 0; fb < nfb; ++fb) {
       const int mu = g.A.foff[sa] + fa, nu = g.B.foff[sb] + fb;
       const int32_t ip = g.pairmap[(int64_t)mu * g.nbf + nu];
       if (ip < 0) continue;
-      double v = V[fa][fb];
+      half_row(fa);
+      double v = value(fb);
       if (same) {
-        if (NA == NB) v = 0.5 * (V[fa][fb] + V[fb < NA ? fb : 0][fa < NB ? fa : 0]);
+        if constexpr (NA == NB) {
+          half_row(fb);
+          v = 0.5 * (v + value(fa));
+        }
         if (mu == nu) v *= 0.5;   // diagonal pairs stored x1/2
       }
       g.out[ip + P * g.npair] = v;
