@@ -1866,15 +1866,21 @@ int boys_table(mgw_ctx* c, const double** out) {
   return MGW_OK;
 }
 
-// ket functions (shell, function) grouped by angular momentum: kfun holds
-// them class by class; first[l] .. first[l + 1] is class l
-void ket_functions(const mgw_shells* sh, std::vector<int32_t>& kfun, std::vector<int>& first) {
+// ket shells and ket functions (shell, function) grouped by angular momentum:
+// kshell and kfun hold them class by class; sfirst[l] .. sfirst[l + 1] and
+// first[l] .. first[l + 1] are class l
+void ket_functions(const mgw_shells* sh, std::vector<int32_t>& kshell, std::vector<int>& sfirst,
+                   std::vector<int32_t>& kfun, std::vector<int>& first) {
   first.assign(8, 0);
+  sfirst.assign(8, 0);
   kfun.clear();
+  kshell.clear();
   for (int l = 0; l <= 6; ++l) {
     first[l] = (int)kfun.size() / 2;
+    sfirst[l] = (int)kshell.size();
     for (int k = 0; k < sh->nshell; ++k) {
       if (sh->am[k] != l) continue;
+      kshell.push_back(k);
       const int nf = sh->function_offset[k + 1] - sh->function_offset[k];
       for (int f = 0; f < nf; ++f) {
         kfun.push_back(k);
@@ -1883,6 +1889,7 @@ void ket_functions(const mgw_shells* sh, std::vector<int32_t>& kfun, std::vector
     }
   }
   first[7] = (int)kfun.size() / 2;
+  sfirst[7] = (int)kshell.size();
 }
 
 }  // namespace
@@ -1910,9 +1917,9 @@ int mgw_eri_2center_ao(mgw_ctx* c, const mgw_shells* auxil, int where, double* e
   EriShells U;
   int nunit = 0;
   MGW_TRY(upload_shells(c, "int_unit", &unit, U, nunit));
-  std::vector<int32_t> kfun;
-  std::vector<int> first;
-  ket_functions(auxil, kfun, first);
+  std::vector<int32_t> kfun, kshell;
+  std::vector<int> first, sfirst;
+  ket_functions(auxil, kshell, sfirst, kfun, first);
   // bra pairs (P shell, its unit shell) grouped by l_P, in the same order
   std::vector<int32_t> kshell_pairs;
   std::vector<int> pfirst(8, 0);
@@ -1925,8 +1932,8 @@ int mgw_eri_2center_ao(mgw_ctx* c, const mgw_shells* auxil, int where, double* e
       }
   }
   pfirst[7] = (int)kshell_pairs.size() / 2;
-  int32_t *kf_d, *pr_d;
-  MGW_TRY(upload(c, "int_kfun", kfun.data(), kfun.size(), &kf_d));
+  int32_t *kf_d, *ks_d, *pr_d;
+  MGW_TRY(upload_group(c, "int_kfun", {part_of(kfun.data(), kfun.size(), &kf_d), part_of(kshell.data(), kshell.size(), &ks_d)}));
   MGW_TRY(upload(c, "int_pairs", kshell_pairs.data(), kshell_pairs.size(), &pr_d));
   const double* boys = nullptr;
   MGW_TRY(boys_table(c, &boys));
@@ -1941,6 +1948,8 @@ int mgw_eri_2center_ao(mgw_ctx* c, const mgw_shells* auxil, int where, double* e
       e.npairs = pfirst[la + 1] - pfirst[la];
       e.kfun = kf_d + 2 * (int64_t)first[lc];
       e.nkfun = first[lc + 1] - first[lc];
+      e.kshell = ks_d + sfirst[lc];
+      e.nkshell = sfirst[lc + 1] - sfirst[lc];
       e.boys = boys;
       e.metric = 1;
       e.naux = naux;
@@ -2003,13 +2012,13 @@ int mgw_eri_3center_ao(mgw_ctx* c, const mgw_shells* basis, const mgw_shells* au
     pairs.insert(pairs.end(), cls[k].begin(), cls[k].end());
   }
   cfirst[64] = (int64_t)pairs.size() / 2;
-  std::vector<int32_t> kfun;
-  std::vector<int> first;
-  ket_functions(auxil, kfun, first);
-  int32_t *pm_d, *pr_d, *kf_d;
+  std::vector<int32_t> kfun, kshell;
+  std::vector<int> first, sfirst;
+  ket_functions(auxil, kshell, sfirst, kfun, first);
+  int32_t *pm_d, *pr_d, *kf_d, *ks_d;
   MGW_TRY(upload(c, "int_pairmap", pmap.data(), pmap.size(), &pm_d));
   MGW_TRY(upload(c, "int_pairs", pairs.data(), pairs.size(), &pr_d));
-  MGW_TRY(upload(c, "int_kfun", kfun.data(), kfun.size(), &kf_d));
+  MGW_TRY(upload_group(c, "int_kfun", {part_of(kfun.data(), kfun.size(), &kf_d), part_of(kshell.data(), kshell.size(), &ks_d)}));
   const double* boys = nullptr;
   MGW_TRY(boys_table(c, &boys));
   double* out = eri_3center_tmp;
@@ -2030,6 +2039,8 @@ int mgw_eri_3center_ao(mgw_ctx* c, const mgw_shells* basis, const mgw_shells* au
           e.npairs = cfirst[l1 * 8 + l2 + 1] - cfirst[l1 * 8 + l2];
           e.kfun = kf_d + 2 * (int64_t)first[lc];
           e.nkfun = first[lc + 1] - first[lc];
+          e.kshell = ks_d + sfirst[lc];
+          e.nkshell = sfirst[lc + 1] - sfirst[lc];
           e.boys = boys;
           e.metric = 0;
           e.pairmap = pm_d;

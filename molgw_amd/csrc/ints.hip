@@ -65,6 +65,8 @@ int launch_eri_class(const EriLaunch& e, hipStream_t s) {
   g.pairs = reinterpret_cast<const int2*>(e.pairs);
   g.kfun = reinterpret_cast<const int2*>(e.kfun);
   g.nkfun = e.nkfun;
+  g.kshell = e.kshell;
+  g.nkshell = e.nkshell;
   g.boys = e.boys;
   g.metric = e.metric;
   g.pairmap = e.pairmap;
@@ -72,9 +74,15 @@ int launch_eri_class(const EriLaunch& e, hipStream_t s) {
   g.npair = e.npair;
   g.naux = e.naux;
   g.out = e.out;
-  MGW_REQUIRE(e.npairs < (1LL << 31) && (e.nkfun + WG - 1) / WG < 65536, MGW_ERR_ARG,
+  // (s s| and (p s|: 16 or 32 ket shells side by side, the rest of the workgroup
+  // slices the primitive pairs (ints_kernel.h has what other widths measured)
+  const bool by_shell = e.la + e.lb <= 1;
+  g.lanes = 16;
+  while (g.lanes < 32 && g.lanes < e.nkshell) g.lanes *= 2;
+  const int per_block = by_shell ? g.lanes : WG, nket = by_shell ? e.nkshell : e.nkfun;
+  MGW_REQUIRE(e.npairs < (1LL << 31) && (nket + per_block - 1) / per_block < 65536, MGW_ERR_ARG,
               "integrals: too many shell pairs or auxiliary functions in one class");
-  const dim3 grid((unsigned)e.npairs, (unsigned)((e.nkfun + WG - 1) / WG));
+  const dim3 grid((unsigned)e.npairs, (unsigned)((nket + per_block - 1) / per_block));
   switch (e.la) {
     case 0: return launch_la0(e.lb, e.lc, grid, g, s);
     case 1: return launch_la1(e.lb, e.lc, grid, g, s);

@@ -275,8 +275,10 @@ struct EriLaunch {
   EriShells A, B, C;
   const int32_t* pairs = nullptr;
   int64_t npairs = 0;
-  const int32_t* kfun = nullptr;
+  const int32_t* kfun = nullptr;     // ket functions (shell, function) of the class
   int nkfun = 0;
+  const int32_t* kshell = nullptr;   // ket shells of the class
+  int nkshell = 0;
   const double* boys = nullptr;
   int metric = 0;
   const int32_t* pairmap = nullptr;

@@ -40,3 +40,21 @@ def test_contracted_kets(lines, bas, ket, gt):
     want = N.eri_2center(ax)
     assert np.max(np.abs(met - want)) < 1e-12 * np.max(np.abs(want))
     np.testing.assert_array_equal(met, met.T)
+
+
+@pytest.mark.parametrize('natom', [1, 2, 16, 17, 32, 33])
+def test_ket_shell_counts(natom):
+    # one d shell an atom in the auxiliary basis: at and beside the 16 and 32
+    # lanes of ket shells of the (s s| and (p s| kernels
+    m = Molecule.from_lines([f'H {0.9 * k} {0.3 * (k % 3)} {0.2 * (k % 2)}' for k in range(natom)])
+    bs, ax = (BasisSet(m.atoms, m.coords, b, BASIS, 'PURE') for b in ('cc-pVDZ', 'cc-pVDZ-RI'))
+    ib = upper_pairs(bs.nbf)
+    k, l = ib[0] - 1, ib[1] - 1
+    ref = N.eri_3center(bs, ax)[k, l, :].copy()
+    ref[k == l] *= 0.5
+    want = N.eri_2center(ax)
+    with Engine(0) as e:
+        got = e.eri_3center_ao(bs, ax, ib)
+        met = e.eri_2center_ao(ax)
+    assert np.max(np.abs(got - ref)) < 1e-12 * np.max(np.abs(ref))
+    assert np.max(np.abs(met - want)) < 1e-12 * np.max(np.abs(want))
