@@ -378,6 +378,7 @@ constexpr int PL_K = 32;       // k per tile of the plane layout
 constexpr int PL_ROWS = 128;   // rows padded to the product's tile
 typedef float pf4 __attribute__((ext_vector_type(4)));
 typedef _Float16 ph8 __attribute__((ext_vector_type(8)));
+typedef _Float16 ph4 __attribute__((ext_vector_type(4)));
 typedef unsigned int pu4 __attribute__((ext_vector_type(4)));
 
 __device__ inline double plane_scale(double bound) {
@@ -464,7 +465,7 @@ struct PlaneGemmArgs {
 // (M == N), entries with m < n not written. Tiles of one matrix before the
 // next.
 template <bool LOWER, int BM, int KLASS>
-__global__ void __launch_bounds__(256, 2)
+__global__ void __launch_bounds__(256, 3)
 plane_gemm_kernel(PlaneGemmArgs g) {
   constexpr int WM = 2, WN = 2, NT = 256;
   static_assert(BM == 64 || BM == 128, "tile");
@@ -570,38 +571,73 @@ plane_gemm_kernel(PlaneGemmArgs g) {
     for (int i = 0; i < FM; ++i) {
       const int m = m0 + wm * TM + i * 16 + fr;
 #pragma unroll
-      for (int j = 0; j < FN; ++j)
+      for (int j = 0; j < FN; ++j) {
+        const int nb = n0 + wn * TN + j * 16 + 4 * fq;
+        ph4 hi, lo;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const int n = n0 + wn * TN + j * 16 + 4 * fq + r;
-          const int orow = g.op_trans ? n : m, ok = g.op_trans ? m : n;
-          if (orow >= g.op_rpad || ok >= okmax) continue;
-          const double v = (m < g.M && n < g.N) ? g.alpha * ((double)part[i][j][r] * unscale) : 0.0;
+          const double v = (m < g.M && nb + r < g.N) ? g.alpha * ((double)part[i][j][r] * unscale) : 0.0;
           const float y = (float)(v * so);
-          const _Float16 h = (_Float16)y;
-          const int64_t idx = ((int64_t)(ok / PL_K) * g.op_rpad + orow) * PL_K + (ok % PL_K);
-          O[idx] = h;
-          O[idx + g.op_q] = (_Float16)(y - (float)h);
+          hi[r] = (_Float16)y;
+          lo[r] = (_Float16)(y - (float)hi[r]);
         }
+        if (!g.op_trans) {
+          // a lane's four columns are neighbours along k: one 8-byte store a plane
+          if (m >= g.op_rpad || nb >= okmax) continue;
+          const int64_t idx = ((int64_t)(nb / PL_K) * g.op_rpad + m) * PL_K + (nb % PL_K);
+          *reinterpret_cast<ph4*>(O + idx) = hi;
+          *reinterpret_cast<ph4*>(O + idx + g.op_q) = lo;
+        } else {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            if (nb + r >= g.op_rpad || m >= okmax) continue;
+            const int64_t idx = ((int64_t)(m / PL_K) * g.op_rpad + nb + r) * PL_K + (m % PL_K);
+            O[idx] = hi[r];
+            O[idx + g.op_q] = lo[r];
+          }
+        }
+      }
     }
     return;
   }
+  // whole tiles load what they add to without a bounds check around each
+  // element, sixteen at a time (above the diagonal too, where they write
+  // nothing); with a check the loads come one by one. 2688 rows, 32 frequencies:
+  // the updates of all levels 2.63 -> 2.25 ms
   double* __restrict__ C = g.C + (int64_t)f * g.strideC;
+  const bool whole = m0 + BM <= g.M && n0 + BM <= g.N;
 #pragma unroll
-  for (int i = 0; i < FM; ++i) {
-    const int m = m0 + wm * TM + i * 16 + fr;
+  for (int j = 0; j < FN; ++j) {
+    double* __restrict__ col[4];
 #pragma unroll
-    for (int j = 0; j < FN; ++j)
+    for (int r = 0; r < 4; ++r)
+      col[r] = C + (m0 + wm * TM + fr) + (int64_t)(n0 + wn * TN + j * 16 + 4 * fq + r) * g.ldc;
+    if (whole) {
+      double v[4][FM];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int n = n0 + wn * TN + j * 16 + 4 * fq + r;
-        if (m >= g.M || n >= g.N) continue;
-        if (LOWER && m < n) continue;
-        const int64_t idx = m + (int64_t)n * g.ldc;
-        double v = g.alpha * ((double)part[i][j][r] * unscale);
-        if (g.beta != 0.0) v += g.beta * C[idx];
-        C[idx] = v;
-      }
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int i = 0; i < FM; ++i) v[r][i] = g.beta != 0.0 ? col[r][16 * i] : 0.0;
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int i = 0; i < FM; ++i) {
+          if (LOWER && m0 + wm * TM + i * 16 + fr < n0 + wn * TN + j * 16 + 4 * fq + r) continue;
+          const double t = g.alpha * ((double)part[i][j][r] * unscale);
+          col[r][16 * i] = g.beta != 0.0 ? t + g.beta * v[r][i] : t;
+        }
+    } else {
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int i = 0; i < FM; ++i) {
+          const int m = m0 + wm * TM + i * 16 + fr, n = n0 + wn * TN + j * 16 + 4 * fq + r;
+          if (m >= g.M || n >= g.N || (LOWER && m < n)) continue;
+          double t = g.alpha * ((double)part[i][j][r] * unscale);
+          if (g.beta != 0.0) t += g.beta * col[r][16 * i];
+          col[r][16 * i] = t;
+        }
+    }
   }
 }
 

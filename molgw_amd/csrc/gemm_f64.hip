@@ -374,18 +374,26 @@ gemm_f64_kernel(GemmDev g) {
     const double* __restrict__ W = g.dot_w ? g.dot_w + (int64_t)batch * g.strideDotW : nullptr;
 #pragma unroll
     for (int j = 0; j < FN; ++j) {
+      // the loads of a column group go out together: no bounds check around
+      // each, but indices held to the last row and column
+      double dv[4][FM], wv[FM];
+#pragma unroll
+      for (int i = 0; i < FM; ++i) {
+        const int m = min(m0 + wm * TM + i * 16 + fr, g.M - 1);
+        wv[i] = W ? W[m] : 1.0;
+        if (D) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) dv[r][i] = D[m + (int64_t)min(n0 + wn * TN + j * 16 + fk + 4 * r, g.N - 1) * g.lddot];
+        }
+      }
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int nl = wn * TN + j * 16 + fk + 4 * r;
-        const int n = n0 + nl;
         double part = 0.0;
 #pragma unroll
         for (int i = 0; i < FM; ++i) {
-          const int m = m0 + wm * TM + i * 16 + fr;
-          if (m < g.M && n < g.N) {
-            const double c = g.alpha * acc[i][j][r];
-            part += D ? c * (g.dot_cc * c + g.dot_cd * D[m + (int64_t)n * g.lddot]) : (W ? W[m] : 1.0) * c * c;
-          }
+          const double c = g.alpha * acc[i][j][r];
+          if (m0 + wm * TM + i * 16 + fr < g.M) part += D ? c * (g.dot_cc * c + g.dot_cd * dv[r][i]) : wv[i] * c * c;
         }
         part += __shfl_xor(part, 8, 16);
         part += __shfl_xor(part, 4, 16);
