@@ -884,32 +884,68 @@ int launch_dot_reduce(const double* part, int nrb, int64_t ncol, int nomega, con
 
 // sigma_calc(kc, m) = - sum_iw weight_iw / (2 pi) sum_p
 //     [1/((wc - e_p) + i w) + 1/((wc - e_p) - i w)] v(p, m, iw)
-// (src/m_gw_selfenergy_grid.f90:306-317). One workgroup per (kc, m).
-__global__ void sigma_imag_sum_kernel(const double* __restrict__ v, int np, int nse, int nomega,
-                                      const double* __restrict__ omega, const double* __restrict__ weight,
-                                      const double* __restrict__ ep, const double* __restrict__ wc,
-                                      int ncalc, double* __restrict__ sigma_calc) {
+// (src/m_gw_selfenergy_grid.f90:306-317). One workgroup per (kc, m), a thread per
+// state p. Up to 128 states leave threads over, which form the terms of further
+// frequencies; the sums keep the order of one frequency at a time (the Pade
+// continuation carries a change of the last bit to the tenth digit), so the
+// result does not depend on which of the two ways is taken. Memory latencies and
+// divisions in a row bound it: 41 states, 16 frequencies 15.1 -> 9 us (394
+// states 27 us).
+__global__ void __launch_bounds__(256)
+sigma_imag_sum_kernel(const double* __restrict__ v, int np, int nse, int nomega,
+                      const double* __restrict__ omega, const double* __restrict__ weight,
+                      const double* __restrict__ ep, const double* __restrict__ wc,
+                      int ncalc, double* __restrict__ sigma_calc) {
   __shared__ double red[4][2];
-  const int kc = blockIdx.x, m = blockIdx.y;
+  __shared__ double term[2][256];
+  const int kc = blockIdx.x, m = blockIdx.y, tid = threadIdx.x;
   const double wr = wc[2 * kc], wi = wc[2 * kc + 1];
   double sr = 0.0, si = 0.0;
-  for (int iw = 0; iw < nomega; ++iw) {
-    const double w = omega[iw];
-    const double c = -weight[iw] / (2.0 * 3.14159265358979323);
-    const double* vv = v + (int64_t)np * m + (int64_t)np * nse * iw;
-    double ar = 0.0, ai = 0.0;
-    for (int p = threadIdx.x; p < np; p += blockDim.x) {
-      const double dr = wr - ep[p];
-      // 1/(dr + i(wi + w)) + 1/(dr + i(wi - w))
-      const double i1 = wi + w, i2 = wi - w;
-      const double d1 = dr * dr + i1 * i1, d2 = dr * dr + i2 * i2;
-      const double gr = dr / d1 + dr / d2;
-      const double gi = -i1 / d1 - i2 / d2;
-      ar += gr * vv[p];
-      ai += gi * vv[p];
+  auto add = [&](int p, int iw, double& ar, double& ai) __attribute__((always_inline)) {
+    const double w = omega[iw], vv = v[(int64_t)np * (m + (int64_t)nse * iw) + p];
+    const double dr = wr - ep[p];
+    // 1/(dr + i(wi + w)) + 1/(dr + i(wi - w))
+    const double i1 = wi + w, i2 = wi - w;
+    const double d1 = dr * dr + i1 * i1, d2 = dr * dr + i2 * i2;
+    const double gr = dr / d1 + dr / d2;
+    const double gi = -i1 / d1 - i2 / d2;
+    ar = fma(gr, vv, ar);
+    ai = fma(gi, vv, ai);
+  };
+  auto coef = [&](int iw) { return -weight[iw] / (2.0 * 3.14159265358979323); };
+  if (np <= 128) {
+    const int nf = 256 / np, p = tid % np, g = tid / np;
+    for (int iw = 0; iw < nomega; iw += nf) {
+      double ar = 0.0, ai = 0.0;
+      if (g < nf && iw + g < nomega) add(p, iw + g, ar, ai);
+      term[0][tid] = ar;
+      term[1][tid] = ai;
+      __syncthreads();
+      if (tid < np)
+        for (int j = 0; j < nf && iw + j < nomega; ++j) {
+          const double c = coef(iw + j);
+          sr = fma(c, term[0][j * np + tid], sr);
+          si = fma(c, term[1][j * np + tid], si);
+        }
+      __syncthreads();
     }
-    sr += c * ar;
-    si += c * ai;
+  } else {
+    constexpr int U = 8;          // frequencies whose terms are formed together
+    for (int iw = 0; iw < nomega; iw += U) {
+      double ar[U], ai[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) ar[u] = ai[u] = 0.0;
+      for (int p = tid; p < np; p += 256)
+#pragma unroll
+        for (int u = 0; u < U; ++u) add(p, min(iw + u, nomega - 1), ar[u], ai[u]);
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (iw + u < nomega) {
+          const double c = coef(iw + u);
+          sr = fma(c, ar[u], sr);
+          si = fma(c, ai[u], si);
+        }
+    }
   }
   for (int o = 32; o > 0; o >>= 1) { sr += __shfl_xor(sr, o, 64); si += __shfl_xor(si, o, 64); }
   if ((threadIdx.x & 63) == 0) { red[threadIdx.x >> 6][0] = sr; red[threadIdx.x >> 6][1] = si; }
@@ -1064,39 +1100,58 @@ int launch_pade(const double* wc, const double* sc, int ncalc, int nse, const do
 
 // ------------------------------------------------------------------ QP equation
 // Graphical solution (src/m_selfenergy_tools.f90:253-420) and linearisation
-// (:202-249) per state p of [nsemin, nsemax]. One thread per state.
-__global__ void qp_kernel(const double* __restrict__ sigma, int nomega, int nse,
-                          const double* __restrict__ omega, const double* __restrict__ se_e0,
-                          const double* __restrict__ exc, const double* __restrict__ e0,
-                          double* __restrict__ eqp, double* __restrict__ zz,
-                          double* __restrict__ elin) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= nse) return;
+// (:202-249) per state p of [nsemin, nsemax]. One wave per state, a lane per
+// interval of the frequency grid; the few lanes whose interval holds a crossing
+// are then taken in order. One thread per state waited for 51 frequencies' loads
+// in turn: 17.8 -> 3.6 us.
+__global__ void __launch_bounds__(64)
+qp_kernel(const double* __restrict__ sigma, int nomega, int nse,
+          const double* __restrict__ omega, const double* __restrict__ se_e0,
+          const double* __restrict__ exc, const double* __restrict__ e0,
+          double* __restrict__ eqp, double* __restrict__ zz,
+          double* __restrict__ elin) {
+  const int p = blockIdx.x, lane = threadIdx.x;
   constexpr int NFP = 4;
   double zw[NFP], ef[NFP];
   for (int j = 0; j < NFP; ++j) { zw[j] = -1.0; ef[j] = 0.0; }
   const double* sg = sigma + 2 * (int64_t)p * nomega;
   const double c = exc[p] + e0[p];
-  double xprev = omega[0] + se_e0[p];
-  double fprev = sg[0] + c;
-  double gprev = fprev - xprev;
-  for (int ix = 1; ix < nomega; ++ix) {
-    const double x = omega[ix] + se_e0[p];
-    const double f = sg[2 * ix] + c;
-    const double gx = f - x;
-    if (gprev * gx < 0.0) {
-      const double z0 = 1.0 / (1.0 - (f - fprev) / (x - xprev));
-      if (z0 >= 0.00001 && z0 > zw[NFP - 1]) {
-        int jf = 0;
-        while (!(z0 > zw[jf])) ++jf;
-        for (int j = NFP - 1; j > jf; --j) { zw[j] = zw[j - 1]; ef[j] = ef[j - 1]; }
-        zw[jf] = z0;
+  for (int base = 1; base < nomega; base += 64) {
+    const int ix = base + lane;
+    double z0 = -1.0, root = 0.0;
+    bool cross = false;
+    if (ix < nomega) {
+      const double xprev = omega[ix - 1] + se_e0[p], x = omega[ix] + se_e0[p];
+      const double fprev = sg[2 * (ix - 1)] + c, f = sg[2 * ix] + c;
+      const double gprev = fprev - xprev, gx = f - x;
+      if (gprev * gx < 0.0) {
+        z0 = 1.0 / (1.0 - (f - fprev) / (x - xprev));
+        cross = z0 >= 0.00001;
         const double gp = (gx - gprev) / (x - xprev);
-        ef[jf] = xprev - gprev / gp;
+        root = xprev - gprev / gp;
       }
     }
-    xprev = x; fprev = f; gprev = gx;
+    for (unsigned long long todo = __ballot(cross); todo; todo &= todo - 1) {
+      const int src = __ffsll(todo) - 1;
+      const double zc = __shfl(z0, src, 64), rc = __shfl(root, src, 64);
+      if (!(zc > zw[NFP - 1])) continue;
+      // before the first entry that it exceeds
+      bool placed = false;
+      double zi = zc, ri = rc;
+#pragma unroll
+      for (int j = 0; j < NFP; ++j) {
+        if (placed || zi > zw[j]) {
+          placed = true;
+          const double zt = zw[j], rt = ef[j];
+          zw[j] = zi;
+          ef[j] = ri;
+          zi = zt;
+          ri = rt;
+        }
+      }
+    }
   }
+  if (lane != 0) return;
   const int n0 = nomega / 2;
   double e, z;
   double zmax = zw[0];
@@ -1122,7 +1177,7 @@ __global__ void qp_kernel(const double* __restrict__ sigma, int nomega, int nse,
 int launch_qp(const double* sigma, int nomega, int nse, const double* omega, const double* se_e0,
               const double* exc, const double* e0, double* eqp, double* zz, double* elin,
               hipStream_t s) {
-  hipLaunchKernelGGL(qp_kernel, dim3(nblocks(nse, 64)), dim3(64), 0, s, sigma, nomega, nse, omega,
+  hipLaunchKernelGGL(qp_kernel, dim3(nse), dim3(64), 0, s, sigma, nomega, nse, omega,
                      se_e0, exc, e0, eqp, zz, elin);
   MGW_LAUNCH_CHECK();
   return MGW_OK;
