@@ -538,7 +538,6 @@ int ao2mo(mgw_ctx* c, int mlo, int mhi, int nlo, int nhi, double* out, int preci
       MGW_TRY(dbuf(c, "ao2mo_max", 2, &mx));
       MGW_TRY(dbuf(c, "ao2mo_maxpart", ABSMAX_BLOCKS, &part));
       MGW_TRY(launch_absmax_scalar(C, (int64_t)nbf * c->nstate, part, mx, c->stream));
-      MGW_TRY(launch_fill(mx + 1, 1, 0.0, c->stream));
     }
     MGW_TRY(ao2mo_first(c, B, C, flo, nf1, H, precision, f16, mx, half != nullptr));
     if (!half) {
@@ -844,7 +843,6 @@ int polarizability_grid(mgw_ctx* c, const mgw_ranges* r, double spin_fact, int n
   MGW_TRY(upload_group(c, "chi_in", {part_of(ia.data(), ia.size(), &ia_d), part_of(omega_im, (size_t)nomega, &om_d)}));
   MGW_TRY(dbuf(c, "chi_sw", (size_t)npole * nomega, &sw));
   MGW_TRY(dbuf(c, "cas_n2", npole, &n2));
-  MGW_TRY(dbuf(c, "ones", naux, &ones));
   // what the host needs of the factorisation, in one piece: the trace of chi0,
   // ln det, the partial sums of ||L^-1||^2 and the flags of every frequency
   const size_t nres = (size_t)nomega * (2 + FROB_BLOCKS) + (nomega + 1) / 2;
@@ -854,7 +852,6 @@ int polarizability_grid(mgw_ctx* c, const mgw_ranges* r, double spin_fact, int n
   int32_t* const info_d = reinterpret_cast<int32_t*>(frob + (size_t)FROB_BLOCKS * nomega);
   // 1 - chi0, then its inverse Cholesky factor, resident for the self-energy
   MGW_TRY(dbuf(c, "wpol_linv", (size_t)naux * naux * nomega, &chi));
-  MGW_TRY(launch_fill(ones, naux, 1.0, c->stream));
   MGW_TRY(launch_chi_weights(ia_d, npole, find_buf(c, "energy"), find_buf(c, "occupation"), om_d,
                              nomega, sw, c->stream));
   MGW_TRY(launch_colnorm2(x, naux, naux, npole, n2, c->stream));
@@ -866,7 +863,14 @@ int polarizability_grid(mgw_ctx* c, const mgw_ranges* r, double spin_fact, int n
   g.B = x; g.ldb = naux; g.transB = true; g.strideB = 0;
   g.C = chi; g.ldc = naux; g.strideC = (int64_t)naux * naux;
   g.kscale = sw; g.strideK = npole;
-  g.diag_add = ones; g.strideDiag = 0;
+  g.strideDiag = 0;
+  auto plus_one = [&]() -> int {     // the product's 1, which the split path adds by itself
+    if (g.diag_add) return MGW_OK;
+    MGW_TRY(dbuf(c, "ones", naux, &ones));
+    MGW_TRY(launch_fill(ones, naux, 1.0, c->stream));
+    g.diag_add = ones;
+    return MGW_OK;
+  };
   g.batch = nomega;
   g.lower_only = true;
   g.upper_zero = true;   // the Cholesky wants the strict upper triangle zero
@@ -896,6 +900,7 @@ int polarizability_grid(mgw_ctx* c, const mgw_ranges* r, double spin_fact, int n
         if (g.splits > 1)
           MGW_TRY(dbuf(c, "chi_ksplit", gemm_f64_split_doubles(naux, naux, nomega, g.splits), &g.split_work));
       }
+      MGW_TRY(plus_one());
       MGW_TRY(gemm_f64(g, c->stream));
     }
   }
@@ -923,8 +928,7 @@ int polarizability_grid(mgw_ctx* c, const mgw_ranges* r, double spin_fact, int n
   if (planes) MGW_TRY(scratch_done(c, "chol_planes"));
   // D = L^-1 - 1 stays resident: chi = L^-T L^-1 - 1 = D^T D + D + D^T, and
   // the self-energy product works on the screening part D alone
-  MGW_TRY(launch_lower_frob2(chi, naux, nomega, frob, c->stream));
-  MGW_TRY(launch_diag_add(chi, naux, nomega, -1.0, c->stream));
+  MGW_TRY(launch_lower_frob2(chi, naux, nomega, -1.0, frob, c->stream));
   std::vector<double> hres(nres);
   MGW_TRY(download(c, hres.data(), res, nres));
   const int32_t* info = reinterpret_cast<const int32_t*>(hres.data() + (size_t)(2 + FROB_BLOCKS) * nomega);
@@ -945,6 +949,7 @@ int polarizability_grid(mgw_ctx* c, const mgw_ranges* r, double spin_fact, int n
     }
     // a reduced-precision 1 - chi0 that is not positive definite: rebuild
     // this frequency in FP64 and factor it again
+    MGW_TRY(plus_one());
     GemmF64 g1 = g;
     g1.precision = MGW_FP64;
     g1.batch = 1;
@@ -957,8 +962,7 @@ int polarizability_grid(mgw_ctx* c, const mgw_ranges* r, double spin_fact, int n
     MGW_REQUIRE(one == 0, MGW_ERR_SOLVER,
                 "Cholesky of the FP64 rebuild of 1-chi0 failed at frequency " + std::to_string(k) + " (column " +
                     std::to_string(one) + "; reduced-precision column " + std::to_string(info[k]) + ")");
-    MGW_TRY(launch_lower_frob2(g1.C, naux, 1, frob + (size_t)FROB_BLOCKS * k, c->stream));
-    MGW_TRY(launch_diag_add(g1.C, naux, 1, -1.0, c->stream));
+    MGW_TRY(launch_lower_frob2(g1.C, naux, 1, -1.0, frob + (size_t)FROB_BLOCKS * k, c->stream));
     ++c->escalations;
     rebuilt = true;
   }

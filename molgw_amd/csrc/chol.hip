@@ -643,17 +643,18 @@ plane_gemm_kernel(PlaneGemmArgs g) {
 
 // ---------------------------------------------------------------- traces
 // partial[f][b] = sum over columns j = b, b + FROB_BLOCKS, ... of
-// sum_{i >= j} m_f(i, j)^2.
+// sum_{i >= j} m_f(i, j)^2; diag_add is added to the diagonal behind its read.
 __global__ void __launch_bounds__(256)
-lower_frob2_kernel(const double* __restrict__ m, int n, double* __restrict__ partial) {
+lower_frob2_kernel(double* __restrict__ m, int n, double diag_add, double* __restrict__ partial) {
   __shared__ double red[4];
   const int b = blockIdx.x, f = blockIdx.y;
-  const double* __restrict__ a = m + (int64_t)f * n * n;
+  double* __restrict__ a = m + (int64_t)f * n * n;
   double s = 0.0;
   for (int j = b; j < n; j += FROB_BLOCKS)
     for (int i = j + threadIdx.x; i < n; i += 256) {
       const double v = a[i + (int64_t)j * n];
       s += v * v;
+      if (i == j) a[i + (int64_t)j * n] = v + diag_add;
     }
   for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
@@ -982,13 +983,21 @@ bool chol_epi_planes() {
   return e ? std::atoi(e) != 0 : true;
 }
 
+// Does the recursion on a block of size m reach a level in FP16x3 (chol_rec's
+// rule)? Without one its operand bounds are not needed.
+static bool chol_lowp_levels(int m, int f16_min) {
+  if (m <= (chol_leaf_block() ? LEAF : NB)) return false;
+  const int m1 = chol_split(m), m2 = m - m1;
+  return std::min(m1, m2) >= f16_min || chol_lowp_levels(m1, f16_min) || chol_lowp_levels(m2, f16_min);
+}
+
 int chol_inverse_batched(double* A, int n, int nbatch, double* logdet, int32_t* info, double* work,
                          hipStream_t stream, double* bounds, void* planes) {
   if (n <= 0 || nbatch <= 0) return MGW_OK;
   MGW_REQUIRE(nbatch <= 65535, MGW_ERR_ARG, "chol_inverse_batched: batch too large");
   MGW_REQUIRE(!bounds || planes || n <= NB, MGW_ERR_ARG, "chol_inverse_batched: FP16x3 products need planes");
   const int f16_min = bounds ? chol_f16_min() : 0;
-  if (bounds && f16_min > 0) {
+  if (bounds && f16_min > 0 && chol_lowp_levels(n, f16_min)) {
     hipLaunchKernelGGL(chol_diagmax_kernel, dim3(nbatch), dim3(256), 0, stream, A, n, (int64_t)n * n, bounds + 4);
     hipLaunchKernelGGL(chol_bounds_kernel, dim3(1), dim3(256), 0, stream, bounds + 4, nbatch, bounds);
     MGW_HIP(hipGetLastError());
@@ -1002,8 +1011,8 @@ int chol_inverse_batched(double* A, int n, int nbatch, double* logdet, int32_t* 
   return chol_rec(c, 0, n, work, 0);
 }
 
-int launch_lower_frob2(const double* m, int n, int nbatch, double* partial, hipStream_t s) {
-  hipLaunchKernelGGL(lower_frob2_kernel, dim3(FROB_BLOCKS, nbatch), dim3(256), 0, s, m, n, partial);
+int launch_lower_frob2(double* m, int n, int nbatch, double diag_add, double* partial, hipStream_t s) {
+  hipLaunchKernelGGL(lower_frob2_kernel, dim3(FROB_BLOCKS, nbatch), dim3(256), 0, s, m, n, diag_add, partial);
   MGW_HIP(hipGetLastError());
   return MGW_OK;
 }

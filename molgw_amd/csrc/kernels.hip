@@ -324,7 +324,8 @@ int launch_absmax(const double* x, int64_t n, double* part, hipStream_t s) {
   return MGW_OK;
 }
 
-// out[0] = max of the ABSMAX_BLOCKS partial maxima
+// out[0] = max of the ABSMAX_BLOCKS partial maxima, out[1] = 0 (where the caller
+// collects the maximum of a product)
 __global__ void __launch_bounds__(256) absmax_finish_kernel(const double* __restrict__ part, double* __restrict__ out) {
   __shared__ double red[256];
   const int tid = threadIdx.x;
@@ -336,7 +337,10 @@ __global__ void __launch_bounds__(256) absmax_finish_kernel(const double* __rest
     if (tid < w) red[tid] = fmax(red[tid], red[tid + w]);
     __syncthreads();
   }
-  if (tid == 0) out[0] = red[0];
+  if (tid == 0) {
+    out[0] = red[0];
+    out[1] = 0.0;
+  }
 }
 
 int launch_absmax_scalar(const double* x, int64_t n, double* part, double* out, hipStream_t s) {

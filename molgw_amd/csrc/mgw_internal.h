@@ -230,7 +230,7 @@ bool chol_epi_planes();
 int chol_inverse_batched(double* A, int n, int nbatch, double* logdet, int32_t* info, double* work,
                          hipStream_t stream, double* bounds = nullptr, void* planes = nullptr);
 // tr[f] = sum of squares of the lower triangle of M_f (n x n, stride n^2).
-int launch_lower_frob2(const double* m, int n, int nbatch, double* partial, hipStream_t s);
+int launch_lower_frob2(double* m, int n, int nbatch, double diag_add, double* partial, hipStream_t s);
 constexpr int FROB_BLOCKS = 64;
 int gemm_autotune_mode(int mode); // -1 query; returns the previous mode
 // The same tuner for the split-operand kernel families: launch(c) runs
