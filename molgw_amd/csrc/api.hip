@@ -895,7 +895,7 @@ int polarizability_grid(mgw_ctx* c, const mgw_ranges* r, double spin_fact, int n
     } else {
       if (g.precision == MGW_FP64) {
         // K split where the tiles' last round would leave the GPU mostly idle
-        // (naux 1372, 21385 transitions, 32 frequencies: 26.1 -> 24.4 ms)
+        // (naux 1372, 21385 transitions, 32 frequencies: 30.7 -> 26.5 ms)
         g.splits = gemm_f64_splits(naux, naux, npole, nomega, true);
         if (g.splits > 1)
           MGW_TRY(dbuf(c, "chi_ksplit", gemm_f64_split_doubles(naux, naux, nomega, g.splits), &g.split_work));
