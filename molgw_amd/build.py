@@ -25,8 +25,8 @@ SOURCES = ['gemm_f64.hip', 'gemm_lowp.hip', 'chi0_split.hip', 'wb_split.hip', 'c
            'ints_l3_lb3.hip', 'ints_l4.hip']
 
 # compile time in seconds, measured here (to start the slow ones first)
-SLOW = {'ints_l3_lb3.hip': 200, 'ints_l3_lb2.hip': 90, 'ints_l2.hip': 60, 'ints_l3.hip': 50, 'ints_l4.hip': 40,
-        'api.hip': 40, 'chi0_split.hip': 30}
+SLOW = {'ints_l3_lb3.hip': 126, 'gemm_f64.hip': 100, 'ints_l3_lb2.hip': 67, 'ints_l2.hip': 66, 'ints_l3.hip': 53,
+        'ints_l1.hip': 50, 'ints_l4.hip': 34, 'chi0_split.hip': 30, 'chol.hip': 18, 'gemm_lowp.hip': 17}
 
 CFLAGS = [
     f'--offload-arch={ARCH}', '-O3', '-std=c++17', '-fPIC', '-Wall', '-Wno-unused-result',
@@ -57,7 +57,7 @@ def build(verbose: bool = False) -> str:
         obj = os.path.join(BUILD, src.replace('.hip', '.o'))
         objs.append(obj)
         cmds.append([HIPCC, *CFLAGS, '-c', os.path.join(CSRC, src), '-o', obj])
-    # the integral kernels of l_a = 3 take minutes: start them first
+    # start the slow ones first
     order = sorted(range(len(cmds)), key=lambda k: -SLOW.get(SOURCES[k], 0))
     cmds = [cmds[k] for k in order]
     with ThreadPoolExecutor(max_workers=min(len(cmds), max(4, min(8, os.cpu_count() or 4)))) as ex:
