@@ -96,6 +96,7 @@ struct mgw_ctx {
   Ledger ledger;
   Profiler prof;
   bool trim_eagerly = false;
+  bool spare_in_use = false;   // a spare workspace is between its allocation and its product's launch
   // pinned host memory (STAGE_BYTES) through which small vectors go to and come
   // from the device; used up to stage_used since the last synchronisation of
   // the stream, before which no byte of it is written again
@@ -195,6 +196,25 @@ int check_mo_matches_ri(const mgw_ctx* c) {
 }
 
 // ------------------------------------------------------------------ buffers
+// Workspaces that a call is faster with but does not need (dbuf_if_room): they
+// stay cached like the others, and go first when a buffer finds no room.
+const char* const SPARE_BUFFERS[] = {"chi_ksplit", "hf_ksplit"};
+
+int release(mgw_ctx* c, const std::string& name);
+
+// MGW_ALLOC_LIMIT (bytes, read at every allocation): the most that a context's
+// buffers may take together; unset or 0: what the device has.
+int64_t alloc_limit() {
+  const char* e = std::getenv("MGW_ALLOC_LIMIT");
+  return e ? std::atoll(e) : 0;
+}
+
+hipError_t device_alloc(mgw_ctx* c, size_t bytes, void** out) {
+  const int64_t limit = alloc_limit();
+  if (limit > 0 && c->ledger.current + (int64_t)bytes > limit) return hipErrorOutOfMemory;
+  return hipMallocAsync(out, bytes, c->stream);
+}
+
 int ensure(mgw_ctx* c, const std::string& name, size_t bytes, void** out) {
   DevBuf& b = c->ledger.bufs[name];
   if (bytes == 0) bytes = 8;
@@ -208,7 +228,19 @@ int ensure(mgw_ctx* c, const std::string& name, size_t bytes, void** out) {
       b.ptr = nullptr;
       b.bytes = 0;
     }
-    hipError_t e = hipMallocAsync(&b.ptr, bytes, c->stream);
+    hipError_t e = device_alloc(c, bytes, &b.ptr);
+    if (e == hipErrorOutOfMemory) {
+      // once more without the spare workspaces, the pool's blocks of other
+      // sizes handed back to the device
+      (void)hipGetLastError();
+      for (const char* spare : SPARE_BUFFERS)
+        if (name != spare && !c->spare_in_use) MGW_TRY(release(c, spare));
+      MGW_HIP(hipStreamSynchronize(c->stream));
+      hipMemPool_t pool;
+      MGW_HIP(hipDeviceGetDefaultMemPool(&pool, c->device));
+      MGW_HIP(hipMemPoolTrimTo(pool, 0));
+      e = device_alloc(c, bytes, &b.ptr);
+    }
     if (e != hipSuccess) {
       b.ptr = nullptr;
       set_error("hipMallocAsync(" + name + ", " + std::to_string(bytes) + " bytes): " + hipGetErrorString(e));
@@ -229,6 +261,17 @@ int dbuf(mgw_ctx* c, const std::string& name, size_t count, T** out) {
   MGW_TRY(ensure(c, name, count * sizeof(T), &p));
   *out = static_cast<T*>(p);
   return MGW_OK;
+}
+
+// One of SPARE_BUFFERS, or null where there is no room for it (or none is asked
+// for); in use until spare_done.
+int dbuf_if_room(mgw_ctx* c, const std::string& name, size_t count, double** out) {
+  *out = nullptr;
+  if (!count) return MGW_OK;
+  const int rc = dbuf(c, name, count, out);
+  if (rc == MGW_ERR_NOMEM) return MGW_OK;
+  c->spare_in_use = rc == MGW_OK;
+  return rc;
 }
 
 double* find_buf(mgw_ctx* c, const std::string& name) {
@@ -262,6 +305,11 @@ bool is_resident_input(const std::string& name) {
 // so other contexts sharing the GPU keep running). When the context is set to
 // trim eagerly, they are freed here.
 int scratch_done(mgw_ctx* c, const std::string& name);
+
+int spare_done(mgw_ctx* c, const std::string& name) {
+  c->spare_in_use = false;
+  return scratch_done(c, name);
+}
 
 // End of the use of a list that is short for all but the largest molecules: a
 // free costs the host 10 to 20 us and the next call an allocation, so one of up
@@ -893,19 +941,16 @@ int polarizability_grid(mgw_ctx* c, const mgw_ranges* r, double spin_fact, int n
       MGW_TRY(dbuf(c, "chi_split", (bytes + 7) / 8, &work));
       MGW_TRY(chi0_split_syrk(x, naux, npole, sw, nomega, precision, work, bytes, chi, c->stream));
     } else {
-      if (g.precision == MGW_FP64) {
-        // K split where the tiles' last round would leave the GPU mostly idle
-        // (naux 1372, 21385 transitions, 32 frequencies: 30.7 -> 26.5 ms)
-        g.splits = gemm_f64_splits(naux, naux, npole, nomega, true);
-        if (g.splits > 1)
-          MGW_TRY(dbuf(c, "chi_ksplit", gemm_f64_split_doubles(naux, naux, nomega, g.splits), &g.split_work));
-      }
       MGW_TRY(plus_one());
-      MGW_TRY(gemm_f64(g, c->stream));
+      // K split of the last round's tiles, which would leave the GPU mostly idle
+      // (naux 1372, 21385 transitions, 32 frequencies: 30.7 -> 26.5 ms)
+      if (g.precision == MGW_FP64)
+        MGW_TRY(dbuf_if_room(c, "chi_ksplit", gemm_f64_split_doubles(naux, naux, npole, nomega, true), &g.split_work));
+      const int rc = gemm_f64(g, c->stream);
+      if (g.split_work) MGW_TRY(spare_done(c, "chi_ksplit"));
+      MGW_TRY(rc);
     }
   }
-  if (g.splits > 1) MGW_TRY(scratch_done(c, "chi_ksplit"));
-  g.splits = 1;
   g.split_work = nullptr;
   if (precision != MGW_FP64) MGW_TRY(scratch_done(c, "chi_split"));
   // 1 - chi0 = L L^T for every frequency, then L^-1 in place (chol.hip)
@@ -1578,10 +1623,6 @@ int64_t mgw_footprint_bytes_nse(int nbf, int nauxil, int nstate, int nocc, int n
   } else {
     stage_w = na * nb * no + na * npole + na * na * (int64_t)nomega_chi_imag + npole * nomega_chi_imag +
               (int64_t)mgw::chol_work_doubles((int)na) * nomega_chi_imag + 4 + nomega_chi_imag;
-    if (precision == MGW_FP64)
-      stage_w += (int64_t)mgw::gemm_f64_split_doubles(
-          (int)na, (int)na, nomega_chi_imag,
-          mgw::gemm_f64_splits((int)na, (int)na, (int)npole, std::max(1, nomega_chi_imag), true));
     if (precision == MGW_FP16X3)
       stage_w += (int64_t)((mgw::chol_plane_bytes((int)na, nomega_chi_imag) + 7) / 8);
     if (split_precision(precision))
@@ -2123,8 +2164,7 @@ int mgw_hartree_exchange_ri(mgw_ctx* c, const double* x, int nbf, int nx, double
   // the exchange sums over naux x nx rows into nbf x nbf: few tiles, so the
   // rows are split (nbf 768, naux 2688, nx 160: 30 -> 5.0 ms); gamma and the
   // Hartree matrix read their operands once (17 -> 0.44 and 2.9 -> 1.4 ms)
-  const int splits = gemm_f64_splits(nbf, nbf, naux * nx, 1, true);
-  if (splits > 1) MGW_TRY(dbuf(c, "hf_ksplit", gemm_f64_split_doubles(nbf, nbf, 1, splits), &kwork));
+  MGW_TRY(dbuf_if_room(c, "hf_ksplit", gemm_f64_split_doubles(nbf, nbf, naux * nx, 1, true), &kwork));
   {
     ProfScope ps(&c->prof, MGW_KCLASS_GEMM_OTHER,
                  2.0 * naux * (double)nbf * nbf * nx * 2.0 + 4.0 * naux * (double)nbf * nbf,
@@ -2148,16 +2188,17 @@ int mgw_hartree_exchange_ri(mgw_ctx* c, const double* x, int nbf, int nx, double
     k.C = kv; k.ldc = nbf;
     k.alpha = -1.0;
     k.lower_only = true;
-    k.splits = splits;
     k.split_work = kwork;
-    MGW_TRY(gemm_f64(k, c->stream));
+    const int rc = gemm_f64(k, c->stream);
+    if (kwork) MGW_TRY(spare_done(c, "hf_ksplit"));
+    MGW_TRY(rc);
     MGW_TRY(launch_hartree_gamma(h, xd, naux, nbf, nx, spin_fact, gpart, gam, c->stream));
     MGW_TRY(launch_hartree_j(B, gam, naux, nbf, jv, c->stream));
   }
   if (hartree_ao) MGW_TRY(download(c, hartree_ao, jv, (size_t)nbf * nbf));
   if (exchange_ao) MGW_TRY(download(c, exchange_ao, kv, (size_t)nbf * nbf));
   MGW_TRY(sync(c));
-  for (const char* b : {"hf_x", "hf_gamma", "hf_gpart", "hf_ksplit", "hf_j", "hf_k"}) MGW_TRY(scratch_done(c, b));
+  for (const char* b : {"hf_x", "hf_gamma", "hf_gpart", "hf_j", "hf_k"}) MGW_TRY(scratch_done(c, b));
   MGW_TRY(scratch_done(c, "hf_h"));
   return MGW_OK;
 }

@@ -26,9 +26,11 @@
 //   * A wave whose part of the tile lies past the edge or above the diagonal of
 //     a symmetric update leaves the matrix cores to the others.
 //   * With fewer tiles than the GPU's slots, or a last round of workgroups that
-//     would be mostly empty, the K range is split (gemm_f64_splits): partial
-//     products go to a workspace and gemm_f64_reduce_kernel sums them in a
-//     fixed order and applies the epilogue.
+//     would be mostly empty, the K range of that round's tiles is split
+//     (split_plan): their partial products go to a workspace and
+//     gemm_f64_reduce_kernel sums them in order and applies the epilogue. The
+//     whole rounds before it run as they are, so the workspace holds two
+//     rounds' tiles at most (128 MiB), whatever the product's size.
 //
 // Fragment layout of v_mfma_f64_16x16x4_f64 (checked on gfx950): operand "a"
 // lane l = a[i = l & 15][k = l >> 4], operand "b" lane l = b[k = l >> 4][j = l & 15],
@@ -84,8 +86,11 @@ struct GemmDev {
   int batch_outer;     // walk the tiles of one batch entry before the next
   int tiles_m, tiles_n, batch;
   int64_t nblocks;
-  int splits, kchunk;  // K range per split (a multiple of BK)
-  double* part;        // splits > 1: part[split][batch][n][m], else null
+  // the tiles (over all batch entries) behind the first `whole` take `splits`
+  // workgroups of kchunk (a multiple of BK) along K each
+  int64_t whole, rest;
+  int splits, kchunk;
+  double* part;        // splits > 1: part[tile - whole][split][n - n0][m - m0], else null
   const double* dotB; int64_t lddot;
   double dot_cc, dot_cd;
   double* dotpart; int64_t strideDot;
@@ -104,6 +109,35 @@ __device__ inline void store_result(const GemmDev& g, double* __restrict__ C, co
   if (g.beta != 0.0) v += g.beta * C[idx];
   C[idx] = v;
   if (g.lower_only && m > n && !g.no_mirror) C[n + (int64_t)m * g.ldc] = g.upper_zero ? 0.0 : v;
+}
+
+// First row and column of a tile: square tiles of a symmetric update walk the
+// lower triangle, the others groups of GROUP_M tile rows.
+template <int BM, int BN>
+__device__ inline void tile_origin(const GemmDev& g, int tile, int& m0, int& n0) {
+  int bm, bn;
+  if (g.lower_only && BM == BN) {
+    tri_grouped(tile, g.tiles_m, bm, bn);
+  } else {
+    const int per_group = GROUP_M * g.tiles_n;
+    const int group = tile / per_group;
+    const int first_m = group * GROUP_M;
+    const int gsize = min(g.tiles_m - first_m, GROUP_M);
+    const int in_group = tile - group * per_group;
+    bm = first_m + in_group % gsize;
+    bn = in_group / gsize;
+  }
+  m0 = bm * BM;
+  n0 = bn * BN;
+}
+
+// Tile and batch entry of the u-th tile over all batch entries: batch fastest
+// when the entries share operands (the frequencies of one chi0 tile read the
+// same panels), batch slowest when they do not.
+__device__ inline void tile_of_unit(const GemmDev& g, int64_t u, int& tile, int& batch) {
+  const int64_t per = (g.whole + g.rest) / g.batch;
+  batch = (int)(g.batch_outer ? u / per : u % g.batch);
+  tile = (int)(g.batch_outer ? u % per : u / g.batch);
 }
 
 template <int BM, int BN, int WM, int WN, bool TA, bool TB, bool DOT, int KLASS>
@@ -133,29 +167,15 @@ gemm_f64_kernel(GemmDev g) {
   const int wm = wave % WM;
   const int wn = wave / WM;
 
-  // logical block: batch fastest when the batch entries share operands (the
-  // frequencies of one chi0 tile read the same panels), batch slowest when
-  // they do not; then the K split; then the tile in grouped order
-  const int64_t L = xcd_logical(blockIdx.x, g.nblocks);
-  const int64_t per = g.nblocks / g.batch;
-  const int batch = (int)(g.batch_outer ? L / per : L % g.batch);
-  const int ts = (int)(g.batch_outer ? L % per : L / g.batch);
-  const int split = ts % g.splits;
-  const int tile = ts / g.splits;
-  int bm, bn;
-  if (g.lower_only && BM == BN) {
-    tri_grouped(tile, g.tiles_m, bm, bn);
-  } else {
-    const int per_group = GROUP_M * g.tiles_n;
-    const int group = tile / per_group;
-    const int first_m = group * GROUP_M;
-    const int gsize = min(g.tiles_m - first_m, GROUP_M);
-    const int in_group = tile - group * per_group;
-    bm = first_m + in_group % gsize;
-    bn = in_group / gsize;
-  }
-  const int m0 = bm * BM;
-  const int n0 = bn * BN;
+  // logical block: the whole tiles, then the K splits of the others, one split
+  // of all of them before the next (they share its range of the panels)
+  const bool in_split = blockIdx.x >= g.whole;
+  const int64_t L = in_split ? xcd_logical(blockIdx.x - g.whole, g.nblocks - g.whole) : xcd_logical(blockIdx.x, g.whole);
+  const int split = in_split ? (int)(L / g.rest) : 0;
+  const int64_t unit = in_split ? g.whole + L % g.rest : L;
+  int tile, batch, m0, n0;
+  tile_of_unit(g, unit, tile, batch);
+  tile_origin<BM, BN>(g, tile, m0, n0);
   // symmetric rank-k update: tiles strictly above the diagonal have nothing to do
   if (g.lower_only && m0 + BM - 1 < n0) return;
 
@@ -166,7 +186,7 @@ gemm_f64_kernel(GemmDev g) {
   // K range: a lower-triangular A has no terms beyond the tile's last row
   const int kall = g.tri_a ? min(g.K, m0 + BM) : g.K;
   const int kb = split * g.kchunk;
-  const int ke = min(kall, kb + g.kchunk);
+  const int ke = in_split ? min(kall, kb + g.kchunk) : kall;
   const int nslab = ke > kb ? (ke - kb + BK - 1) / BK : 0;
 
   // this thread's pair i of the A slab: column c of ACOLS, row r + i * NT / ACOLS
@@ -410,7 +430,7 @@ gemm_f64_kernel(GemmDev g) {
         double sum = 0.0;
 #pragma unroll
         for (int w = 0; w < WM; ++w) sum += red[w][nl];
-        out[(int64_t)bm * g.N + n] = sum;
+        out[(int64_t)(m0 / BM) * g.N + n] = sum;
       }
     }
     return;
@@ -419,7 +439,7 @@ gemm_f64_kernel(GemmDev g) {
   double* __restrict__ C = g.C + (int64_t)batch * g.strideC;
   const double* __restrict__ dg = g.diag_add ? g.diag_add + (int64_t)batch * g.strideDiag : nullptr;
   double* __restrict__ P =
-      g.part ? g.part + ((int64_t)split * g.batch + batch) * (int64_t)g.M * g.N : nullptr;
+      in_split ? g.part + ((unit - g.whole) * g.splits + split) * (BM * BN) - (m0 + (int64_t)n0 * BM) : nullptr;
 #pragma unroll
   for (int i = 0; i < FM; ++i) {
     const int m = m0 + wm * TM + i * 16 + fr;
@@ -430,29 +450,33 @@ gemm_f64_kernel(GemmDev g) {
         const int n = n0 + wn * TN + j * 16 + fk + 4 * r;
         if (m >= g.M || n >= g.N) continue;
         if (g.lower_only && m < n) continue;
-        if (P) P[m + (int64_t)n * g.M] = acc[i][j][r];
+        if (in_split) P[m + (int64_t)n * BM] = acc[i][j][r];
         else store_result(g, C, dg, m, n, acc[i][j][r]);
       }
     }
   }
 }
 
-// Sum of the K splits in order, then the epilogue. Memory-bound: a thread
-// owns one (m, n) of one batch entry, consecutive threads consecutive m.
+// Sum of the K splits in order, then the epilogue. Memory-bound: a thread owns
+// one (m, n) of one tile, consecutive threads consecutive m.
+template <int B>
 __global__ void __launch_bounds__(256) gemm_f64_reduce_kernel(GemmDev g) {
-  const int m = blockIdx.x * 256 + threadIdx.x, n = blockIdx.y, b = blockIdx.z;
-  if (m >= g.M || (g.lower_only && m < n)) return;
-  const int64_t mn = (int64_t)g.M * g.N;
-  const double* __restrict__ p = g.part + (int64_t)b * mn + m + (int64_t)n * g.M;
+  int tile, batch, m0, n0;
+  tile_of_unit(g, g.whole + blockIdx.y, tile, batch);
+  tile_origin<B, B>(g, tile, m0, n0);
+  const int e = blockIdx.x * 256 + threadIdx.x;
+  const int m = m0 + e % B, n = n0 + e / B;
+  if (m >= g.M || n >= g.N || (g.lower_only && m < n)) return;
+  const double* __restrict__ p = g.part + (int64_t)blockIdx.y * g.splits * (B * B) + e;
   double s = 0.0;
-  for (int q = 0; q < g.splits; ++q) s += p[(int64_t)q * g.batch * mn];
-  store_result(g, g.C + (int64_t)b * g.strideC, g.diag_add ? g.diag_add + (int64_t)b * g.strideDiag : nullptr, m, n,
-               s);
+  for (int q = 0; q < g.splits; ++q) s += p[(int64_t)q * (B * B)];
+  store_result(g, g.C + (int64_t)batch * g.strideC,
+               g.diag_add ? g.diag_add + (int64_t)batch * g.strideDiag : nullptr, m, n, s);
 }
 
 // NB: B not transposed only (column tiles that are no power of two)
 template <int BM, int BN, int WM, int WN, bool DOT, int KLASS, bool NB = false>
-int launch_cfg(const GemmF64& h, hipStream_t stream) {
+int launch_cfg(const GemmF64& h, hipStream_t stream, int splits = 1, int64_t whole = 0) {
   GemmDev g;
   g.M = h.M; g.N = h.N; g.K = h.K;
   g.A = h.A; g.lda = h.lda; g.strideA = h.strideA;
@@ -473,17 +497,18 @@ int launch_cfg(const GemmF64& h, hipStream_t stream) {
   g.dotB = h.dotB; g.lddot = h.lddot; g.dotpart = h.dotpart; g.strideDot = h.strideDot;
   g.dot_cc = h.dot_cc; g.dot_cd = h.dot_cd;
   g.dot_w = h.dot_w; g.strideDotW = h.strideDotW;
-  g.splits = std::max(1, h.splits);
-  g.kchunk = ((h.K + g.splits - 1) / g.splits + BK - 1) / BK * BK;
-  g.part = g.splits > 1 ? h.split_work : nullptr;
-  MGW_REQUIRE(g.splits == 1 || (h.split_work && !h.dotpart && h.N <= 65535 && h.batch <= 65535), MGW_ERR_ARG,
-              "gemm_f64: a split K needs a workspace and a plain output");
   // square-tile symmetric updates enumerate the lower triangle of tiles only;
   // other lower-only shapes launch the full grid and skip upper tiles
   const int64_t tiles = (h.lower_only && BM == BN) ? (int64_t)g.tiles_m * (g.tiles_m + 1) / 2
                                                    : (int64_t)g.tiles_m * g.tiles_n;
-  g.nblocks = tiles * g.splits * h.batch;
-  MGW_REQUIRE(tiles * g.splits < (1ll << 31) && g.nblocks < (1ll << 31), MGW_ERR_ARG, "gemm_f64: too many tiles");
+  const int64_t units = tiles * h.batch;
+  MGW_REQUIRE(units < (1ll << 31), MGW_ERR_ARG, "gemm_f64: too many tiles");
+  g.splits = splits;
+  g.whole = splits > 1 ? whole : units;
+  g.rest = units - g.whole;
+  g.kchunk = (int)(((h.K + (int64_t)splits - 1) / splits + BK - 1) / BK * BK);
+  g.part = splits > 1 ? h.split_work : nullptr;
+  g.nblocks = g.whole + g.rest * splits;
   MGW_REQUIRE(h.batch >= 1, MGW_ERR_ARG, "gemm_f64: batch out of range");
   dim3 grid((unsigned)g.nblocks, 1, 1);
   dim3 block(64 * WM * WN, 1, 1);
@@ -499,10 +524,12 @@ int launch_cfg(const GemmF64& h, hipStream_t stream) {
   MGW_GEMM_CASE(1, 1)
 #undef MGW_GEMM_CASE
   MGW_HIP(hipGetLastError());
-  if (g.splits > 1) {
-    hipLaunchKernelGGL(gemm_f64_reduce_kernel, dim3((h.M + 255) / 256, h.N, h.batch), dim3(256), 0, stream, g);
-    MGW_HIP(hipGetLastError());
-  }
+  if constexpr (BM == BN && !DOT)
+    if (splits > 1) {
+      hipLaunchKernelGGL(gemm_f64_reduce_kernel<BM>, dim3(BM * BM / 256, (unsigned)g.rest), dim3(256), 0,
+                         stream, g);
+      MGW_HIP(hipGetLastError());
+    }
   return MGW_OK;
 }
 
@@ -522,9 +549,10 @@ int gemm_f64_dot_rowblocks(int M) { return (M + 63) / 64; }
 namespace {
 
 constexpr int NCFG = 4;
+constexpr int TUNE_SPLIT = 4;      // products with a split K, of candidates of their own
 
 struct TuneKey {
-  int klass, ta, tb, lower, mb, nb, kb;
+  int klass, ta, tb, lower, mb, nb, kb;   // lower: plus what tells candidate lists of one family apart
   bool operator<(const TuneKey& o) const {
     return std::tie(klass, ta, tb, lower, mb, nb, kb) < std::tie(o.klass, o.ta, o.tb, o.lower, o.mb, o.nb, o.kb);
   }
@@ -619,29 +647,69 @@ int64_t tile_count(int M, int N, int batch, bool lower, int b) {
   return (lower ? tm * (tm + 1) / 2 : tm * tn) * batch;
 }
 
-// Cost in cycles of a plain product on b x b tiles (128 or 64) with the K range
-// in s splits. Two workgroups of 128x128 or four of 64x64 share a CU's four
-// SIMDs; a round of them lasts as long as its K range plus a fixed prologue
-// and epilogue. A k step costs the sharing workgroups' MFMA cycles at the
-// part of the peak that they reach together (128x128: 0.55 alone, 0.85 for
+// How a plain product runs on b x b tiles (128 or 64): the first `whole` tiles
+// by one workgroup each, the others by `splits` workgroups along K.
+struct SplitPlan {
+  int b, splits;
+  int64_t whole, rest;
+};
+
+// The cheapest plan in cycles. Two workgroups of 128x128 or four of 64x64 share
+// a CU's four SIMDs; a round of them lasts as long as its K range plus a fixed
+// prologue and epilogue. A k step costs the sharing workgroups' MFMA cycles at
+// the part of the peak that they reach together (128x128: 0.55 alone, 0.85 for
 // two; 64x64: 0.25, 0.45, 0.6, 0.68), so a last round that does not fill the
-// slots is cheaper than a whole one. Partial products are written and read
-// once at HBM's copy rate (1.9 KB per cycle).
-double tile_cost(int M, int N, int K, int batch, bool lower, int b, int s) {
-  const int64_t tiles = tile_count(M, N, batch, lower, b) * s;
+// slots is cheaper than a whole one. With `split`, the K range of the last
+// round's tiles may be split, into at most two rounds of workgroups (64x64: 64,
+// 128x128: 128 MiB of partial products); those are written and read once at
+// HBM's copy rate (1.9 KB per cycle). Equal costs take the smaller tiles, also
+// when a product fits one of them: the larger one only adds idle waves.
+SplitPlan split_plan(int M, int N, int K, int batch, bool lower, bool split) {
   constexpr double step128[3] = {0.0, 256.0 / 0.55, 512.0 / 0.85};
   constexpr double step64[5] = {0.0, 64.0 / 0.25, 128.0 / 0.45, 192.0 / 0.6, 256.0 / 0.68};
-  const double* step = b == 128 ? step128 : step64;
-  const int share = b == 128 ? 2 : 4, slots = 256 * share;
-  double c = ((double)K / s + 48.0) * ((double)(tiles / slots) * step[share] + step[(tiles % slots + 255) / 256]);
-  if (s > 1) c += 10000.0 + 16.0 * s * M * (double)N * batch * (lower ? 0.5 : 1.0) / 1900.0;
-  return c;
+  SplitPlan best{};
+  double cost = 0.0;
+  for (const int b : {64, 128}) {
+    const double* step = b == 128 ? step128 : step64;
+    const int share = b == 128 ? 2 : 4, slots = 256 * share;
+    const int64_t tiles = tile_count(M, N, batch, lower, b);
+    const int64_t rest = tiles % slots, whole = tiles - rest;
+    const double full = (K + 48.0) * (double)(whole / slots) * step[share];
+    // 8 bytes of a partial product written and read, cycles per split
+    const double traffic = 16.0 * M * (double)N * batch * (lower ? 0.5 : 1.0) * rest / tiles / 1900.0;
+    for (int s = 1; s == 1 || (split && rest > 0 && K / s >= 64 && s * rest <= 2 * slots); ++s) {
+      const int64_t wgs = s * rest;
+      double c = full + ((double)K / s + 48.0) *
+                            ((double)(wgs / slots) * step[share] + step[(wgs % slots + 255) / 256]);
+      if (s > 1) c += 10000.0 + s * traffic;
+      else if (split) c *= 0.95;      // a split has to gain one part in twenty
+      if (best.b == 0 || c < cost) {
+        cost = c;
+        best = SplitPlan{b, s, s > 1 ? whole : tiles, s > 1 ? rest : 0};
+      }
+    }
+  }
+  return best;
 }
 
-// Tiles: 128x128 with four waves, or 64x64 (also when a product fits one such
-// tile: the larger one only adds idle waves).
-int default_cfg(int M, int N, int K, int batch, bool lower, int s) {
-  return tile_cost(M, N, K, batch, lower, 64, s) <= tile_cost(M, N, K, batch, lower, 128, s) ? 3 : 2;
+template <int KLASS>
+int launch_split_cfg(const SplitPlan& p, int cfg, const GemmF64& h, hipStream_t stream) {
+  if (p.b == 64) return launch_cfg<64, 64, 2, 2, false, KLASS>(h, stream, p.splits, p.whole);
+  if (cfg == 0) return launch_cfg<128, 128, 2, 2, false, KLASS>(h, stream, p.splits, p.whole);
+  return launch_cfg<128, 128, 4, 2, false, KLASS>(h, stream, p.splits, p.whole);
+}
+
+// The tuner may pick the waves of a 128-wide tile (0: four, 1: eight), not the
+// tile, which decides what is split.
+int launch_split(const SplitPlan& p, const GemmF64& h, hipStream_t stream) {
+  MGW_REQUIRE(!h.dotpart && !h.no_tune && h.beta == 0.0, MGW_ERR_ARG, "gemm_f64: a split K needs a plain output");
+  auto launch = [&](int cfg) {
+    return h.klass == MGW_KCLASS_GEMM_CHI0 ? launch_split_cfg<MGW_KCLASS_GEMM_CHI0>(p, cfg, h, stream)
+                                           : launch_split_cfg<MGW_KCLASS_GEMM_OTHER>(p, cfg, h, stream);
+  };
+  if (p.b == 64) return launch(0);
+  return autotune_select(h.klass, h.transA ? 1 : 0, h.transB ? 1 : 0, log2_bucket(h.M), log2_bucket(h.N),
+                         log2_bucket((int64_t)h.K * h.batch), 2, 0, launch, stream, TUNE_SPLIT + (h.lower_only ? 1 : 0));
 }
 
 int tune(const GemmF64& h, hipStream_t stream, int* best) {
@@ -666,24 +734,9 @@ int tune(const GemmF64& h, hipStream_t stream, int* best) {
 
 }  // namespace
 
-// K splits of a plain product: the cheapest count by tile_cost. A function of
-// the shape only, so every tile configuration sums in the same order.
-int gemm_f64_splits(int M, int N, int K, int batch, bool lower) {
-  int best = 1;
-  double cost = 0.0;
-  // at most 2 GiB of partial products
-  for (int s = 1; s <= 256 && (s == 1 || (K / s >= 64 && (double)s * M * N * batch <= 268435456.0)); ++s) {
-    const double c = std::min(tile_cost(M, N, K, batch, lower, 128, s), tile_cost(M, N, K, batch, lower, 64, s));
-    if (s == 1 || c < cost) {
-      cost = s == 1 ? 0.95 * c : c;
-      best = s;
-    }
-  }
-  return best;
-}
-
-size_t gemm_f64_split_doubles(int M, int N, int batch, int splits) {
-  return splits > 1 ? (size_t)splits * batch * M * N : 0;
+size_t gemm_f64_split_doubles(int M, int N, int K, int batch, bool lower) {
+  const SplitPlan p = split_plan(M, N, K, batch, lower, true);
+  return p.splits > 1 ? (size_t)p.rest * p.splits * p.b * p.b : 0;
 }
 
 int gemm_autotune_mode(int mode) {
@@ -696,9 +749,9 @@ int gemm_autotune_mode(int mode) {
 }
 
 int autotune_select(int family, int ns, int h, int mb, int nb, int kb, int ncand, int fallback,
-                    const std::function<int(int)>& launch, hipStream_t stream) {
+                    const std::function<int(int)>& launch, hipStream_t stream, int list) {
   Tuner& t = tuner();
-  const TuneKey key{family, ns, h, 0, mb, nb, kb};
+  const TuneKey key{family, ns, h, list, mb, nb, kb};
   int choice = fallback;
   bool need_tune = false;
   {
@@ -764,9 +817,11 @@ int gemm_f64(const GemmF64& h, hipStream_t stream) {
               "gemm_f64: a triangular A must be square and not transposed");
   MGW_REQUIRE(h.dotpart != nullptr || h.C != nullptr, MGW_ERR_ARG, "gemm_f64: no output");
   if (h.dotpart) return launch_cfg<64, 64, 2, 2, true, MGW_KCLASS_GEMM_WB>(h, stream);
-  int cfg = default_cfg(h.M, h.N, h.K, h.batch, h.lower_only, std::max(1, h.splits));
+  const SplitPlan plan = split_plan(h.M, h.N, h.K, h.batch, h.lower_only, h.split_work != nullptr);
+  if (plan.splits > 1) return launch_split(plan, h, stream);
+  int cfg = plan.b == 64 ? 3 : 2;
   // few columns, and rows enough to fill the GPU: column tiles that N fills
-  if (h.splits <= 1 && !h.transB && !h.lower_only && h.N < 1024 &&
+  if (!h.transB && !h.lower_only && h.N < 1024 &&
       ((int64_t)h.M + 127) / 128 * ((h.N + 111) / 112) * h.batch >= 512) {
     const int fn = narrow_fn(h.N, h.K);
     if (fn > 0)

@@ -120,9 +120,8 @@ struct GemmF64 {
   double dot_cc = 0.0, dot_cd = 1.0;
   double* dotpart = nullptr; int64_t strideDot = 0;
   const double* dot_w = nullptr; int64_t strideDotW = 0;
-  // K split into `splits` partial products (gemm_f64_splits) kept in
-  // split_work (gemm_f64_split_doubles) and summed in order (FP64, no dots)
-  int splits = 1;
+  // room for the partial products of a split K (FP64, beta 0, no dots):
+  // gemm_f64_split_doubles; without it the product runs unsplit
   double* split_work = nullptr;
   // kernel class: the hot classes get their own kernel symbol so that
   // profiler per-kernel statistics separate them
@@ -156,8 +155,8 @@ size_t chi0_split_workspace(int naux, int npole, int nomega, int precision);
 int chi0_split_syrk(const double* x, int naux, int npole, const double* sw, int nomega, int precision,
                     void* work, size_t work_bytes, double* chi, hipStream_t stream);
 int gemm_f64_dot_rowblocks(int M);   // row blocks of the FP64 dot epilogue's partials
-int gemm_f64_splits(int M, int N, int K, int batch, bool lower);
-size_t gemm_f64_split_doubles(int M, int N, int batch, int splits);
+// doubles of a split K's partial products, at most 128 MiB; 0: no split gains
+size_t gemm_f64_split_doubles(int M, int N, int K, int batch, bool lower);
 // v(n, f) = B_n^T chi(iw_f) B_n = sum_m C (C + 2 B), C = D_f B, from bf16-split
 // operands (MGW_BF16X3 / MGW_BF16X6) of D_f = L_f^-1 - 1 (lower triangle of
 // naux x naux, stride naux^2) and B (naux x ncol); writes the row-block
@@ -238,9 +237,10 @@ int gemm_autotune_mode(int mode); // -1 query; returns the previous mode
 // Key: family, planes, fp16 flag and three log2 shape buckets. With tuning
 // on, an unseen key times every candidate on the actual operands (the last
 // run's output stands) and records the fastest; otherwise the recorded
-// choice, or `fallback`, is launched.
+// choice, or `fallback`, is launched. list: another number for another list of
+// candidates, so that recorded choices are not taken for it.
 int autotune_select(int family, int ns, int h, int mb, int nb, int kb, int ncand, int fallback,
-                    const std::function<int(int)>& launch, hipStream_t stream);
+                    const std::function<int(int)>& launch, hipStream_t stream, int list = 0);
 constexpr int MGW_TUNE_CHI_SYRK = 105;   // K-split chi0 SYRK variants
 constexpr int MGW_TUNE_WB_DOT = 107;     // W.B dot pipelines
 inline int log2_floor(int64_t v) {
