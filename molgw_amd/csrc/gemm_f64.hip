@@ -617,14 +617,15 @@ int launch_by_class(int cfg, const GemmF64& h, hipStream_t stream) {
 // transforms of the occupied states or of a window, the exchange's half
 // transform): the FN whose tiles cover N in the least time, 0 when 128-column
 // tiles do. In units of 16 columns at 1 TFLOP/s, measured at 65536 x 16 FN x
-// 4096: FN = 1 .. 8 run at 23, 38, 42, 48, 58, 53, 56 and 65 TFLOP/s (up to 3
-// the rows' traffic bounds them); a workgroup's fixed cost is that of 60 k, or
-// of 150 for the two widest, of which only two share a CU.
+// 4096: FN = 1 .. 6 and 8 run at 23, 38, 42, 48, 58, 53 and 65 TFLOP/s (up to 3
+// the rows' traffic bounds them; 112 columns, at 56, always cost more than
+// 128); a workgroup's fixed cost is that of 60 k, or of 150 for 128 columns, of
+// which only two share a CU.
 int narrow_fn(int N, int K) {
-  constexpr double w[9] = {0.0, 1 / 23.0, 2 / 38.0, 3 / 42.0, 4 / 48.0, 5 / 58.0, 6 / 53.0, 7 / 56.0, 8 / 65.0};
-  auto cost = [&](int fn) { return (N + 16 * fn - 1) / (16 * fn) * w[fn] * (K + (fn >= 7 ? 150.0 : 60.0)); };
+  constexpr double w[9] = {0.0, 1 / 23.0, 2 / 38.0, 3 / 42.0, 4 / 48.0, 5 / 58.0, 6 / 53.0, 0.0, 8 / 65.0};
+  auto cost = [&](int fn) { return (N + 16 * fn - 1) / (16 * fn) * w[fn] * (K + (fn == 8 ? 150.0 : 60.0)); };
   int best = 8;
-  for (int fn = 7; fn >= 1; --fn)
+  for (int fn = 6; fn >= 1; --fn)
     if (cost(fn) < cost(best)) best = fn;
   return best == 8 ? 0 : best;
 }
@@ -637,8 +638,7 @@ int launch_narrow(int fn, const GemmF64& h, hipStream_t stream) {
     case 3: return launch_cfg<128, 48, 4, 1, false, KLASS, true>(h, stream);
     case 4: return launch_cfg<128, 64, 2, 2, false, KLASS, true>(h, stream);
     case 5: return launch_cfg<128, 80, 4, 1, false, KLASS, true>(h, stream);
-    case 6: return launch_cfg<128, 96, 2, 2, false, KLASS, true>(h, stream);
-    default: return launch_cfg<128, 112, 4, 1, false, KLASS, true>(h, stream);
+    default: return launch_cfg<128, 96, 2, 2, false, KLASS, true>(h, stream);
   }
 }
 
