@@ -1034,6 +1034,41 @@ int polarizability_grid(mgw_ctx* c, const mgw_ranges* r, double spin_fact, int n
   return MGW_OK;
 }
 
+// v(n, f) = sum over rows of the FP64 product g's fused column dots, for all its
+// columns and frequencies. The sums of the single 64-row blocks take 256 MiB at
+// most, or what blocks of 128 rows would on all frequencies; where there is less
+// room, fewer frequencies or columns go at a time. No sum depends on it.
+int column_dots(mgw_ctx* c, const GemmF64& g, double* v) {
+  const int64_t nrb = gemm_f64_dot_rowblocks(g.M), per_f = nrb * g.N;
+  int64_t room = std::max<int64_t>(int64_t(1) << 25, (int64_t)wb_split_rowblocks(g.M) * g.N * g.batch);
+  room = std::min(room, per_f * g.batch);
+  double* part = nullptr;
+  for (;;) {
+    const int rc = dbuf(c, "dot_part", (size_t)room, &part);
+    if (rc == MGW_OK) break;
+    if (rc != MGW_ERR_NOMEM || room <= 64 * nrb) return rc;
+    room = std::max(64 * nrb, room / 2);
+  }
+  const int nf = (int)std::max<int64_t>(1, std::min<int64_t>(g.batch, room / per_f));
+  const int nc = (int)std::min<int64_t>(g.N, std::max<int64_t>(1, room / nrb));
+  for (int f0 = 0; f0 < g.batch; f0 += nf)
+    for (int c0 = 0; c0 < g.N; c0 += nc) {
+      GemmF64 h = g;
+      h.batch = std::min(nf, g.batch - f0);
+      h.N = std::min(nc, g.N - c0);
+      h.A = g.A + g.strideA * f0;
+      h.B = g.B + g.ldb * c0;
+      if (g.dotB) h.dotB = g.dotB + g.lddot * c0;
+      if (g.dot_w) h.dot_w = g.dot_w + g.strideDotW * f0;
+      h.dotpart = part;
+      h.strideDot = nrb * h.N;
+      MGW_TRY(gemm_f64(h, c->stream));
+      // with fewer columns than all, one frequency: h.N values in a row of v
+      MGW_TRY(launch_dot_reduce(part, (int)nrb, h.N, h.batch, nullptr, v + (int64_t)g.N * f0 + c0, c->stream));
+    }
+  return MGW_OK;
+}
+
 // ------------------------------------------------------------------ A7
 int gw_selfenergy_imag(mgw_ctx* c, const mgw_ranges* r, int ncalc, const double* omega_calc, int precision) {
   MGW_REQUIRE(c->has_chi, MGW_ERR_STATE, "no chi: call mgw_polarizability_grid first");
@@ -1047,9 +1082,9 @@ int gw_selfenergy_imag(mgw_ctx* c, const mgw_ranges* r, int ncalc, const double*
   MGW_TRY(dbuf(c, "eri_pm", (size_t)naux * ncol, &epm));
   MGW_TRY(ao2mo(c, glo, ghi, r->nsemin, r->nsemax, epm, precision));
   const bool split = split_precision(precision);
-  const int nrb = split ? wb_split_rowblocks(naux) : gemm_f64_dot_rowblocks(naux);
-  double *part, *v, *om_d, *wt_d, *ep_d, *wc_d, *sc;
-  MGW_TRY(dbuf(c, "dot_part", (size_t)nrb * ncol * nomega, &part));
+  const int nrb = wb_split_rowblocks(naux);
+  double *part = nullptr, *v, *om_d, *wt_d, *ep_d, *wc_d, *sc;
+  if (split) MGW_TRY(dbuf(c, "dot_part", (size_t)nrb * ncol * nomega, &part));
   MGW_TRY(dbuf(c, "dot_v", (size_t)ncol * nomega, &v));
   // diag(B_m^T chi(iw) B_m) for every (p, m) and iw (src/m_gw_selfenergy_grid.f90:297-310).
   // With chi = L^-T L^-1 - 1 and D = L^-1 - 1 (lower triangular, resident):
@@ -1060,7 +1095,6 @@ int gw_selfenergy_imag(mgw_ctx* c, const mgw_ranges* r, int ncalc, const double*
   g.A = find_buf(c, "wpol_linv"); g.lda = naux; g.strideA = (int64_t)naux * naux; g.tri_a = true;
   g.B = epm; g.ldb = naux; g.strideB = 0;
   g.dotB = epm; g.lddot = naux; g.dot_cc = 1.0; g.dot_cd = 2.0;
-  g.dotpart = part; g.strideDot = (int64_t)nrb * ncol;
   g.batch = nomega;
   g.batch_outer = true;   // one L^-1 stays in cache while B streams past it
   {
@@ -1072,11 +1106,13 @@ int gw_selfenergy_imag(mgw_ctx* c, const mgw_ranges* r, int ncalc, const double*
       MGW_TRY(dbuf(c, "wb_split", (bytes + 7) / 8, &work));
       MGW_TRY(wb_split_dot(g.A, naux, nomega, epm, ncol, precision, work, bytes, part, c->stream));
     } else {
-      MGW_TRY(gemm_f64(g, c->stream));
+      MGW_TRY(column_dots(c, g, v));
     }
   }
-  if (split) MGW_TRY(scratch_done(c, "wb_split"));
-  MGW_TRY(launch_dot_reduce(part, nrb, ncol, nomega, nullptr, v, c->stream));
+  if (split) {
+    MGW_TRY(scratch_done(c, "wb_split"));
+    MGW_TRY(launch_dot_reduce(part, nrb, ncol, nomega, nullptr, v, c->stream));
+  }
   std::vector<double> ep(np);
   for (int k = 0; k < np; ++k) ep[k] = c->energy_in_g()[c->so() + glo - 1 + k];
   MGW_TRY(upload_group(c, "sgi_in", {part_of(c->chi_omega.data(), (size_t)nomega, &om_d),
@@ -1303,24 +1339,20 @@ int contour_sigma(mgw_ctx* c, const mgw_ranges* r, double eta, int nomega, const
   double* epm = nullptr;
   MGW_TRY(dbuf(c, "eri_pm", (size_t)naux * ncol, &epm));
   MGW_TRY(ao2mo(c, glo, ghi, r->nsemin, r->nsemax, epm, MGW_FP64));
-  const int nrb = gemm_f64_dot_rowblocks(naux);
-  double *part, *v;
-  MGW_TRY(dbuf(c, "dot_part", (size_t)nrb * ncol * nf, &part));
+  double* v = nullptr;
   MGW_TRY(dbuf(c, "dot_v", (size_t)ncol * nf, &v));
   GemmF64 g;
   g.M = naux; g.N = (int)ncol; g.K = naux;
   g.transA = true; g.A = find_buf(c, "cd_u"); g.lda = naux; g.strideA = (int64_t)naux * naux;
   g.B = epm; g.ldb = naux; g.strideB = 0;
   g.dot_w = find_buf(c, "cd_w"); g.strideDotW = naux;
-  g.dotpart = part; g.strideDot = (int64_t)nrb * ncol;
   g.batch = nf;
   g.batch_outer = true;
   {
     ProfScope ps(&c->prof, MGW_KCLASS_GEMM_WB, 2.0 * naux * (double)naux * ncol * nf,
                  8.0 * ((double)naux * naux * nf + (double)naux * ncol), c->stream);
-    MGW_TRY(gemm_f64(g, c->stream));
+    MGW_TRY(column_dots(c, g, v));
   }
-  MGW_TRY(launch_dot_reduce(part, nrb, ncol, nf, nullptr, v, c->stream));
   std::vector<double> ep(np);
   std::vector<int32_t> ps(np);
   for (int k = 0; k < np; ++k) {
@@ -1636,9 +1668,7 @@ int64_t mgw_footprint_bytes_nse(int nbf, int nauxil, int nstate, int nocc, int n
   // self-energy stage: half transform and (P|pm) for the ne states p, all m
   int64_t stage_s = na * nb * ne + na * ne * ns + na * npole + (int64_t(1) << 27);
   if (technique != MGW_TECH_ONE_SHOT)   // column-dot partials and v on every frequency
-    stage_s += (int64_t)((split_precision(precision) ? mgw::wb_split_rowblocks((int)na)
-                                                     : mgw::gemm_f64_dot_rowblocks((int)na)) + 1) *
-               ns * ne * nomega_chi_imag;
+    stage_s += (int64_t)(mgw::wb_split_rowblocks((int)na) + 1) * ns * ne * nomega_chi_imag;
   if (technique != MGW_TECH_ONE_SHOT && split_precision(precision))
     stage_s += (int64_t)((mgw::wb_split_workspace((int)na, ns * ne, nomega_chi_imag, precision) + 7) / 8);
   // the temporaries of the W stage stay cached while the self-energy runs
