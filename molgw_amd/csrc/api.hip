@@ -2512,7 +2512,15 @@ int mgw_gw_selfenergy_qs(mgw_ctx* c, const mgw_ranges* r, double spin_fact, doub
   double *w, *b, *sig_i;
   MGW_TRY(dbuf(c, "sigma_w", (size_t)npole * nse * ic, &w));
   MGW_TRY(dbuf(c, "qs_b", (size_t)npole * nse * ic, &b));
-  MGW_TRY(dbuf(c, "qs_sigma_i", (size_t)nse * nse * ic, &sig_i));
+  // and the products of jc states within 1 GiB too; where there is less room,
+  // fewer, down to none (each product then adds to the sum by itself)
+  const size_t per_product = (size_t)nse * nse * sizeof(double);
+  int jc = (int)std::max<size_t>(1, std::min<size_t>((size_t)ic, (size_t(1) << 30) / per_product));
+  for (; jc > 0; jc /= 2) {
+    const int rc = dbuf(c, "qs_sigma_i", (size_t)nse * nse * jc, &sig_i);
+    if (rc == MGW_OK) break;
+    if (rc != MGW_ERR_NOMEM) return rc;
+  }
   const double* ws = find_buf(c, "wpol_ws");
   const double* pole = find_buf(c, "wpol_pole");
   for (int i0 = 0; i0 < ng; i0 += ic) {
@@ -2527,19 +2535,23 @@ int mgw_gw_selfenergy_qs(mgw_ctx* c, const mgw_ranges* r, double spin_fact, doub
     MGW_TRY(gemm_f64(g, c->stream));
     MGW_TRY(launch_qs_scale(w, b, npole, nse, cnt, pole, eq_d, ei_d + i0, fi_d + i0, spin_fact, eta, c->stream));
     // Sigma(p, q) += sum_i sum_s w(s, p, i) b(s, q, i)   (:736-744): one
-    // product per i in one batched launch, then the sum over i in order. One
-    // launch per i left all but a few of the CUs idle (nse = 96, npole = 1520, 96
-    // states i: 11.0 ms in 96 launches, 0.15 ms in two).
-    GemmF64 h;
-    h.M = nse; h.N = nse; h.K = npole;
-    h.transA = true; h.A = w; h.lda = npole; h.strideA = (int64_t)npole * nse;
-    h.B = b; h.ldb = npole; h.strideB = (int64_t)npole * nse;
-    h.C = sig_i; h.ldc = nse; h.strideC = (int64_t)nse * nse;
-    h.batch = cnt;
-    h.batch_outer = true;
-    h.klass = MGW_KCLASS_GEMM_SIGMA;
-    MGW_TRY(gemm_f64(h, c->stream));
-    MGW_TRY(launch_batch_sum(sig_i, (int64_t)nse * nse, cnt, i0 > 0 ? 1 : 0, sig, c->stream));
+    // product per i in one batched launch, then the sum over i in a fixed
+    // order. One launch per i left all but a few of the CUs idle (nse = 96,
+    // npole = 1520, 96 states i: 11.0 ms in 96 launches, 0.15 ms in two).
+    for (int k = 0; k < cnt; k += std::max(1, jc)) {
+      const int n = std::min(std::max(1, jc), cnt - k), later = i0 + k > 0 ? 1 : 0;
+      GemmF64 h;
+      h.M = nse; h.N = nse; h.K = npole;
+      h.transA = true; h.A = w + (int64_t)npole * nse * k; h.lda = npole; h.strideA = (int64_t)npole * nse;
+      h.B = b + (int64_t)npole * nse * k; h.ldb = npole; h.strideB = (int64_t)npole * nse;
+      h.C = jc > 0 ? sig_i : sig; h.ldc = nse; h.strideC = (int64_t)nse * nse;
+      if (jc == 0) h.beta = later;
+      h.batch = n;
+      h.batch_outer = true;
+      h.klass = MGW_KCLASS_GEMM_SIGMA;
+      MGW_TRY(gemm_f64(h, c->stream));
+      if (jc > 0) MGW_TRY(launch_batch_sum(sig_i, (int64_t)nse * nse, n, later, sig, c->stream));
+    }
   }
   MGW_TRY(launch_symmetrize(sig, nse, c->stream));
   if (selfenergy_mo) {

@@ -5,7 +5,8 @@ import numpy as np
 import pytest
 
 from molgw_amd.gw import Engine, selfenergy_set_state_range
-from molgw_amd.workloads import synthetic_system
+from molgw_amd.workloads import dense_ri, synthetic_system
+from oracle import gw_oracle as O
 
 pytestmark = pytest.mark.gpu
 MIB = 1 << 20
@@ -100,3 +101,38 @@ def test_contour_dot_partials(monkeypatch):
         got, _ = eng.gw_selfenergy_contour(rng, omega, e0, 12)
         assert eng.memory()[0] <= limit
     np.testing.assert_array_equal(got, ref)
+
+
+def test_qs_state_products(monkeypatch):
+    """The QS self-energy's products of the single states i: 1 GiB of them at a
+    time also where there are fewer poles than states, and fewer where there is
+    less room."""
+    n, naux = 640, 4
+    s = synthetic_system(n, naux, 5, seed=27, scale=0.3)
+    g = np.random.default_rng(28)
+    pole, ws = np.array([0.4, 1.1]), g.standard_normal((naux, 2))
+    rng = selfenergy_set_state_range(s.occupation)
+    with loaded(s) as eng:
+        eng.set_spectral_function(pole, ws)
+        before = eng.memory()[0]
+        ref, _ = eng.gw_selfenergy_qs(rng, eta=0.05)
+        held = eng.memory()[0]
+    # (P|pi) and its half transform, w and its scaled copy, the result
+    operands = 8 * (2 * naux * n * n + 2 * 2 * n * n + 4 * n * n)
+    assert held - before <= operands + 1024 * MIB + MIB
+    epi = np.einsum('pkl,km,li->pmi', dense_ri(s), s.c_matrix, s.c_matrix, optimize=True)
+    want = O.gw_selfenergy_qs(epi, ws, pole, s.energy, s.occupation, rng, eta=0.05)
+    # each entry: 2 n terms of at most max w^2 / eta, each off by a few times naux 2^-53
+    w = np.einsum('ps,pmi->smi', ws, epi)
+    size = np.einsum('smi->m', w * w) / 0.05
+    bound = 4 * (2 * naux + 2 * n) * 2.0 ** -53 * np.sqrt(size[:, None] * size[None, :])
+    assert np.all(np.abs(ref - want) <= bound)
+    for room in (64 * MIB, MIB):
+        with loaded(s) as eng:
+            eng.set_spectral_function(pole, ws)
+            limit = eng.memory()[0] + operands + room
+            monkeypatch.setenv('MGW_ALLOC_LIMIT', str(limit))
+            got, _ = eng.gw_selfenergy_qs(rng, eta=0.05)
+            monkeypatch.delenv('MGW_ALLOC_LIMIT')
+            assert eng.memory()[0] <= limit
+            assert np.all(np.abs(got - want) <= bound)
