@@ -679,6 +679,14 @@ static int sigma_ichunks(int nsb, int nse, int ni) {
   return (int)std::max<int64_t>(1, std::min<int64_t>(ni, (2048 + have - 1) / have));
 }
 
+// frequencies per launch: partial sums of 256 MiB, or 63 frequencies' if those
+// take more
+static int sigma_group(int npole, int nse, int ni, int nomega) {
+  const int nsb = (npole + SIGMA_SB - 1) / SIGMA_SB;
+  const int64_t fit = (int64_t(1) << 24) / ((int64_t)sigma_ichunks(nsb, nse, ni) * nsb * nse) - 1;
+  return std::min(nomega, (int)std::max<int64_t>(63, std::min<int64_t>(SIGMA_MAXK, fit)));
+}
+
 int launch_sigma_poles(const double* w, int npole, int nse, int ni, const double* pole,
                        const double* omega, int nomega, const double* e0p, const double* ei,
                        const double* fi, const double* ep, const double* occp, double spin_fact,
@@ -688,8 +696,9 @@ int launch_sigma_poles(const double* w, int npole, int nse, int ni, const double
   MGW_REQUIRE(nse <= 65535, MGW_ERR_ARG, "sigma_poles: too many states");
   const int nsb = (npole + SIGMA_SB - 1) / SIGMA_SB;
   const int want = sigma_ichunks(nsb, nse, ni), ichunk = (ni + want - 1) / want, nz = (ni + ichunk - 1) / ichunk;
-  for (int k0 = 0; k0 < nomega; k0 += SIGMA_MAXK) {
-    const int nk = std::min(SIGMA_MAXK, nomega - k0);
+  const int group = sigma_group(npole, nse, ni, nomega);
+  for (int k0 = 0; k0 < nomega; k0 += group) {
+    const int nk = std::min(group, nomega - k0);
     const dim3 grid(nsb, nse, nz);
     if (nk < 4)
       hipLaunchKernelGGL(sigma_poles_kernel<1>, grid, dim3(256), 0, s, w, npole, nse, ni, ichunk, nsb, pole,
@@ -707,7 +716,7 @@ int launch_sigma_poles(const double* w, int npole, int nse, int ni, const double
 
 int64_t sigma_part_doubles(int npole, int nse, int ni, int nomega) {
   const int nsb = (npole + SIGMA_SB - 1) / SIGMA_SB;
-  return (int64_t)sigma_ichunks(nsb, nse, ni) * nsb * nse * (std::min(nomega, SIGMA_MAXK) + 1) * 2;
+  return (int64_t)sigma_ichunks(nsb, nse, ni) * nsb * nse * (sigma_group(npole, nse, ni, nomega) + 1) * 2;
 }
 
 // ------------------------------------------------------------------ chi (imaginary axis)

@@ -136,3 +136,26 @@ def test_qs_state_products(monkeypatch):
             monkeypatch.delenv('MGW_ALLOC_LIMIT')
             assert eng.memory()[0] <= limit
             assert np.all(np.abs(got - want) <= bound)
+
+
+def test_pole_self_energy_partial_sums():
+    """256 MiB of partial sums however many poles and frequencies there are; the
+    frequencies of one launch do not change another's result."""
+    n, naux, npole = 60, 2, 1000000
+    s = synthetic_system(n, naux, 5, seed=29, scale=0.3)
+    g = np.random.default_rng(30)
+    pole, ws = np.sort(g.uniform(0.4, 3.0, npole)), g.standard_normal((naux, npole)) * 1e-3
+    rng = selfenergy_set_state_range(s.occupation)
+    omega = np.linspace(-0.3, 0.3, 300)
+    with loaded(s) as eng:
+        eng.set_spectral_function(pole, ws)
+        before = eng.memory()[0]
+        got, egw = eng.gw_selfenergy(rng, omega, s.energy, eta=0.05)
+        held = eng.memory()[0]
+        sub, sub_egw = eng.gw_selfenergy(rng, omega[100:104], s.energy, eta=0.05)
+    # w of two states i, the half transform and (P|pi), the result
+    operands = 8 * (2 * npole * n + 2 * naux * n * n + 2 * 300 * n)
+    assert held - before <= operands + 257 * MIB
+    # the poles' sums are taken in another order: npole n terms of one sign each
+    scale = np.max(np.abs(got))
+    assert np.max(np.abs(sub - got[100:104])) <= 2 * npole * n * 2.0 ** -53 * scale and abs(sub_egw - egw) <= 1e-9 * abs(egw)
