@@ -159,9 +159,10 @@ struct mgw_ctx {
     int n, nbatch;
     const void *a, *logdet, *info, *work, *bounds, *planes;
     int f16_min;
+    bool leaf_block;
     bool operator<(const GraphKey& o) const {
-      return std::tie(n, nbatch, a, logdet, info, work, bounds, planes, f16_min) <
-             std::tie(o.n, o.nbatch, o.a, o.logdet, o.info, o.work, o.bounds, o.planes, o.f16_min);
+      return std::tie(n, nbatch, a, logdet, info, work, bounds, planes, f16_min, leaf_block) <
+             std::tie(o.n, o.nbatch, o.a, o.logdet, o.info, o.work, o.bounds, o.planes, o.f16_min, o.leaf_block);
     }
   };
   bool use_graphs = false;
@@ -840,8 +841,9 @@ int gw_selfenergy(mgw_ctx* c, const mgw_ranges* r, double spin_fact, double eta,
   return MGW_OK;
 }
 
-// The batched Cholesky sequence (6 n / 64 launches, no host synchronisation)
-// is captured once per shape and buffer set into a HIP graph and replayed
+// The batched Cholesky sequence (about 5 launches per 128 columns, no host
+// synchronisation) is captured once per shape, buffer set and setting of the
+// switches that decide its kernels into a HIP graph and replayed
 // when the context has graphs enabled; the autotuner's timing mode launches
 // eagerly because it synchronises.
 void clear_graphs(mgw_ctx* c) {
@@ -854,7 +856,7 @@ int run_chol(mgw_ctx* c, double* A, int n, int nbatch, double* logdet, int32_t* 
   if (!c->use_graphs || gemm_autotune_mode(-1) == 1)
     return chol_inverse_batched(A, n, nbatch, logdet, info, work, c->stream, bounds, planes);
   const mgw_ctx::GraphKey key{n, nbatch, A, logdet, info, work, bounds, planes,
-                             bounds ? chol_f16_min() * 2 + (chol_epi_planes() ? 1 : 0) : 0};
+                             bounds ? chol_f16_min() * 2 + (chol_epi_planes() ? 1 : 0) : 0, chol_leaf_block()};
   auto it = c->graphs.find(key);
   if (it == c->graphs.end()) {
     MGW_HIP(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));

@@ -305,10 +305,6 @@ chol_block_kernel(double* __restrict__ A, int n, int64_t strideA, int k, int m, 
 // at every factorisation) chol_diag_kernel on blocks of up to 64. A 128 leaf
 // takes the place of two 64 leaves and the four products that join them.
 constexpr int LEAF = 2 * NB;
-bool chol_leaf_block() {
-  const char* e = std::getenv("MGW_CHOL_LEAF");
-  return e ? std::atoi(e) != 0 : true;
-}
 
 int gemm_chol(const GemmF64& g0, hipStream_t stream) {
   GemmF64 g = g0;
@@ -980,6 +976,11 @@ size_t chol_plane_bytes(int n, int nbatch) {
 // for bit). Read at every factorisation.
 bool chol_epi_planes() {
   const char* e = std::getenv("MGW_CHOL_EPI_PLANES");
+  return e ? std::atoi(e) != 0 : true;
+}
+
+bool chol_leaf_block() {
+  const char* e = std::getenv("MGW_CHOL_LEAF");
   return e ? std::atoi(e) != 0 : true;
 }
 

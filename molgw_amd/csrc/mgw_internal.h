@@ -226,6 +226,7 @@ size_t chol_work_doubles(int n);
 size_t chol_plane_bytes(int n, int nbatch);
 int chol_f16_min();
 bool chol_epi_planes();
+bool chol_leaf_block();
 int chol_inverse_batched(double* A, int n, int nbatch, double* logdet, int32_t* info, double* work,
                          hipStream_t stream, double* bounds = nullptr, void* planes = nullptr);
 // tr[f] = sum of squares of the lower triangle of M_f (n x n, stride n^2).
