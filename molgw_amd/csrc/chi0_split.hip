@@ -1466,11 +1466,13 @@ int split_and_syrk(const double* x, int naux, int npole, const double* sw, int n
         return MGW_OK;
       };
       if (NS == 2 && !std::getenv("MGW_CHI_SYRK")) {
-        // the tuner picks among the 128-wide variants (same products in the
-        // same order: identical results) per shape class
+        // the tuner picks among the default (256-wide tiles where they fill the
+        // GPU, list 1, else the 128-wide register prefetch, list 0) and the
+        // other 128-wide variants per shape class: the same products in the
+        // same order, identical results
         static constexpr int CAND[7] = {0, 1, 2, 3, 4, 7, 8};
         MGW_TRY(autotune_select(MGW_TUNE_CHI_SYRK, NS, H ? 1 : 0, log2_floor(naux), log2_floor(L.nkt), log2_floor(nf),
-                                7, 0, [&](int c) { return launch(CAND[c]); }, stream));
+                                7, 0, [&](int c) { return launch(CAND[c]); }, stream, pp ? 1 : 0));
       } else {
         MGW_TRY(launch(var));
       }

@@ -453,7 +453,7 @@ int split_and_dot(const double* d, int naux, int nomega, const double* b, int64_
     // would cost 128 VGPRs and half the occupancy)
     if constexpr (NS == 2) {
       // DEPTH 1 (default) or 3: the same products in the same order, so the
-      // tuner may pick either per shape
+      // tuner may pick either per shape (list 1: list 0 held DEPTH 3 and 2)
       auto launch = [&](int c) -> int {
         if (c == 0)
           hipLaunchKernelGGL((wb_dot_kernel<NS, H, BM, BN, 2, 2, 0, 1>), dim3((unsigned)g.nblocks), dim3(256), 0,
@@ -465,7 +465,7 @@ int split_and_dot(const double* d, int naux, int nomega, const double* b, int64_
         return MGW_OK;
       };
       MGW_TRY(autotune_select(MGW_TUNE_WB_DOT, NS, H ? 1 : 0, log2_floor(naux), log2_floor(ncol), log2_floor(nf), 2, 0,
-                              launch, stream));
+                              launch, stream, 1));
     } else {
       hipLaunchKernelGGL((wb_dot_kernel<NS, H, BM, BN, 2, 2, 4, 2>), dim3((unsigned)g.nblocks), dim3(256), 0, stream, g);
       MGW_HIP(hipGetLastError());
