@@ -543,12 +543,15 @@ int gemm_f64_dot_rowblocks(int M) { return (M + 63) / 64; }
 // ------------------------------------------------------------------ autotuner
 // Candidate tile configurations (all FP64 MFMA, BK = 16):
 //   0: 256x128, 16 waves   1: 128x128, 8 waves   2: 128x128, 4 waves   3: 64x64, 4 waves
-// The defaults (2, and 3 for small products) were measured on MI355X. With tuning on, the first product of a new
-// (class, transposes, lower, log2 M/N/K bucket) times every candidate on
+//   4: 128 x 16 FN, 4 waves (products of few columns only)
+// The defaults (2, 3 for small products, 4 for few columns) were measured on
+// MI355X. With tuning on, the first product of a new (class, transposes, lower
+// or few columns, log2 M/N/K bucket) times every candidate on
 // the actual operands and keeps the fastest; the table can be persisted.
 namespace {
 
 constexpr int NCFG = 4;
+constexpr int TUNE_COLUMNS = 2;    // products that column tiles are the default of, candidate NCFG
 constexpr int TUNE_SPLIT = 4;      // products with a split K, of candidates of their own
 
 struct TuneKey {
@@ -602,17 +605,6 @@ int launch_candidate(int cfg, const GemmF64& h, hipStream_t stream) {
   }
 }
 
-int launch_by_class(int cfg, const GemmF64& h, hipStream_t stream) {
-  switch (h.klass) {
-    case MGW_KCLASS_GEMM_AO2MO: return launch_candidate<MGW_KCLASS_GEMM_AO2MO>(cfg, h, stream);
-    case MGW_KCLASS_GEMM_CASIDA: return launch_candidate<MGW_KCLASS_GEMM_CASIDA>(cfg, h, stream);
-    case MGW_KCLASS_GEMM_SIGMA: return launch_candidate<MGW_KCLASS_GEMM_SIGMA>(cfg, h, stream);
-    case MGW_KCLASS_GEMM_CHI0: return launch_candidate<MGW_KCLASS_GEMM_CHI0>(cfg, h, stream);
-    case MGW_KCLASS_CHOLESKY: return launch_candidate<MGW_KCLASS_CHOLESKY>(cfg, h, stream);
-    default: return launch_candidate<MGW_KCLASS_GEMM_OTHER>(cfg, h, stream);
-  }
-}
-
 // Column tiles of 16 FN < 128 columns for products of few columns (the
 // transforms of the occupied states or of a window, the exchange's half
 // transform): the FN whose tiles cover N in the least time, 0 when 128-column
@@ -639,6 +631,22 @@ int launch_narrow(int fn, const GemmF64& h, hipStream_t stream) {
     case 4: return launch_cfg<128, 64, 2, 2, false, KLASS, true>(h, stream);
     case 5: return launch_cfg<128, 80, 4, 1, false, KLASS, true>(h, stream);
     default: return launch_cfg<128, 96, 2, 2, false, KLASS, true>(h, stream);
+  }
+}
+
+// cfg NCFG: column tiles of 16 fn (kernels of classes other than AO2MO carry the
+// symbol of GEMM_OTHER there, and a profile counts them to it)
+int launch_by_class(int cfg, int fn, const GemmF64& h, hipStream_t stream) {
+  if (cfg == NCFG)
+    return h.klass == MGW_KCLASS_GEMM_AO2MO ? launch_narrow<MGW_KCLASS_GEMM_AO2MO>(fn, h, stream)
+                                            : launch_narrow<MGW_KCLASS_GEMM_OTHER>(fn, h, stream);
+  switch (h.klass) {
+    case MGW_KCLASS_GEMM_AO2MO: return launch_candidate<MGW_KCLASS_GEMM_AO2MO>(cfg, h, stream);
+    case MGW_KCLASS_GEMM_CASIDA: return launch_candidate<MGW_KCLASS_GEMM_CASIDA>(cfg, h, stream);
+    case MGW_KCLASS_GEMM_SIGMA: return launch_candidate<MGW_KCLASS_GEMM_SIGMA>(cfg, h, stream);
+    case MGW_KCLASS_GEMM_CHI0: return launch_candidate<MGW_KCLASS_GEMM_CHI0>(cfg, h, stream);
+    case MGW_KCLASS_CHOLESKY: return launch_candidate<MGW_KCLASS_CHOLESKY>(cfg, h, stream);
+    default: return launch_candidate<MGW_KCLASS_GEMM_OTHER>(cfg, h, stream);
   }
 }
 
@@ -712,15 +720,15 @@ int launch_split(const SplitPlan& p, const GemmF64& h, hipStream_t stream) {
                          log2_bucket((int64_t)h.K * h.batch), 2, 0, launch, stream, TUNE_SPLIT + (h.lower_only ? 1 : 0));
 }
 
-int tune(const GemmF64& h, hipStream_t stream, int* best) {
+int tune(const GemmF64& h, int fn, hipStream_t stream, int* best) {
   hipEvent_t a, b;
   MGW_HIP(hipEventCreate(&a));
   MGW_HIP(hipEventCreate(&b));
   float best_ms = 1e30f;
   *best = -1;
-  for (int cfg = 0; cfg < NCFG; ++cfg) {
+  for (int cfg = 0; cfg < (fn > 0 ? NCFG + 1 : NCFG); ++cfg) {
     MGW_HIP(hipEventRecord(a, stream));
-    MGW_TRY(launch_by_class(cfg, h, stream));
+    MGW_TRY(launch_by_class(cfg, fn, h, stream));
     MGW_HIP(hipEventRecord(b, stream));
     MGW_HIP(hipEventSynchronize(b));
     float ms = 0.0f;
@@ -819,30 +827,27 @@ int gemm_f64(const GemmF64& h, hipStream_t stream) {
   if (h.dotpart) return launch_cfg<64, 64, 2, 2, true, MGW_KCLASS_GEMM_WB>(h, stream);
   const SplitPlan plan = split_plan(h.M, h.N, h.K, h.batch, h.lower_only, h.split_work != nullptr);
   if (plan.splits > 1) return launch_split(plan, h, stream);
-  int cfg = plan.b == 64 ? 3 : 2;
+  int cfg = plan.b == 64 ? 3 : 2, fn = 0;
   // few columns, and rows enough to fill the GPU: column tiles that N fills
   if (!h.transB && !h.lower_only && h.N < 1024 &&
       ((int64_t)h.M + 127) / 128 * ((h.N + 111) / 112) * h.batch >= 512) {
-    const int fn = narrow_fn(h.N, h.K);
-    if (fn > 0)
-      return h.klass == MGW_KCLASS_GEMM_AO2MO ? launch_narrow<MGW_KCLASS_GEMM_AO2MO>(fn, h, stream)
-                                              : launch_narrow<MGW_KCLASS_GEMM_OTHER>(fn, h, stream);
-    cfg = 2;
+    fn = narrow_fn(h.N, h.K);
+    cfg = fn > 0 ? NCFG : 2;
   }
   Tuner& t = tuner();
-  const TuneKey key{h.klass, h.transA ? 1 : 0, h.transB ? 1 : 0, h.lower_only ? 1 : 0,
+  const TuneKey key{h.klass, h.transA ? 1 : 0, h.transB ? 1 : 0, fn > 0 ? TUNE_COLUMNS : h.lower_only ? 1 : 0,
                     log2_bucket(h.M), log2_bucket(h.N), log2_bucket((int64_t)h.K * h.batch)};
   bool need_tune = false;
   {
     std::lock_guard<std::mutex> lk(t.mu);
     load_table(t);
     auto it = t.table.find(key);
-    if (it != t.table.end() && it->second < NCFG) cfg = it->second;
+    if (it != t.table.end() && it->second < (fn > 0 ? NCFG + 1 : NCFG)) cfg = it->second;
     else need_tune = t.mode == 1 && h.beta == 0.0 && !h.no_tune;   // candidates overwrite C: only pure products
   }
   if (need_tune) {
     int best = cfg;
-    MGW_TRY(tune(h, stream, &best));
+    MGW_TRY(tune(h, fn, stream, &best));
     std::lock_guard<std::mutex> lk(t.mu);
     t.table[key] = best;
     cfg = best;
@@ -854,7 +859,7 @@ int gemm_f64(const GemmF64& h, hipStream_t stream) {
       }
     }
   }
-  return launch_by_class(cfg, h, stream);
+  return launch_by_class(cfg, fn, h, stream);
 }
 
 }  // namespace mgw

@@ -1,5 +1,6 @@
 """The tuner's table: entries of candidate lists that changed are not taken for
-the present ones."""
+the present ones, and the column tiles of products of few columns are tuned and
+looked up like any other."""
 import os
 import subprocess
 import sys
@@ -41,3 +42,32 @@ def test_entries_of_former_candidate_lists_are_not_used(tmp_path, family, nomega
     table.write_text(''.join(' '.join(map(str, r)) + '\n' for r in [r for r in rows if r[0] != family] + former))
     again = run(code, table)
     assert sorted(r[:7] for r in again[len(rows):]) == sorted(r[:7] for r in mine)
+
+
+def test_column_tiles_are_tuned(tmp_path):
+    """(P|m n) of a window of 16 states runs on column tiles: with tuning on
+    they are timed beside the other tiles and recorded, an entry is followed,
+    and every candidate gives the same numbers."""
+    table = tmp_path / 'tune.txt'
+    code = ('s = synthetic_system(177, 259, 9, seed=22, scale=0.3)\n'
+            'with Engine(0) as e:\n'
+            '    e.set_eri_3center(s.eri_3center, s.index_basis, s.nbf)\n'
+            '    e.set_mo(s.c_matrix, s.energy, s.occupation)\n'
+            '    ref = e.calculate_eri_3center_mo(1, 177, 2, 17)\n'
+            '    e.destroy_eri_3center_mo()\n'
+            '    e.set_mo(s.c_matrix, s.energy, s.occupation)\n'
+            '    autotune(%s)\n'
+            '    for _ in range(2):\n'
+            '        got = e.calculate_eri_3center_mo(1, 177, 2, 17)\n'
+            '        e.destroy_eri_3center_mo()\n'
+            '        e.set_mo(s.c_matrix, s.energy, s.occupation)\n'
+            '        assert np.array_equal(got, ref)\n')
+    table.touch()
+    rows = run(code % 'True', table)
+    # class AO2MO, list 2, floor(log2) of 259, 16 and 177 x 177
+    key = [0, 0, 0, 2, 8, 4, 14]
+    narrow = [r for r in rows if r[:7] == key]
+    assert len(narrow) == 1 and 0 <= narrow[0][7] < 5
+    for choice in range(5):
+        table.write_text(' '.join(map(str, key + [choice])) + '\n')
+        run(code % 'False', table)
