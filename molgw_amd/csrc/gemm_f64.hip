@@ -84,11 +84,11 @@ struct GemmDev {
   int upper_zero;      // lower_only: write zeros above the diagonal instead of the mirror
   int tri_a;           // A (not transposed) is lower triangular, zeros stored above the diagonal
   int batch_outer;     // walk the tiles of one batch entry before the next
-  int tiles_m, tiles_n, batch;
-  int64_t nblocks;
+  int tiles_m, tiles_n;
+  unsigned tiles, batch;      // tiles of one batch entry
   // the tiles (over all batch entries) behind the first `whole` take `splits`
   // workgroups of kchunk (a multiple of BK) along K each
-  int64_t whole, rest;
+  unsigned whole, rest;
   int splits, kchunk;
   double* part;        // splits > 1: part[tile - whole][split][n - n0][m - m0], else null
   const double* dotB; int64_t lddot;
@@ -134,10 +134,10 @@ __device__ inline void tile_origin(const GemmDev& g, int tile, int& m0, int& n0)
 // Tile and batch entry of the u-th tile over all batch entries: batch fastest
 // when the entries share operands (the frequencies of one chi0 tile read the
 // same panels), batch slowest when they do not.
-__device__ inline void tile_of_unit(const GemmDev& g, int64_t u, int& tile, int& batch) {
-  const int64_t per = (g.whole + g.rest) / g.batch;
-  batch = (int)(g.batch_outer ? u / per : u % g.batch);
-  tile = (int)(g.batch_outer ? u % per : u / g.batch);
+__device__ inline void tile_of_unit(const GemmDev& g, unsigned u, int& tile, int& batch) {
+  const unsigned d = g.batch_outer ? g.tiles : g.batch, q = u / d, r = u - q * d;
+  batch = (int)(g.batch_outer ? q : r);
+  tile = (int)(g.batch_outer ? r : q);
 }
 
 template <int BM, int BN, int WM, int WN, bool TA, bool TB, bool DOT, int KLASS>
@@ -170,9 +170,9 @@ gemm_f64_kernel(GemmDev g) {
   // logical block: the whole tiles, then the K splits of the others, one split
   // of all of them before the next (they share its range of the panels)
   const bool in_split = blockIdx.x >= g.whole;
-  const int64_t L = in_split ? xcd_logical(blockIdx.x - g.whole, g.nblocks - g.whole) : xcd_logical(blockIdx.x, g.whole);
+  const unsigned L = in_split ? xcd_logical32(blockIdx.x - g.whole, g.rest * g.splits) : xcd_logical32(blockIdx.x, g.whole);
   const int split = in_split ? (int)(L / g.rest) : 0;
-  const int64_t unit = in_split ? g.whole + L % g.rest : L;
+  const unsigned unit = in_split ? g.whole + L % g.rest : L;
   int tile, batch, m0, n0;
   tile_of_unit(g, unit, tile, batch);
   tile_origin<BM, BN>(g, tile, m0, n0);
@@ -439,7 +439,7 @@ gemm_f64_kernel(GemmDev g) {
   double* __restrict__ C = g.C + (int64_t)batch * g.strideC;
   const double* __restrict__ dg = g.diag_add ? g.diag_add + (int64_t)batch * g.strideDiag : nullptr;
   double* __restrict__ P =
-      in_split ? g.part + ((unit - g.whole) * g.splits + split) * (BM * BN) - (m0 + (int64_t)n0 * BM) : nullptr;
+      in_split ? g.part + ((int64_t)(unit - g.whole) * g.splits + split) * (BM * BN) - (m0 + (int64_t)n0 * BM) : nullptr;
 #pragma unroll
   for (int i = 0; i < FM; ++i) {
     const int m = m0 + wm * TM + i * 16 + fr;
@@ -493,7 +493,7 @@ int launch_cfg(const GemmF64& h, hipStream_t stream, int splits = 1, int64_t who
   g.batch_outer = h.batch_outer ? 1 : 0;
   g.tiles_m = (h.M + BM - 1) / BM;
   g.tiles_n = (h.N + BN - 1) / BN;
-  g.batch = h.batch;
+  g.batch = (unsigned)h.batch;
   g.dotB = h.dotB; g.lddot = h.lddot; g.dotpart = h.dotpart; g.strideDot = h.strideDot;
   g.dot_cc = h.dot_cc; g.dot_cd = h.dot_cd;
   g.dot_w = h.dot_w; g.strideDotW = h.strideDotW;
@@ -504,13 +504,13 @@ int launch_cfg(const GemmF64& h, hipStream_t stream, int splits = 1, int64_t who
   const int64_t units = tiles * h.batch;
   MGW_REQUIRE(units < (1ll << 31), MGW_ERR_ARG, "gemm_f64: too many tiles");
   g.splits = splits;
-  g.whole = splits > 1 ? whole : units;
-  g.rest = units - g.whole;
+  g.tiles = (unsigned)tiles;
+  g.whole = (unsigned)(splits > 1 ? whole : units);
+  g.rest = (unsigned)units - g.whole;
   g.kchunk = (int)(((h.K + (int64_t)splits - 1) / splits + BK - 1) / BK * BK);
   g.part = splits > 1 ? h.split_work : nullptr;
-  g.nblocks = g.whole + g.rest * splits;
   MGW_REQUIRE(h.batch >= 1, MGW_ERR_ARG, "gemm_f64: batch out of range");
-  dim3 grid((unsigned)g.nblocks, 1, 1);
+  dim3 grid(g.whole + g.rest * splits, 1, 1);
   dim3 block(64 * WM * WN, 1, 1);
   const int ta = h.transA ? 1 : 0, tb = h.transB ? 1 : 0;
 #define MGW_GEMM_CASE(TA_, TB_)                                                                        \
@@ -526,7 +526,7 @@ int launch_cfg(const GemmF64& h, hipStream_t stream, int splits = 1, int64_t who
   MGW_HIP(hipGetLastError());
   if constexpr (BM == BN && !DOT)
     if (splits > 1) {
-      hipLaunchKernelGGL(gemm_f64_reduce_kernel<BM>, dim3(BM * BM / 256, (unsigned)g.rest), dim3(256), 0,
+      hipLaunchKernelGGL(gemm_f64_reduce_kernel<BM>, dim3(BM * BM / 256, g.rest), dim3(256), 0,
                          stream, g);
       MGW_HIP(hipGetLastError());
     }

@@ -16,6 +16,13 @@ __device__ inline int64_t xcd_logical(int64_t w, int64_t G) {
   return (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + i;
 }
 
+// The same in 32 bits (64-bit divisions take a hundred instructions each).
+__device__ inline unsigned xcd_logical32(unsigned w, unsigned G) {
+  const unsigned q = G / NXCD, r = G % NXCD;
+  const unsigned x = w % NXCD, i = w / NXCD;
+  return (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + i;
+}
+
 // Lower-triangle tile t (0-based, of T x T tiles) -> (bm, bn), bm >= bn, in a
 // grouped order: super-rows of TRI_GROUP tile rows, walked column by column,
 // so that concurrent workgroups share TRI_GROUP row panels and few column
