@@ -474,7 +474,12 @@ __global__ void __launch_bounds__(256) gemm_f64_reduce_kernel(GemmDev g) {
                g.diag_add ? g.diag_add + (int64_t)batch * g.strideDiag : nullptr, m, n, s);
 }
 
-// NB: B not transposed only (column tiles that are no power of two)
+// Column tiles (NB): B not transposed only, and of each class the form of A that
+// occurs; the other forms run under the symbol of GEMM_OTHER
+constexpr bool narrow_form(int klass, bool ta) {
+  return klass == MGW_KCLASS_GEMM_OTHER || klass == MGW_KCLASS_GEMM_SIGMA ? klass == MGW_KCLASS_GEMM_OTHER || ta : !ta;
+}
+
 template <int BM, int BN, int WM, int WN, bool DOT, int KLASS, bool NB = false>
 int launch_cfg(const GemmF64& h, hipStream_t stream, int splits = 1, int64_t whole = 0) {
   GemmDev g;
@@ -514,7 +519,7 @@ int launch_cfg(const GemmF64& h, hipStream_t stream, int splits = 1, int64_t who
   dim3 block(64 * WM * WN, 1, 1);
   const int ta = h.transA ? 1 : 0, tb = h.transB ? 1 : 0;
 #define MGW_GEMM_CASE(TA_, TB_)                                                                        \
-  if constexpr (!(NB && TB_))                                                                          \
+  if constexpr (!NB || (!TB_ && narrow_form(KLASS, TA_)))                                              \
     if (ta == TA_ && tb == TB_)                                                                        \
       hipLaunchKernelGGL((gemm_f64_kernel<BM, BN, WM, WN, TA_, TB_, DOT, KLASS>), grid, block, 0,      \
                          stream, g);
@@ -543,15 +548,15 @@ int gemm_f64_dot_rowblocks(int M) { return (M + 63) / 64; }
 // ------------------------------------------------------------------ autotuner
 // Candidate tile configurations (all FP64 MFMA, BK = 16):
 //   0: 256x128, 16 waves   1: 128x128, 8 waves   2: 128x128, 4 waves   3: 64x64, 4 waves
-//   4: 128 x 16 FN, 4 waves (products of few columns only)
-// The defaults (2, 3 for small products, 4 for few columns) were measured on
+//      128 x 16 fn, 4 waves, for products of few columns
+// The defaults (split_plan's 2 or 3; column_tiles' 0, 2 or 3) were measured on
 // MI355X. With tuning on, the first product of a new (class, transposes, lower
 // or few columns, log2 M/N/K bucket) times every candidate on
 // the actual operands and keeps the fastest; the table can be persisted.
 namespace {
 
 constexpr int NCFG = 4;
-constexpr int TUNE_COLUMNS = 2;    // products that column tiles are the default of, candidate NCFG
+constexpr int TUNE_COLUMNS = 2;    // products of few columns: candidate 0 is their column tiles
 constexpr int TUNE_SPLIT = 4;      // products with a split K, of candidates of their own
 
 struct TuneKey {
@@ -605,21 +610,48 @@ int launch_candidate(int cfg, const GemmF64& h, hipStream_t stream) {
   }
 }
 
-// Column tiles of 16 FN < 128 columns for products of few columns (the
-// transforms of the occupied states or of a window, the exchange's half
-// transform): the FN whose tiles cover N in the least time, 0 when 128-column
-// tiles do. In units of 16 columns at 1 TFLOP/s, measured at 65536 x 16 FN x
-// 4096: FN = 1 .. 6 and 8 run at 23, 38, 42, 48, 58, 53 and 65 TFLOP/s (up to 3
-// the rows' traffic bounds them; 112 columns, at 56, always cost more than
-// 128); a workgroup's fixed cost is that of 60 k, or of 150 for 128 columns, of
-// which only two share a CU.
-int narrow_fn(int N, int K) {
-  constexpr double w[9] = {0.0, 1 / 23.0, 2 / 38.0, 3 / 42.0, 4 / 48.0, 5 / 58.0, 6 / 53.0, 0.0, 8 / 65.0};
-  auto cost = [&](int fn) { return (N + 16 * fn - 1) / (16 * fn) * w[fn] * (K + (fn == 8 ? 150.0 : 60.0)); };
-  int best = 8;
-  for (int fn = 6; fn >= 1; --fn)
-    if (cost(fn) < cost(best)) best = fn;
-  return best == 8 ? 0 : best;
+// Tiles of a product of few columns (the transforms, half transforms and
+// self-energy products of a window of states, the blocks of a factorisation): 128
+// rows by 16 fn columns (cfg 0), 64x64 (cfg 3) or 128x128 (cfg 2), whichever is
+// estimated to take the least time; fn: the best of the column tiles.
+//
+// A round of workgroups, `share` per CU, takes (K + fixed) steps, each at the
+// tile's rate; the last round costs 0.15 and a part for the workgroups it has, a
+// lone one 0.33. Rates (TFLOP/s of the tile's area), fixed costs and these parts
+// are fitted to the times of 965 products on random operands: both transforms and
+// the half transform of 50 to 768 functions, 75 to 2688 auxiliary ones and 1 to 768
+// states, self-energy and factorisation products, 65536 rows with K to 4096. Over
+// them the estimate's choice takes 0.6 % more than the best tile on average and
+// 18 % at most. By rows of 128 and the columns' fit alone, with 64x64 below 512
+// workgroups, it was 15 % on average and up to 89 %: rows past the edge, few full
+// rounds and a lone workgroup's latency count as much as columns. 64x64 tiles read
+// their operands twice as often and end at 8 rounds (up to 19 % off beyond).
+void column_tiles(const GemmF64& h, int* cfg, int* fn) {
+  struct Tile {
+    int cfg, bm, bn, share;
+    double rate, fixed;
+  };
+  static constexpr Tile TILES[] = {{2, 128, 128, 2, 70.4, 126.0}, {3, 64, 64, 4, 63.9, 84.8},
+                                   {0, 128, 16, 4, 43.0, 31.6}, {0, 128, 32, 4, 52.7, 43.0},
+                                   {0, 128, 48, 4, 65.7, 78.9}, {0, 128, 64, 4, 66.2, 88.7},
+                                   {0, 128, 80, 3, 68.9, 96.2}};
+  double best = 0.0, best_columns = 0.0;
+  for (const Tile& t : TILES) {
+    const int64_t wgs = (int64_t)((h.M + t.bm - 1) / t.bm) * ((h.N + t.bn - 1) / t.bn) * h.batch;
+    const int64_t slots = 256 * t.share, full = wgs / slots;
+    if (t.cfg == 3 && full >= 8) continue;
+    const double part = (double)(wgs % slots) / slots;
+    const double rounds = full == 0 ? 0.33 + 0.67 * part : full + (part > 0.0 ? 0.15 + 0.85 * part : 0.0);
+    const double cost = (double)t.bm * t.bn * slots / t.rate * (h.K + t.fixed) * rounds;
+    if (best == 0.0 || cost < best) {
+      best = cost;
+      *cfg = t.cfg;
+    }
+    if (t.cfg == 0 && (best_columns == 0.0 || cost < best_columns)) {
+      best_columns = cost;
+      *fn = t.bn / 16;
+    }
+  }
 }
 
 template <int KLASS>
@@ -629,17 +661,24 @@ int launch_narrow(int fn, const GemmF64& h, hipStream_t stream) {
     case 2: return launch_cfg<128, 32, 4, 1, false, KLASS, true>(h, stream);
     case 3: return launch_cfg<128, 48, 4, 1, false, KLASS, true>(h, stream);
     case 4: return launch_cfg<128, 64, 2, 2, false, KLASS, true>(h, stream);
-    case 5: return launch_cfg<128, 80, 4, 1, false, KLASS, true>(h, stream);
-    default: return launch_cfg<128, 96, 2, 2, false, KLASS, true>(h, stream);
+    default: return launch_cfg<128, 80, 4, 1, false, KLASS, true>(h, stream);
   }
 }
 
-// cfg NCFG: column tiles of 16 fn (kernels of classes other than AO2MO carry the
-// symbol of GEMM_OTHER there, and a profile counts them to it)
+// fn > 0: cfg 0 is the column tiles of 16 fn. Of the classes, only the forms that occur have
+// kernels of their own there (narrow_form).
 int launch_by_class(int cfg, int fn, const GemmF64& h, hipStream_t stream) {
-  if (cfg == NCFG)
-    return h.klass == MGW_KCLASS_GEMM_AO2MO ? launch_narrow<MGW_KCLASS_GEMM_AO2MO>(fn, h, stream)
-                                            : launch_narrow<MGW_KCLASS_GEMM_OTHER>(fn, h, stream);
+  if (fn > 0 && cfg == 0) {
+    if (narrow_form(h.klass, h.transA)) {
+      switch (h.klass) {
+        case MGW_KCLASS_GEMM_AO2MO: return launch_narrow<MGW_KCLASS_GEMM_AO2MO>(fn, h, stream);
+        case MGW_KCLASS_GEMM_CASIDA: return launch_narrow<MGW_KCLASS_GEMM_CASIDA>(fn, h, stream);
+        case MGW_KCLASS_GEMM_SIGMA: return launch_narrow<MGW_KCLASS_GEMM_SIGMA>(fn, h, stream);
+        case MGW_KCLASS_CHOLESKY: return launch_narrow<MGW_KCLASS_CHOLESKY>(fn, h, stream);
+      }
+    }
+    return launch_narrow<MGW_KCLASS_GEMM_OTHER>(fn, h, stream);
+  }
   switch (h.klass) {
     case MGW_KCLASS_GEMM_AO2MO: return launch_candidate<MGW_KCLASS_GEMM_AO2MO>(cfg, h, stream);
     case MGW_KCLASS_GEMM_CASIDA: return launch_candidate<MGW_KCLASS_GEMM_CASIDA>(cfg, h, stream);
@@ -726,7 +765,7 @@ int tune(const GemmF64& h, int fn, hipStream_t stream, int* best) {
   MGW_HIP(hipEventCreate(&b));
   float best_ms = 1e30f;
   *best = -1;
-  for (int cfg = 0; cfg < (fn > 0 ? NCFG + 1 : NCFG); ++cfg) {
+  for (int cfg = 0; cfg < NCFG; ++cfg) {
     MGW_HIP(hipEventRecord(a, stream));
     MGW_TRY(launch_by_class(cfg, fn, h, stream));
     MGW_HIP(hipEventRecord(b, stream));
@@ -828,12 +867,7 @@ int gemm_f64(const GemmF64& h, hipStream_t stream) {
   const SplitPlan plan = split_plan(h.M, h.N, h.K, h.batch, h.lower_only, h.split_work != nullptr);
   if (plan.splits > 1) return launch_split(plan, h, stream);
   int cfg = plan.b == 64 ? 3 : 2, fn = 0;
-  // few columns, and rows enough to fill the GPU: column tiles that N fills
-  if (!h.transB && !h.lower_only && h.N < 1024 &&
-      ((int64_t)h.M + 127) / 128 * ((h.N + 111) / 112) * h.batch >= 512) {
-    fn = narrow_fn(h.N, h.K);
-    cfg = fn > 0 ? NCFG : 2;
-  }
+  if (!h.transB && !h.lower_only && h.N < 1024) column_tiles(h, &cfg, &fn);
   Tuner& t = tuner();
   const TuneKey key{h.klass, h.transA ? 1 : 0, h.transB ? 1 : 0, fn > 0 ? TUNE_COLUMNS : h.lower_only ? 1 : 0,
                     log2_bucket(h.M), log2_bucket(h.N), log2_bucket((int64_t)h.K * h.batch)};
@@ -842,7 +876,7 @@ int gemm_f64(const GemmF64& h, hipStream_t stream) {
     std::lock_guard<std::mutex> lk(t.mu);
     load_table(t);
     auto it = t.table.find(key);
-    if (it != t.table.end() && it->second < (fn > 0 ? NCFG + 1 : NCFG)) cfg = it->second;
+    if (it != t.table.end() && it->second < NCFG) cfg = it->second;
     else need_tune = t.mode == 1 && h.beta == 0.0 && !h.no_tune;   // candidates overwrite C: only pure products
   }
   if (need_tune) {

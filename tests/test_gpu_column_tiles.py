@@ -1,7 +1,9 @@
-"""The AO->MO transform's column tiles of 16 FN columns: windows at and beside
-the tiles' edges for every FN that the rule picks. Bound: a sum of K products
-in any order is off by at most K 2^-53 sum |a b|, here K = nbf twice, and twice
-that for the two sides' roundings."""
+"""The AO->MO transform of windows at and beside the edges of every tile that the
+rule for few columns picks. Bound: a sum of K products in any order is off by at
+most K 2^-53 sum |a b|, here K = nbf twice, and twice that for the two sides'
+roundings."""
+import functools
+
 import numpy as np
 import pytest
 
@@ -10,42 +12,55 @@ from molgw_amd.workloads import dense_ri, synthetic_system
 
 pytestmark = pytest.mark.gpu
 EPS = 2.0 ** -53
-NBF, NAUX = 177, 259       # 3 row tiles x 177 products: past the 512 workgroups that the column tiles ask for
 
 
-def column_tile(n, k):
-    """The rule of narrow_fn (gemm_f64.hip); 0 for the 128-wide tiles."""
-    weight = {1: 1 / 23, 2: 2 / 38, 3: 3 / 42, 4: 4 / 48, 5: 5 / 58, 6: 6 / 53, 8: 8 / 65}
-    cost = {fn: -(-n // (16 * fn)) * w * (k + (150 if fn == 8 else 60)) for fn, w in weight.items()}
-    best = min(sorted(cost, reverse=True), key=lambda fn: cost[fn])
-    return 0 if best == 8 else best
+def chosen_tile(m, n, k):
+    """(rows, columns) of the tile that column_tiles (gemm_f64.hip) picks."""
+    tiles = [(128, 128, 2, 70.4, 126), (64, 64, 4, 63.9, 84.8), (128, 16, 4, 43.0, 31.6), (128, 32, 4, 52.7, 43),
+             (128, 48, 4, 65.7, 78.9), (128, 64, 4, 66.2, 88.7), (128, 80, 3, 68.9, 96.2)]
+
+    def cost(tile):
+        bm, bn, share, rate, fixed = tile
+        full, last = divmod(-(-m // bm) * -(-n // bn), 256 * share)
+        if bm == 64 and full >= 8:
+            return float('inf')
+        part = last / (256 * share)
+        rounds = 0.33 + 0.67 * part if full == 0 else full + (0.15 + 0.85 * part if last else 0.0)
+        return bm * bn * 256 * share / rate * (k + fixed) * rounds
+    return min(tiles, key=cost)[:2]
 
 
-@pytest.fixture(scope='module')
-def loaded():
-    s = synthetic_system(NBF, NAUX, 9, seed=22, scale=0.3)
-    with Engine(0) as e:
-        e.set_eri_3center(s.eri_3center, s.index_basis, s.nbf)
-        e.set_mo(s.c_matrix, s.energy, s.occupation)
-        yield e, s, dense_ri(s)
+@functools.lru_cache(maxsize=1)
+def system(nbf, naux):
+    s = synthetic_system(nbf, naux, 9, seed=22, scale=0.3)
+    return s, dense_ri(s)
 
 
-@pytest.mark.parametrize('ncol, fn', [(1, 1), (15, 1), (16, 1), (17, 2), (31, 2), (32, 2), (33, 3), (47, 3), (48, 3),
-                                      (49, 4), (64, 4), (65, 5), (79, 5), (80, 5), (81, 6), (95, 6), (96, 6), (97, 4),
-                                      (112, 4), (129, 5), (161, 6), (176, 6)])
-def test_every_column_tile(loaded, ncol, fn):
-    eng, s, b = loaded
-    assert column_tile(ncol, NBF) == fn and -(-NAUX // 128) * -(-ncol // 112) * NBF >= 512
-    eng.destroy_eri_3center_mo()
-    got = eng.calculate_eri_3center_mo(1, s.nstate, 2, ncol + 1)
-    eng.destroy_eri_3center_mo()
+SMALL, LARGE, LARGER = (131, 129), (177, 371), (309, 637)
+WINDOWS = [(*SMALL, n) for n in (1, 15, 16, 17, 31, 33, 64, 65, 130)] + [
+    (*LARGE, n) for n in (1, 16, 17, 32, 33, 47, 48, 49, 63, 64, 65, 79, 80, 81, 95, 96, 97, 112, 129, 144, 161, 176)] + [
+    (*LARGER, n) for n in (49, 64)]
+
+
+@pytest.mark.parametrize('nbf, naux, ncol', WINDOWS)
+def test_windows(nbf, naux, ncol):
+    s, b = system(nbf, naux)
     c = s.c_matrix
-    ref = np.einsum('pkn,km->pmn', b @ c[:, 1:ncol + 1], c, optimize=True)
-    size = np.einsum('pkn,km->pmn', np.abs(b) @ np.abs(c[:, 1:ncol + 1]), np.abs(c), optimize=True)
+    with Engine(0) as eng:
+        eng.set_eri_3center(s.eri_3center, s.index_basis, s.nbf)
+        eng.set_mo(s.c_matrix, s.energy, s.occupation)
+        got = eng.calculate_eri_3center_mo(1, s.nstate, 2, ncol + 1)
+    if naux > 500:      # rows of the first and last tiles
+        rows = np.r_[0:130, naux - 130:naux]
+        b, got = b[rows], got[rows]
+    half, size = b @ c[:, 1:ncol + 1], np.abs(b) @ np.abs(c[:, 1:ncol + 1])
+    ref = np.einsum('pkn,km->pmn', half, c, optimize=True)
+    size = np.einsum('pkn,km->pmn', size, np.abs(c), optimize=True)
     assert np.all(np.abs(got - ref) <= 4 * s.nbf * EPS * size)
 
 
-def test_no_shape_takes_a_seventh_tile():
-    """112 columns cost more than 128 (a column at 56 against 65 TFLOP/s), so
-    the tiles end at 96."""
-    assert {column_tile(n, k) for n in range(1, 1024) for k in (16, 60, 177, 1000, 10 ** 5)} == set(range(7))
+def test_windows_reach_every_tile():
+    """Of few columns; 128 x 128 is the tile of every larger product."""
+    first = {chosen_tile(nbf * naux, n, nbf) for nbf, naux, n in WINDOWS}
+    assert first >= {(128, 16 * fn) for fn in range(1, 6)} | {(64, 64)}
+    assert chosen_tile(10 ** 6, 128, 2000) == (128, 128)

@@ -49,7 +49,7 @@ def test_column_tiles_are_tuned(tmp_path):
     they are timed beside the other tiles and recorded, an entry is followed,
     and every candidate gives the same numbers."""
     table = tmp_path / 'tune.txt'
-    code = ('s = synthetic_system(177, 259, 9, seed=22, scale=0.3)\n'
+    code = ('s = synthetic_system(177, 371, 9, seed=22, scale=0.3)\n'
             'with Engine(0) as e:\n'
             '    e.set_eri_3center(s.eri_3center, s.index_basis, s.nbf)\n'
             '    e.set_mo(s.c_matrix, s.energy, s.occupation)\n'
@@ -64,10 +64,10 @@ def test_column_tiles_are_tuned(tmp_path):
             '        assert np.array_equal(got, ref)\n')
     table.touch()
     rows = run(code % 'True', table)
-    # class AO2MO, list 2, floor(log2) of 259, 16 and 177 x 177
-    key = [0, 0, 0, 2, 8, 4, 14]
+    # class AO2MO, few columns, floor(log2) of 371 x 177, 16 and 177
+    key = [0, 0, 0, 2, 16, 4, 7]
     narrow = [r for r in rows if r[:7] == key]
-    assert len(narrow) == 1 and 0 <= narrow[0][7] < 5
-    for choice in range(5):
+    assert len(narrow) == 1 and 0 <= narrow[0][7] < 4
+    for choice in range(4):
         table.write_text(' '.join(map(str, key + [choice])) + '\n')
         run(code % 'False', table)
