@@ -625,7 +625,8 @@ int launch_candidate(int cfg, const GemmF64& h, hipStream_t stream) {
 // 18 % at most. By rows of 128 and the columns' fit alone, with 64x64 below 512
 // workgroups, it was 15 % on average and up to 89 %: rows past the edge, few full
 // rounds and a lone workgroup's latency count as much as columns. 64x64 tiles read
-// their operands twice as often and end at 8 rounds (up to 19 % off beyond).
+// their operands twice as often and end at 8 rounds (up to 19 % off beyond); 96
+// columns pay for a long K (2064384 x 90 x 768: 5.9 ms, 6.3 on tiles of 48).
 void column_tiles(const GemmF64& h, int* cfg, int* fn) {
   struct Tile {
     int cfg, bm, bn, share;
@@ -634,7 +635,7 @@ void column_tiles(const GemmF64& h, int* cfg, int* fn) {
   static constexpr Tile TILES[] = {{2, 128, 128, 2, 70.4, 126.0}, {3, 64, 64, 4, 63.9, 84.8},
                                    {0, 128, 16, 4, 43.0, 31.6}, {0, 128, 32, 4, 52.7, 43.0},
                                    {0, 128, 48, 4, 65.7, 78.9}, {0, 128, 64, 4, 66.2, 88.7},
-                                   {0, 128, 80, 3, 68.9, 96.2}};
+                                   {0, 128, 80, 3, 68.9, 96.2}, {0, 128, 96, 3, 67.0, 95.0}};
   double best = 0.0, best_columns = 0.0;
   for (const Tile& t : TILES) {
     const int64_t wgs = (int64_t)((h.M + t.bm - 1) / t.bm) * ((h.N + t.bn - 1) / t.bn) * h.batch;
@@ -661,7 +662,8 @@ int launch_narrow(int fn, const GemmF64& h, hipStream_t stream) {
     case 2: return launch_cfg<128, 32, 4, 1, false, KLASS, true>(h, stream);
     case 3: return launch_cfg<128, 48, 4, 1, false, KLASS, true>(h, stream);
     case 4: return launch_cfg<128, 64, 2, 2, false, KLASS, true>(h, stream);
-    default: return launch_cfg<128, 80, 4, 1, false, KLASS, true>(h, stream);
+    case 5: return launch_cfg<128, 80, 4, 1, false, KLASS, true>(h, stream);
+    default: return launch_cfg<128, 96, 2, 2, false, KLASS, true>(h, stream);
   }
 }
 
