@@ -8,13 +8,14 @@ is filtered by the overlap eigenvalues (setup_x_matrix,
 src/m_hamiltonian_tools.f90:1171-1219, min_overlap 1e-5), the metric by
 eigenvalues above 1e-6 (src/m_eri_calculate.f90:1049-1262), and the pair
 tensor carries the 1/2 on diagonal pairs (src/m_eri_calculate.f90:1840-1841).
-The SCF itself is a textbook closed-shell Roothaan-Hall iteration with DIIS
-from the core-Hamiltonian guess; at convergence its energy and orbitals are
-those of any converged RI-HF run.
+The SCF itself is a textbook closed-shell Roothaan-Hall iteration from the
+core-Hamiltonian guess, by optimal damping and then DIIS; at convergence its
+energy and orbitals are those of any converged RI-HF run.
 """
 from __future__ import annotations
 
 import math
+import warnings
 from dataclasses import dataclass
 
 import numpy as np
@@ -84,6 +85,62 @@ class RIHFResult:
     index_basis: np.ndarray     # (2, npair), 1-based
     nbf: int
     iterations: int
+    converged: bool = True
+
+
+class _NextFock:
+    """The Fock matrix to diagonalise next, from a density (of orbitals), its Fock
+    matrix and their commutator in the orthonormal basis.
+
+    While the commutator is FAR or more: optimal damping (Cances and Le Bris,
+    Int. J. Quantum Chem. 79, 82 (2000)). A mixed density takes the step towards
+    the new one that minimises the energy, which is quadratic in the density,
+    so the mixed density's energy never rises. Then DIIS over the last densities.
+    DIIS alone wandered from the core-Hamiltonian guess of long alkanes, which
+    has no gap: C18H38 took 51 to 64 iterations, or did not converge in 100,
+    depending on the last bits of the integrals; this way 21."""
+
+    FAR = 0.1
+
+    def __init__(self, diis: int):
+        self.diis = diis
+        self.mixed = None               # density and Fock matrix of the damped steps
+        self.fs, self.errs = [], []
+
+    def __call__(self, d, f, err):
+        if np.abs(err).max() >= self.FAR:
+            self.fs, self.errs = [], []
+            if self.mixed is None:
+                self.mixed = d, f
+            else:
+                dm, fm = self.mixed
+                slope, curvature = np.sum(fm * (d - dm)), np.sum((d - dm) * (f - fm))
+                step = min(1.0, -slope / curvature) if curvature > 0.0 and slope < 0.0 else 1.0
+                self.mixed = dm + step * (d - dm), fm + step * (f - fm)
+            return self.mixed[1]
+        self.mixed = None
+        self.fs.append(f)
+        self.errs.append(err)
+        if len(self.fs) > self.diis:
+            self.fs.pop(0)
+            self.errs.pop(0)
+        nd = len(self.fs)
+        if nd < 2:
+            return f
+        bm = -np.ones((nd + 1, nd + 1))
+        bm[nd, nd] = 0.0
+        for a in range(nd):
+            for b in range(nd):
+                bm[a, b] = np.sum(self.errs[a] * self.errs[b])
+        rhs = np.zeros(nd + 1)
+        rhs[nd] = -1.0
+        coef = np.linalg.solve(bm, rhs)[:nd]
+        return sum(cf * ff for cf, ff in zip(coef, self.fs))
+
+
+def _warn_unless(converged: bool, it: int, err: float) -> None:
+    if not converged:
+        warnings.warn(f'RI-HF not converged in {it} iterations (commutator {err:.1e})', stacklevel=3)
 
 
 def _pack(eri3: np.ndarray, index_basis: np.ndarray) -> np.ndarray:
@@ -140,35 +197,19 @@ def run_rihf(mol: Molecule, basis: str, auxil_basis: str, basis_dir: str, gaussi
     eps, c = solve(h)
     d = 2.0 * c[:, :nocc] @ c[:, :nocc].T
     e_old = 0.0
-    fs, errs = [], []
-    it = 0
+    next_fock = _NextFock(diis)
+    converged, it, err = False, 0, np.inf
     for it in range(1, max_iter + 1):
         f, j, k = fock(d)
         energy = 0.5 * np.sum(d * (h + f)) + enuc
         err = x.T @ (f @ d @ s - s @ d @ f) @ x
-        fs.append(f)
-        errs.append(err)
-        if len(fs) > diis:
-            fs.pop(0)
-            errs.pop(0)
-        if len(fs) > 1:
-            nd = len(fs)
-            bm = -np.ones((nd + 1, nd + 1))
-            bm[nd, nd] = 0.0
-            for a_ in range(nd):
-                for b_ in range(nd):
-                    bm[a_, b_] = np.sum(errs[a_] * errs[b_])
-            rhs = np.zeros(nd + 1)
-            rhs[nd] = -1.0
-            coef = np.linalg.solve(bm, rhs)[:nd]
-            f_use = sum(cf * ff for cf, ff in zip(coef, fs))
-        else:
-            f_use = f
-        eps, c = solve(f_use)
+        eps, c = solve(next_fock(d, f, err))
         d = 2.0 * c[:, :nocc] @ c[:, :nocc].T
         if abs(energy - e_old) < tol and np.abs(err).max() < 1e-7:
+            converged = True
             break
         e_old = energy
+    _warn_unless(converged, it, np.abs(err).max())
     # final orbitals from the converged Fock matrix itself
     f, j, k = fock(d)
     eps, c = solve(f)
@@ -181,7 +222,7 @@ def run_rihf(mol: Molecule, basis: str, auxil_basis: str, basis_dir: str, gaussi
     occ = np.zeros(nstate)
     occ[:nocc] = 2.0
     ib = upper_pairs(bs.nbf)
-    return RIHFResult(float(energy), comps, c, eps, occ, _pack(e3, ib), m2, ib, bs.nbf, it)
+    return RIHFResult(float(energy), comps, c, eps, occ, _pack(e3, ib), m2, ib, bs.nbf, it, converged)
 
 
 @dataclass
@@ -201,6 +242,7 @@ class DeviceRIHF:
     naux: int                   # kept auxiliary functions
     naux_bas: int
     iterations: int
+    converged: bool = True
 
     @property
     def nstate(self) -> int:
@@ -253,35 +295,19 @@ def run_rihf_device(mol: Molecule, basis: str, auxil_basis: str, basis_dir: str,
 
     eps, c = solve(h)
     e_old = 0.0
-    fs, errs = [], []
-    it = 0
+    next_fock = _NextFock(diis)
+    converged, it, err = False, 0, np.inf
     for it in range(1, max_iter + 1):
         d = 2.0 * c[:, :nocc] @ c[:, :nocc].T
         f, j, kx = fock(c)
         energy = 0.5 * np.sum(d * (h + f)) + enuc
         err = x.T @ (f @ d @ s - s @ d @ f) @ x
-        fs.append(f)
-        errs.append(err)
-        if len(fs) > diis:
-            fs.pop(0)
-            errs.pop(0)
-        if len(fs) > 1:
-            nd = len(fs)
-            bm = -np.ones((nd + 1, nd + 1))
-            bm[nd, nd] = 0.0
-            for a_ in range(nd):
-                for b_ in range(nd):
-                    bm[a_, b_] = np.sum(errs[a_] * errs[b_])
-            rhs = np.zeros(nd + 1)
-            rhs[nd] = -1.0
-            coef = np.linalg.solve(bm, rhs)[:nd]
-            f_use = sum(cf * ff for cf, ff in zip(coef, fs))
-        else:
-            f_use = f
-        eps, c = solve(f_use)
+        eps, c = solve(next_fock(d, f, err))
         if abs(energy - e_old) < tol and np.abs(err).max() < 1e-7:
+            converged = True
             break
         e_old = energy
+    _warn_unless(converged, it, np.abs(err).max())
     # final orbitals from the Fock matrix of the converged density itself
     f, j, kx = fock(c)
     eps, c = solve(f)
@@ -293,7 +319,7 @@ def run_rihf_device(mol: Molecule, basis: str, auxil_basis: str, basis_dir: str,
              'nucleus_nucleus': enuc}
     occ = np.zeros(nstate)
     occ[:nocc] = 2.0
-    return DeviceRIHF(float(energy), comps, c, eps, occ, f, s, ib, bs.nbf, kept, aux.nbf, it)
+    return DeviceRIHF(float(energy), comps, c, eps, occ, f, s, ib, bs.nbf, kept, aux.nbf, it, converged)
 
 
 def water_cluster(m: int, seed: int = 0, oo_min: float = 2.7, volume_per_molecule: float = 45.0,
