@@ -37,7 +37,10 @@
 // Boys function: F_L(T) by a 7-term Taylor series around the nearest point
 // of a table F_n(k h), h = 0.05, T <= 36 (error below 2e-15 relative), then
 // downward recursion; above T = 36, F_0 = sqrt(pi / T) / 2 (the neglected
-// tail is e^-T < 3e-16) and upward recursion.
+// tail is e^-T < 3e-16) and upward recursion. The recursions' divisions are
+// products with a reciprocal and a correction by the residual, as accurate as
+// divisions (0.3 % of the alkane's time; without it the rounding of the one
+// reciprocal adds up over the orders, 2.2 -> 5.3e-16 for F_10).
 #pragma once
 #include "mgw_internal.h"
 
@@ -132,6 +135,14 @@ struct EriArgs {
   double* out;
 };
 
+// a / b for a given rounded r = 1 / b: one product and the residual's correction,
+// as accurate as a division; r alone would leave its own rounding in every
+// order of the recursions below
+__device__ inline double corrected_quotient(double a, double b, double r) {
+  const double q = a * r;
+  return fma(fma(-b, q, a), r, q);
+}
+
 template <int L>
 __device__ inline void boys_eval(double T, const double* __restrict__ tab, double* f) {
   if (T < BOYS_TMAX) {
@@ -145,12 +156,13 @@ __device__ inline void boys_eval(double T, const double* __restrict__ tab, doubl
     f[L] = s;
     const double e = exp(-T);
 #pragma unroll
-    for (int n = L - 1; n >= 0; --n) f[n] = (2.0 * T * f[n + 1] + e) * (1.0 / (double)(2 * n + 1));
+    for (int n = L - 1; n >= 0; --n)
+      f[n] = corrected_quotient(2.0 * T * f[n + 1] + e, (double)(2 * n + 1), 1.0 / (double)(2 * n + 1));
   } else {
     const double e = exp(-T), h = 0.5 / T;
-    f[0] = 0.5 * sqrt(6.28318530717958647693 * h);
+    f[0] = 0.5 * sqrt(corrected_quotient(6.28318530717958647693, 2.0 * T, h));
 #pragma unroll
-    for (int n = 0; n < L; ++n) f[n + 1] = ((double)(2 * n + 1) * f[n] - e) * h;
+    for (int n = 0; n < L; ++n) f[n + 1] = corrected_quotient((double)(2 * n + 1) * f[n] - e, 2.0 * T, h);
   }
 }
 
