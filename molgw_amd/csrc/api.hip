@@ -939,7 +939,7 @@ int polarizability_grid(mgw_ctx* c, const mgw_ranges* r, double spin_fact, int n
     } else {
       MGW_TRY(plus_one());
       // K split of the last round's tiles, which would leave the GPU mostly idle
-      // (naux 1372, 21385 transitions, 32 frequencies: 30.7 -> 26.5 ms)
+      // (naux 1372, 21385 transitions, 32 frequencies: 30.7 -> 25.7 ms)
       if (g.precision == MGW_FP64)
         MGW_TRY(dbuf_if_room(c, "chi_ksplit", gemm_f64_split_doubles(naux, naux, npole, nomega, true), &g.split_work));
       const int rc = gemm_f64(g, c->stream);

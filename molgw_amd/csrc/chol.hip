@@ -735,10 +735,10 @@ int plane_gemm(const CholCtx& c, const Fp16Planes& da, const _Float16* pa, int a
 //   [A21 A22]   A22 -= L21 L21^T, factor and invert A22 (recursion),
 //               (L^-1)21 = -(L^-1)22 L21 (L^-1)11.
 // The products are batched MFMA GEMMs (FP64, or FP16x3 on planes for the
-// large levels when the factorisation has operand bounds); the leaves
-// are factored and inverted by chol_block_kernel (or chol_diag_kernel). `w` is this block's work (chol_need(m) doubles per
-// matrix, matrix stride c.sw); `l21_off` the L21-plane stack used by the
-// enclosing levels (elements per matrix).
+// large levels when the factorisation has operand bounds); the leaves are
+// factored and inverted by chol_block_kernel (or chol_diag_kernel). `w` is this
+// block's work (chol_need(m) doubles per matrix, matrix stride c.sw); `l21_off` the
+// L21-plane stack used by the enclosing levels (elements per matrix).
 int chol_rec(const CholCtx& c, int k0, int m, double* w, int64_t l21_off) {
   const int n = c.n;
   const int64_t s2 = (int64_t)n * n;

@@ -229,7 +229,8 @@ bool chol_epi_planes();
 bool chol_leaf_block();
 int chol_inverse_batched(double* A, int n, int nbatch, double* logdet, int32_t* info, double* work,
                          hipStream_t stream, double* bounds = nullptr, void* planes = nullptr);
-// tr[f] = sum of squares of the lower triangle of M_f (n x n, stride n^2).
+// Partial sums (FROB_BLOCKS per matrix) of the squares of the lower triangle of
+// M_f (n x n, stride n^2), whose diagonal then grows by diag_add.
 int launch_lower_frob2(double* m, int n, int nbatch, double diag_add, double* partial, hipStream_t s);
 constexpr int FROB_BLOCKS = 64;
 int gemm_autotune_mode(int mode); // -1 query; returns the previous mode
@@ -333,7 +334,8 @@ int launch_hartree_gamma(const double* h, const double* x, int naux, int nbf, in
                          double* gamma, hipStream_t s);
 // j(k, l) = j(l, k) = sum_P B(P, k, l) gamma(P) for B symmetric in (k, l)
 int launch_hartree_j(const double* b, const double* gamma, int naux, int nbf, double* j, hipStream_t s);
-// out(e) (+)= sum_b m(e + n b) over b < nbatch, in order
+// out(e) (+)= sum_b m(e + n b) over b < nbatch, in a fixed order (every fourth b, then
+// the four sums)
 int launch_batch_sum(const double* m, int64_t n, int nbatch, int accumulate, double* out, hipStream_t s);
 int launch_sigma_poles(const double* w, int npole, int nse, int ni, const double* pole,
                        const double* omega, int nomega, const double* e0p, const double* ei,
