@@ -1,5 +1,6 @@
 import os
 import sys
+import time
 
 import pytest
 
@@ -22,3 +23,21 @@ def engine():
     e = Engine(0)
     yield e
     e.close()
+
+
+@pytest.fixture(autouse=True)
+def _solves_outlast_the_arrivals(request, monkeypatch):
+    """test_gpu_serving.py asks that requests arriving 2 ms apart overlap. Its
+    small solves take less than that once buffers are warm, so whether they do
+    hangs on which files ran before; here each waits 3 ms, its data loaded."""
+    if getattr(request.node, 'originalname', '') != 'test_each_result_same_alone_and_in_the_mix':
+        yield
+        return
+    from molgw_amd.gw import Engine
+    load = Engine.set_mo
+
+    def set_mo(self, *args, **kw):
+        load(self, *args, **kw)
+        time.sleep(0.003)
+    monkeypatch.setattr(Engine, 'set_mo', set_mo)
+    yield
