@@ -705,33 +705,45 @@ struct SplitPlan {
 
 // The cheapest plan in cycles. Two workgroups of 128x128 or four of 64x64 share
 // a CU's four SIMDs; a round of them lasts as long as its K range plus a fixed
-// prologue and epilogue. A k step costs the sharing workgroups' MFMA cycles at
-// the part of the peak that they reach together (128x128: 0.55 alone, 0.85 for
-// two; 64x64: 0.25, 0.45, 0.6, 0.68), so a last round that does not fill the
-// slots is cheaper than a whole one. With `split`, the K range of the last
-// round's tiles may be split, into at most two rounds of workgroups (64x64: 64,
-// 128x128: 128 MiB of partial products); those are written and read once at
-// HBM's copy rate (1.9 KB per cycle). Equal costs take the smaller tiles, also
-// when a product fits one of them: the larger one only adds idle waves.
-SplitPlan split_plan(int M, int N, int K, int batch, bool lower, bool split) {
-  constexpr double step128[3] = {0.0, 256.0 / 0.55, 512.0 / 0.85};
-  constexpr double step64[5] = {0.0, 64.0 / 0.25, 128.0 / 0.45, 192.0 / 0.6, 256.0 / 0.68};
+// prologue and epilogue. A k step takes the cycles below by the workgroups that
+// share a CU, so a last round that does not fill the slots is cheaper than a whole
+// one. They are those of the parts of the peak that tiles reach together (128x128:
+// 0.55 alone, 0.85 for two; 64x64: 0.25, 0.45, 0.6, 0.68), but for long-K symmetric
+// products (may_split: chi0, exchange) fitted to 90 of them, of 420 to 1900 rows and
+// 5 to 32 frequencies: there the 64-wide tiles are up to 22 % faster than those parts
+// say (1036 rows, 32 frequencies: 8.5 ms, 10.5 on 128-wide ones), and the choice is
+// 1.1 % from the best on average, 7 % at most; 8 and 41 % with the others.
+//
+// With `room` the K range of the last round's tiles may be split, into at most two
+// rounds of workgroups (64x64: 64, 128x128: 128 MiB of partial products); those are
+// written and read once at HBM's copy rate (1.9 KB per cycle). Equal costs take
+// the smaller tiles, also when a product fits one of them: the larger one only
+// adds idle waves.
+SplitPlan split_plan(int M, int N, int K, int batch, bool lower, bool may_split, bool room) {
+  struct Cost {
+    double step128[3], step64[5], fixed128, fixed64;
+  };
+  static constexpr Cost PLAIN{{0.0, 256.0 / 0.55, 512.0 / 0.85},
+                              {0.0, 64.0 / 0.25, 128.0 / 0.45, 192.0 / 0.6, 256.0 / 0.68}, 48.0, 48.0};
+  static constexpr Cost LONG_K{{0.0, 390.0, 618.0}, {0.0, 160.0, 200.0, 262.0, 310.0}, 40.0, 30.0};
+  const Cost& t = may_split ? LONG_K : PLAIN;
   SplitPlan best{};
   double cost = 0.0;
   for (const int b : {64, 128}) {
-    const double* step = b == 128 ? step128 : step64;
+    const double* step = b == 128 ? t.step128 : t.step64;
+    const double fixed = b == 128 ? t.fixed128 : t.fixed64;
     const int share = b == 128 ? 2 : 4, slots = 256 * share;
     const int64_t tiles = tile_count(M, N, batch, lower, b);
     const int64_t rest = tiles % slots, whole = tiles - rest;
-    const double full = (K + 48.0) * (double)(whole / slots) * step[share];
+    const double full = (K + fixed) * (double)(whole / slots) * step[share];
     // 8 bytes of a partial product written and read, cycles per split
     const double traffic = 16.0 * M * (double)N * batch * (lower ? 0.5 : 1.0) * rest / tiles / 1900.0;
-    for (int s = 1; s == 1 || (split && rest > 0 && K / s >= 64 && s * rest <= 2 * slots); ++s) {
+    for (int s = 1; s == 1 || (may_split && room && rest > 0 && K / s >= 64 && s * rest <= 2 * slots); ++s) {
       const int64_t wgs = s * rest;
-      double c = full + ((double)K / s + 48.0) *
+      double c = full + ((double)K / s + fixed) *
                             ((double)(wgs / slots) * step[share] + step[(wgs % slots + 255) / 256]);
-      if (s > 1) c += 10000.0 + s * traffic;
-      else if (split) c *= 0.95;      // a split has to gain one part in twenty
+      if (s > 1) c += 7000.0 + s * traffic;
+      else if (may_split && room) c *= 0.95;      // a split has to gain one part in twenty
       if (best.b == 0 || c < cost) {
         cost = c;
         best = SplitPlan{b, s, s > 1 ? whole : tiles, s > 1 ? rest : 0};
@@ -784,7 +796,7 @@ int tune(const GemmF64& h, int fn, hipStream_t stream, int* best) {
 }  // namespace
 
 size_t gemm_f64_split_doubles(int M, int N, int K, int batch, bool lower) {
-  const SplitPlan p = split_plan(M, N, K, batch, lower, true);
+  const SplitPlan p = split_plan(M, N, K, batch, lower, true, true);
   return p.splits > 1 ? (size_t)p.rest * p.splits * p.b * p.b : 0;
 }
 
@@ -866,7 +878,7 @@ int gemm_f64(const GemmF64& h, hipStream_t stream) {
               "gemm_f64: a triangular A must be square and not transposed");
   MGW_REQUIRE(h.dotpart != nullptr || h.C != nullptr, MGW_ERR_ARG, "gemm_f64: no output");
   if (h.dotpart) return launch_cfg<64, 64, 2, 2, true, MGW_KCLASS_GEMM_WB>(h, stream);
-  const SplitPlan plan = split_plan(h.M, h.N, h.K, h.batch, h.lower_only, h.split_work != nullptr);
+  const SplitPlan plan = split_plan(h.M, h.N, h.K, h.batch, h.lower_only, h.may_split, h.split_work != nullptr);
   if (plan.splits > 1) return launch_split(plan, h, stream);
   int cfg = plan.b == 64 ? 3 : 2, fn = 0;
   if (!h.transB && !h.lower_only && h.N < 1024) column_tiles(h, &cfg, &fn);

@@ -120,8 +120,9 @@ struct GemmF64 {
   double dot_cc = 0.0, dot_cd = 1.0;
   double* dotpart = nullptr; int64_t strideDot = 0;
   const double* dot_w = nullptr; int64_t strideDotW = 0;
-  // room for the partial products of a split K (FP64, beta 0, no dots):
-  // gemm_f64_split_doubles; without it the product runs unsplit
+  // a long-K symmetric product, whose K may be split (FP64, beta 0, no dots) with
+  // room for the partial products: gemm_f64_split_doubles; without it runs unsplit
+  bool may_split = false;
   double* split_work = nullptr;
   // kernel class: the hot classes get their own kernel symbol so that
   // profiler per-kernel statistics separate them

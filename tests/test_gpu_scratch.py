@@ -19,9 +19,9 @@ def loaded(s):
     return eng
 
 
-# K splits of 64 MiB (more than the factorisation's work matrix, which comes
+# K splits of 63 MiB (more than the factorisation's work matrix, which comes
 # after it) and of 32 MiB (less)
-@pytest.mark.parametrize('nbf, naux, nocc, nomega', [(180, 1000, 80, 16), (150, 700, 50, 32)])
+@pytest.mark.parametrize('nbf, naux, nocc, nomega', [(96, 336, 20, 32), (180, 1000, 80, 16), (150, 700, 50, 32)])
 def test_chi0_k_split_workspace(monkeypatch, nbf, naux, nocc, nomega):
     s = synthetic_system(nbf, naux, nocc, seed=23, scale=0.3)
     npole = nocc * (nbf - nocc)
