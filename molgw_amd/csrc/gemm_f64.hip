@@ -712,7 +712,10 @@ struct SplitPlan {
 // products (may_split: chi0, exchange) fitted to 90 of them, of 420 to 1900 rows and
 // 5 to 32 frequencies: there the 64-wide tiles are up to 22 % faster than those parts
 // say (1036 rows, 32 frequencies: 8.5 ms, 10.5 on 128-wide ones), and the choice is
-// 1.1 % from the best on average, 7 % at most; 8 and 41 % with the others.
+// 1.1 % from the best on average, 7 % at most; 8 and 41 % with the others. A single
+// product whose operand does not stay in the 256 MiB last-level cache has the first
+// ones: 64-wide tiles read it twice as often, and no other frequency's product does
+// at the same time (exchange, 768 functions, 430080 rows: 16.9 ms a call, 17.4 on them).
 //
 // With `room` the K range of the last round's tiles may be split, into at most two
 // rounds of workgroups (64x64: 64, 128x128: 128 MiB of partial products); those are
@@ -726,7 +729,8 @@ SplitPlan split_plan(int M, int N, int K, int batch, bool lower, bool may_split,
   static constexpr Cost PLAIN{{0.0, 256.0 / 0.55, 512.0 / 0.85},
                               {0.0, 64.0 / 0.25, 128.0 / 0.45, 192.0 / 0.6, 256.0 / 0.68}, 48.0, 48.0};
   static constexpr Cost LONG_K{{0.0, 390.0, 618.0}, {0.0, 160.0, 200.0, 262.0, 310.0}, 40.0, 30.0};
-  const Cost& t = may_split ? LONG_K : PLAIN;
+  const bool streamed = batch == 1 && 8.0 * std::max(M, N) * K > 256.0 * (1 << 20);
+  const Cost& t = may_split && !streamed ? LONG_K : PLAIN;
   SplitPlan best{};
   double cost = 0.0;
   for (const int b : {64, 128}) {
